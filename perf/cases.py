@@ -256,14 +256,15 @@ class _Program:
         self.case = case
         self.kind = case["kind"]
         self.holder = None
+        engine = _shared_engine()                # before the scenes' threads ask for it
         if self.kind in ("batch", "served"):
             parts = list(enumerate(_parts(case)))
             with ThreadPoolExecutor(8) as ex:
                 self.scenes = list(ex.map(lambda p: _scene(p[1], seed * 1000 + p[0]), parts))
             if self.kind == "batch":
-                self.holder = oe.Batch(_shared_engine(), self.scenes)
+                self.holder = oe.Batch(engine, self.scenes)
             else:
-                self.holder = oe.Server(_shared_engine(), max_batch=case["max_batch"], streams=case["streams"])
+                self.holder = oe.Server(engine, max_batch=case["max_batch"], streams=case["streams"])
                 self.slots = [self.holder.add_scene(s) for s in self.scenes]
         else:
             self.scenes = [_scene(case, seed)]
