@@ -92,8 +92,6 @@ oe::HostMesh mesh_from(int32_t element, const float* xyz, int32_t nv, const int3
     return m;
 }
 
-void copy3(std::vector<float>& src, float* dst) { std::memcpy(dst, src.data(), src.size() * sizeof(float)); }
-
 // Reads of a served scene first wait for every request submitted for it.
 void wait_served(oe::Scene& sc) {
     if (sc.server) sc.server->wait_slot(sc.server_slot);
@@ -449,9 +447,7 @@ oe_status oe_scene_info(oe_scene* s, int32_t* nv, int32_t* ne, int32_t* S, int32
         return guard([&] {                                   \
             OE_REQUIRE(s && xyz, "bad argument");            \
             wait_served(*s->scene);                          \
-            std::vector<float> h;                            \
-            s->scene->ps->method(h);                         \
-            copy3(h, xyz);                                   \
+            s->scene->ps->method(xyz);                       \
         });                                                  \
     }
 
@@ -988,9 +984,9 @@ oe_status oe_scene_save_vtk(oe_scene* s, const char* path) {
         OE_REQUIRE(s && path, "bad argument");
         oe::Scene& sc = *s->scene;
         wait_served(sc);
-        std::vector<float> rest, pos, m;
-        sc.ps->get_init_position(rest);
-        sc.ps->get_position(pos);
+        std::vector<float> rest(3 * static_cast<size_t>(sc.ps->n)), pos(rest.size()), m;
+        sc.ps->get_init_position(rest.data());
+        sc.ps->get_position(pos.data());
         sc.ps->get_mass(m);
         std::vector<float> u(pos.size());
         for (size_t i = 0; i < u.size(); ++i) u[i] = pos[i] - rest[i];

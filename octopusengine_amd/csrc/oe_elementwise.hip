@@ -285,6 +285,40 @@ __global__ __launch_bounds__(kExplicitVertexBlock) void k_explicit_vertex(PSView
     ps.f[vid] = f4(0.f, 0.f, 0.f, 0.f);
 }
 
+// Packed xyz of a run of records for the host.  The output is pinned host
+// memory, so the pass is bound by the link: a block transposes its 256 records
+// through LDS and writes whole 16-byte words (three 4-byte stores per vertex,
+// 12 bytes apart, would send each link packet a third full).  The sum
+// rest + u is formed in double and rounded once, as the state is stored.
+__global__ __launch_bounds__(kBlock) void k_pack3(const float4* rec, const float4* rest, float unit, int first,
+                                                  int count, float* out) {
+    __shared__ float4 words[kBlock * 3 / 4];
+    float* const flat = reinterpret_cast<float*>(words);
+    const int b0 = blockIdx.x * kBlock, t = threadIdx.x;
+    if (b0 + t < count) {
+        const size_t i = static_cast<size_t>(first) + b0 + t;
+        float4 u = gload(rec, i);
+        if (rest) {
+            const float4 X = gload(rest, i);
+            if (unit == 0.f) u.w = 0.f;
+            const dvec3 d = dunpack(u, unit);
+            u.x = static_cast<float>(X.x + d.x);
+            u.y = static_cast<float>(X.y + d.y);
+            u.z = static_cast<float>(X.z + d.z);
+        }
+        flat[3 * t] = u.x;
+        flat[3 * t + 1] = u.y;
+        flat[3 * t + 2] = u.z;
+    }
+    __syncthreads();
+    const int n_float = 3 * min(kBlock, count - b0);
+    const size_t o = static_cast<size_t>(b0) * 3;   // a multiple of 768 floats
+    if (4 * t + 4 <= n_float)
+        reinterpret_cast<float4*>(out + o)[t] = words[t];
+    else
+        for (int k = 4 * t; k < n_float; ++k) out[o + k] = flat[k];
+}
+
 // ------------------------------------------------------------ batched forms
 // One launch covers every vertex of every scene of a batch; each block belongs
 // to one scene (VSeg), whose description is read with scalar loads.
@@ -354,8 +388,10 @@ void launch_batch_velocity(const BatchVArgs& b, int nblocks, hipStream_t s) {
     if (nblocks > 0) hipLaunchKernelGGL(k_batch_velocity, dim3(nblocks), dim3(kBlock), 0, s, b);
 }
 
-namespace {
-}  // namespace
+void launch_pack3(const float4* rec, const float4* rest, float unit, int first, int count, float* out, hipStream_t s) {
+    if (count > 0)
+        hipLaunchKernelGGL(k_pack3, dim3(grid_for(count)), dim3(kBlock), 0, s, rec, rest, unit, first, count, out);
+}
 
 void launch_vbd_predict(const PSView& ps, float4* y, float4* prev_it_p, float dt, const float g[3], hipStream_t s) {
     if (ps.n <= 0) return;

@@ -32,6 +32,9 @@ void launch_explicit_vertex(const PSView& ps, const OwnersView& own, const float
                             const float* gravity, float dt, hipStream_t s);
 void launch_copy_colour(const PSView& ps, const int* slot_vid, int first, int count, const float4* p_new,
                         hipStream_t s);
+// Read-back: out[0 .. 3 count) = packed xyz of records first .. first + count
+// (see Engine::read3); out is pinned host memory, 16-byte aligned.
+void launch_pack3(const float4* rec, const float4* rest, float unit, int first, int count, float* out, hipStream_t s);
 
 struct SceneDev;
 // All vertices of one scene, covered by blocks [block_begin, next segment's

@@ -38,6 +38,60 @@ Engine::~Engine() {
     }
 }
 
+// --------------------------------------------------------------- Readback
+void Readback::ensure() {
+    for (int i = 0; i < 2; ++i) {
+        if (!half[i]) OE_HIP(hipHostMalloc(reinterpret_cast<void**>(&half[i]), sizeof(float) * 3 * kChunk, hipHostMallocDefault));
+        if (!done[i]) OE_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
+    }
+}
+
+Readback::~Readback() {
+    for (int i = 0; i < 2; ++i) {
+        if (done[i]) (void)hipEventDestroy(done[i]);
+        if (half[i]) (void)hipHostFree(half[i]);
+    }
+}
+
+namespace {
+// The launches below go to the engine's device whatever device the calling
+// thread has selected (a copy on the stream needs no selection, a launch does).
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int dev) {
+        int cur = dev;
+        OE_HIP(hipGetDevice(&cur));
+        if (cur != dev) {
+            OE_HIP(hipSetDevice(dev));
+            before = cur;
+        }
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+}  // namespace
+
+void Engine::read3(const float4* rec, const float4* rest, float unit, int n, float* out) {
+    constexpr int C = Readback::kChunk;
+    std::lock_guard<std::mutex> lock(readback.m);
+    const OnDevice on(device);
+    readback.ensure();
+    const int chunks = (n + C - 1) / C;
+    auto launch = [&](int k) {
+        launch_pack3(rec, rest, unit, k * C, std::min(C, n - k * C), readback.half[k & 1], stream);
+        OE_LAUNCH_CHECK();
+        OE_HIP(hipEventRecord(readback.done[k & 1], stream));
+    };
+    if (chunks > 0) launch(0);
+    for (int k = 0; k < chunks; ++k) {
+        if (k + 1 < chunks) launch(k + 1);   // half (k + 1) & 1 was emptied in round k - 1
+        OE_HIP(hipEventSynchronize(readback.done[k & 1]));
+        std::memcpy(out + 3 * static_cast<size_t>(k) * C, readback.half[k & 1],
+                    sizeof(float) * 3 * static_cast<size_t>(std::min(C, n - k * C)));
+    }
+}
+
 // ------------------------------------------------------ GPU_ParticleSystem
 namespace {
 std::vector<float4> to_f4(const std::vector<float>& xyz) {
@@ -45,14 +99,6 @@ std::vector<float4> to_f4(const std::vector<float>& xyz) {
     std::vector<float4> out(n);
     for (size_t i = 0; i < n; ++i) out[i] = make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0.f);
     return out;
-}
-void from_f4(const std::vector<float4>& v, std::vector<float>& xyz) {
-    xyz.resize(v.size() * 3);
-    for (size_t i = 0; i < v.size(); ++i) {
-        xyz[3 * i] = v[i].x;
-        xyz[3 * i + 1] = v[i].y;
-        xyz[3 * i + 2] = v[i].z;
-    }
 }
 }  // namespace
 
@@ -92,28 +138,11 @@ PSView GPU_ParticleSystem::get_parameters() const {
 // the records' w lanes are zero until a compensated integrator writes them
 void GPU_ParticleSystem::enable_compensation() { comp = true; }
 
-std::vector<double> GPU_ParticleSystem::full(const DBuf<float4>& rec) const {
-    std::vector<float4> h;
-    rec.download(h, eng->stream);
-    std::vector<double> u(3 * h.size());
-    for (size_t i = 0; i < h.size(); ++i) {
-        const dvec3 d = comp ? dunpack(h[i], lo_unit) : dvec3{h[i].x, h[i].y, h[i].z};
-        u[3 * i] = d.x;
-        u[3 * i + 1] = d.y;
-        u[3 * i + 2] = d.z;
-    }
-    return u;
+void GPU_ParticleSystem::get_position(float* xyz) const {
+    eng->read3(p.get(), init_p.get(), comp ? lo_unit : 0.f, n, xyz);
 }
-
-void GPU_ParticleSystem::get_position(std::vector<float>& xyz) const {
-    const std::vector<double> u = full(p);
-    xyz.resize(u.size());
-    for (size_t i = 0; i < xyz.size(); ++i) xyz[i] = static_cast<float>(rest[i] + u[i]);
-}
-void GPU_ParticleSystem::get_prev_position(std::vector<float>& xyz) const {
-    const std::vector<double> u = full(last_p);
-    xyz.resize(u.size());
-    for (size_t i = 0; i < xyz.size(); ++i) xyz[i] = static_cast<float>(rest[i] + u[i]);
+void GPU_ParticleSystem::get_prev_position(float* xyz) const {
+    eng->read3(last_p.get(), init_p.get(), comp ? lo_unit : 0.f, n, xyz);
 }
 
 // xyz (absolute, 3n floats) -> displacement records from the double
@@ -129,21 +158,9 @@ void GPU_ParticleSystem::upload_split(const float* xyz, DBuf<float4>& rec) {
     }
     rec.upload(h, eng->stream);
 }
-void GPU_ParticleSystem::get_init_position(std::vector<float>& xyz) const {
-    std::vector<float4> h;
-    init_p.download(h, eng->stream);
-    from_f4(h, xyz);
-}
-void GPU_ParticleSystem::get_velocity(std::vector<float>& xyz) const {
-    std::vector<float4> h;
-    v.download(h, eng->stream);
-    from_f4(h, xyz);
-}
-void GPU_ParticleSystem::get_forces(std::vector<float>& xyz) const {
-    std::vector<float4> h;
-    f.download(h, eng->stream);
-    from_f4(h, xyz);
-}
+void GPU_ParticleSystem::get_init_position(float* xyz) const { eng->read3(init_p.get(), nullptr, 0.f, n, xyz); }
+void GPU_ParticleSystem::get_velocity(float* xyz) const { eng->read3(v.get(), nullptr, 0.f, n, xyz); }
+void GPU_ParticleSystem::get_forces(float* xyz) const { eng->read3(f.get(), nullptr, 0.f, n, xyz); }
 void GPU_ParticleSystem::get_masks(std::vector<int>& out) const { mask.download(out, eng->stream); }
 void GPU_ParticleSystem::get_mass(std::vector<float>& out) const { m.download(out, eng->stream); }
 void GPU_ParticleSystem::get_inv_mass(std::vector<float>& out) const { w.download(out, eng->stream); }

@@ -19,10 +19,10 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <memory>
-#include <vector>
-
 #include <map>
+#include <memory>
+#include <mutex>
+#include <vector>
 
 #include "oe_device.hpp"
 #include "oe_elementwise.hpp"
@@ -32,11 +32,32 @@
 
 namespace oe {
 
+// Read-back of per-vertex records through pinned host memory.  k_pack3 writes
+// 12 bytes per vertex straight into one of two pinned halves, which the host
+// copies into the caller's array while the next chunk is written.  A copy of
+// the 16-byte records into pageable memory, then unpacked by the host, took
+// 115 us for the copy alone at 18,785 vertices; this takes 20 us for the whole
+// call.  The halves belong to the engine, are allocated by its first read and
+// are used by one read at a time.
+struct Readback {
+    static constexpr int kChunk = 65536;   // vertices per half (768 KB)
+    std::mutex m;
+    float* half[2] = {nullptr, nullptr};
+    hipEvent_t done[2] = {nullptr, nullptr};
+    void ensure();
+    ~Readback();
+};
+
 struct Engine {
     int device = 0;
     hipStream_t stream = nullptr;
     MemoryPool pool;
     bool autotune = false;   // tune the layout of every VBD / explicit scene created
+    Readback readback;
+    // n records as packed xyz into `out` (host): rest + u in double rounded
+    // once when rest is given (low-order parts of quantum `unit` included when
+    // it is not 0), the records' xyz otherwise.  Synchronising.
+    void read3(const float4* rec, const float4* rest, float unit, int n, float* out);
     explicit Engine(int dev, size_t budget_bytes = SIZE_MAX);
     ~Engine();
     Engine(const Engine&) = delete;
@@ -47,11 +68,11 @@ struct GPU_ParticleSystem {
     GPU_ParticleSystem(Engine* eng, const std::vector<float>& xyz, const std::vector<float>& masses);
     int nb_particles() const { return n; }
     PSView get_parameters() const;
-    void get_position(std::vector<float>& xyz) const;
-    void get_prev_position(std::vector<float>& xyz) const;
-    void get_init_position(std::vector<float>& xyz) const;
-    void get_velocity(std::vector<float>& xyz) const;
-    void get_forces(std::vector<float>& xyz) const;
+    void get_position(float* xyz) const;   // 3 n floats
+    void get_prev_position(float* xyz) const;
+    void get_init_position(float* xyz) const;
+    void get_velocity(float* xyz) const;
+    void get_forces(float* xyz) const;
     void get_masks(std::vector<int>& m) const;
     void get_mass(std::vector<float>& m) const;
     void get_inv_mass(std::vector<float>& w) const;
@@ -75,8 +96,6 @@ struct GPU_ParticleSystem {
 private:
     bool comp = false;
     float lo_unit = 1.f;   // quantum of the low-order parts (lo_unit_for the rest bounding box)
-    // displacement of every vertex, hi + lo in double (lo = 0 without compensation)
-    std::vector<double> full(const DBuf<float4>& rec) const;
     void upload_split(const float* xyz, DBuf<float4>& rec);
 };
 
