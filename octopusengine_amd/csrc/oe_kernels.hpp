@@ -41,6 +41,16 @@ __device__ __forceinline__ const Seg& find_seg(const Seg* __restrict__ segs, int
     return segs[lo];
 }
 
+// Orders the wave's own LDS operations for all of its lanes (a wave's LDS
+// operations complete in order) and keeps the compiler from moving memory
+// accesses across; no workgroup barrier.
+__device__ __forceinline__ void wave_lds_sync() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_wave_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 // Per-vertex accumulator: force (3) + lower triangle of the symmetric 3x3
 // Hessian block (H00, H10, H20, H11, H21, H22).
 struct Acc9 {
@@ -64,6 +74,49 @@ template <int L>
 __device__ __forceinline__ void group_sum(Acc9& a) {
 #pragma unroll
     for (int i = 0; i < 9; ++i) a.v[i] = group_sum<L>(a.v[i]);
+}
+
+// x + (x at lane ctrl(lane)) for the rows in ROWS; other rows add 0.  Every
+// lane of the wave must be active (the cross-lane helpers below as well).
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dpp_add(float x) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xF, false));
+}
+// x + the value of the neighbouring 16-lane row (rows 0 and 1, 2 and 3), and
+// x + the value of the other 32-lane half: v_permlane{16,32}_swap of x with
+// itself leaves the pair's two values in its two results.
+__device__ __forceinline__ float row_pair_add(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float half_pair_add(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Sum over aligned groups of W consecutive lanes, in every lane of the group
+// (quad_perm 1,0,3,2; quad_perm 2,3,0,1; mirror in 8 lanes; mirror in 16;
+// then across rows and halves).  VALU only: a ds_bpermute step of __shfl_xor
+// takes about 40 ns.
+template <int W>
+__device__ __forceinline__ float lanes_sum(float x) {
+    if constexpr (W >= 2) x = dpp_add<0xB1>(x);
+    if constexpr (W >= 4) x = dpp_add<0x4E>(x);
+    if constexpr (W >= 8) x = dpp_add<0x141>(x);
+    if constexpr (W >= 16) x = dpp_add<0x140>(x);
+    if constexpr (W >= 32) x = row_pair_add(x);
+    if constexpr (W >= 64) x = half_pair_add(x);
+    return x;
+}
+// Sum over the lanes that are a multiple of W apart inside aligned groups of
+// L lanes (4 <= W <= L): rotations inside a row, then across rows and halves.
+template <int W, int L>
+__device__ __forceinline__ float parts_sum(float x) {
+    static_assert(W >= 4 && W <= L && L <= 64 && (W == L || L >= 16), "parts of 4 lanes and more, whole rows");
+    if constexpr (W <= 4 && L >= 16) x = dpp_add<0x124>(x);   // row_ror:4
+    if constexpr (W <= 8 && L >= 16) x = dpp_add<0x128>(x);   // row_ror:8
+    if constexpr (W <= 16 && L >= 32) x = row_pair_add(x);
+    if constexpr (W <= 32 && L >= 64) x = half_pair_add(x);
+    return x;
 }
 
 // Jx = sum_k x_k (x) dN_k  (column-major: Jx[c*3+r] = sum_k x_k[r] dN_k[c]);

@@ -9,9 +9,8 @@
 //    Used for P1 and when the XPBD version is requested.  One thread per element.
 //  * "V2" (src/GPU/PBD/GPU_PBD_FEM.cu:206-263, and V1 :141-204 which has the
 //    same arithmetic): beta = -2E / (sum w |grad E|^2 + 4E/(k dt^2)), zero when
-//    E < 1e-12, every node moved.  One group of LPE lanes per element: lanes
-//    q < Q evaluate the quadrature points, lanes k < S own the nodes; the
-//    node positions and per-quadrature stresses are staged in LDS.
+//    E < 1e-12, every node moved.  One group of lanes per element (V2Plan);
+//    the node positions and per-quadrature stresses are staged in LDS.
 // Energies per material: src/GPU/PBD/GPU_PBD_FEM_Materials.cu:31-66,97-118.
 #include "oe_kernels.hpp"
 #include "oe_xpbd.hpp"
@@ -125,115 +124,159 @@ __global__ __launch_bounds__(256) void k_xpbd_v0(XpbdArgs a) {
     }
 }
 
-// With LPE = 64 (27-node hexahedra) the two 32-lane halves of the wave split
-// the node sum of each point's Jx and the point sum of each node's gradient,
-// and add their parts with one cross-half shuffle, halving the chain of
-// dependent LDS reads and FMAs a wave runs per projection.
-template <int S, int Q, int LPE>
-__global__ __launch_bounds__(256) void k_xpbd_v2(XpbdArgs a) {
-    constexpr int SPLIT = LPE > 32 ? LPE / 32 : 1;
-    constexpr int W = LPE / SPLIT;   // lanes per part
-    static_assert(S <= W && Q <= W, "element does not fit the lane group");
-    constexpr int EPB = 256 / LPE;
-    constexpr int KH = (S + SPLIT - 1) / SPLIT;   // nodes per part (point stage)
-    constexpr int QH = (Q + SPLIT - 1) / SPLIT;   // points per part (node stage)
-    __shared__ float sx[EPB][S][3];
-    __shared__ float sP[EPB][Q][9];
-    // Large shape-derivative tables (27-node hexahedra, 8.7 KB) are staged in
-    // LDS; smaller ones are read from the cache (measured: the copy costs the
-    // 20-node tetrahedra 0.3 us per colour and saves the 27-node hexahedra 2 us).
-    constexpr bool kDnLds = Q * S * 3 > 1024;
-    __shared__ float dn_s[kDnLds ? Q * S * 3 : 1];
-    if constexpr (kDnLds)
-        for (int i = threadIdx.x; i < Q * S * 3; i += 256) dn_s[i] = gload(a.fem.dN, i);
-    const float* __restrict__ dnt = kDnLds ? static_cast<const float*>(dn_s) : a.fem.dN;
-    const int le = threadIdx.x / LPE;
-    const int lane = threadIdx.x % LPE;
-    const int sub = lane % W, part = lane / W;
+// Lanes of one element in the V2 projection.  The point stage gives a
+// quadrature point WP lanes' worth of room, PP times over: part p sums its KP
+// nodes of every point's Jx.  The node stage gives the nodes WN lanes, PN
+// times over: part p sums its QN points of every node's gradient.  A colour
+// holds a few hundred elements, far too few to fill the chip, so a pass lasts
+// as long as one wave's chain of instructions: the sums are split over as many
+// lanes as an element can use, and LDS is read 16 bytes at a time.
+template <int S, int Q>
+struct V2Lanes;
+template <> struct V2Lanes<4, 1> { static constexpr int WP = 4, PP = 1, WN = 4, PN = 1; };
+template <> struct V2Lanes<8, 8> { static constexpr int WP = 8, PP = 4, WN = 8, PN = 4; };
+template <> struct V2Lanes<10, 4> { static constexpr int WP = 4, PP = 4, WN = 16, PN = 1; };
+template <> struct V2Lanes<20, 11> { static constexpr int WP = 16, PP = 4, WN = 32, PN = 2; };
+template <> struct V2Lanes<27, 27> { static constexpr int WP = 32, PP = 2, WN = 32, PN = 2; };
+
+template <int S, int Q>
+struct V2Plan {
+    using L = V2Lanes<S, Q>;
+    static constexpr int WP = L::WP, WN = L::WN, LPE = L::WP * L::PP;
+    static_assert(LPE == L::WN * L::PN && LPE <= 64 && Q <= WP && S <= WN, "lanes of one element");
+    static constexpr int KP = (S + L::PP - 1) / L::PP;   // nodes a part sums (point stage)
+    static constexpr int QN = (Q + L::PN - 1) / L::PN;   // points a part sums (node stage)
+    int q, k;            // the lane's point and node (clamped)
+    bool point, node;    // whether it has one
+    int kp[KP];          // the nodes of the lane's part (clamped, weight 0 past the last)
+    float dp[KP][3];     // their dN at point q
+    int qn[QN];          // the points of the lane's part
+    float dn[QN][3];     // dN of node k there
+    __device__ __forceinline__ void init(const float* dN, int lane) {
+        const int sp = lane % WP, sn = lane % WN;
+        point = sp < Q;
+        node = sn < S;
+        q = point ? sp : Q - 1;
+        k = node ? sn : S - 1;
+#pragma unroll
+        for (int j = 0; j < KP; ++j) {
+            const int n = lane / WP * KP + j;
+            const bool in = n < S;
+            kp[j] = in ? n : S - 1;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float d = gload(dN, (q * S + kp[j]) * 3 + c);
+                dp[j][c] = in ? d : 0.f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < QN; ++j) {
+            const int n = lane / WN * QN + j;
+            const bool in = n < Q;
+            qn[j] = in ? n : Q - 1;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float d = gload(dN, (qn[j] * S + k) * 3 + c);
+                dn[j][c] = in ? d : 0.f;
+            }
+        }
+    }
+};
+
+// Both constraints of the element whose node values are x[0 .. S) in LDS (xyz;
+// w the inverse mass), moved in place.  sP: Q rows of 3 float4 of scratch of
+// the lane group.  Every lane of the wave must call it.
+template <int S, int Q>
+__device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, const V2Plan<S, Q>& pl, const float JXi[9],
+                                           float V, float4* x, float4* sP) {
+    using P_ = V2Plan<S, Q>;
+    const float alpha_nh = 1.f + mt.mu / mt.lambda;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        float Jx[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) Jx[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < P_::KP; ++j) {
+            const float4 u = x[pl.kp[j]];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                Jx[3 * c] = fmaf(u.x, pl.dp[j][c], Jx[3 * c]);
+                Jx[3 * c + 1] = fmaf(u.y, pl.dp[j][c], Jx[3 * c + 1]);
+                Jx[3 * c + 2] = fmaf(u.z, pl.dp[j][c], Jx[3 * c + 2]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 9; ++i) Jx[i] = parts_sum<P_::WP, P_::LPE>(Jx[i]);
+        float F[9], P[9], Ps[9], e;
+        deformation_gradient(Jx, JXi, F);
+        xpbd_material(mt.material, m, alpha_nh, F, P, e);
+        scale_stress(P, JXi, V, Ps);
+        if (pl.point) {   // the parts hold the same values
+            sP[3 * pl.q] = make_float4(Ps[0], Ps[1], Ps[2], Ps[3]);
+            sP[3 * pl.q + 1] = make_float4(Ps[4], Ps[5], Ps[6], Ps[7]);
+            sP[3 * pl.q + 2] = make_float4(Ps[8], 0.f, 0.f, 0.f);
+        }
+        const float C = lanes_sum<P_::WP>(pl.point ? e * V : 0.f);
+        wave_lds_sync();
+        float g0 = 0.f, g1 = 0.f, g2 = 0.f;
+#pragma unroll
+        for (int j = 0; j < P_::QN; ++j) {
+            const float4 a = sP[3 * pl.qn[j]], b = sP[3 * pl.qn[j] + 1];
+            const float c = sP[3 * pl.qn[j] + 2].x;
+            g0 += a.x * pl.dn[j][0] + a.w * pl.dn[j][1] + b.z * pl.dn[j][2];
+            g1 += a.y * pl.dn[j][0] + b.x * pl.dn[j][1] + b.w * pl.dn[j][2];
+            g2 += a.z * pl.dn[j][0] + b.y * pl.dn[j][1] + c * pl.dn[j][2];
+        }
+        g0 = parts_sum<P_::WN, P_::LPE>(g0);
+        g1 = parts_sum<P_::WN, P_::LPE>(g1);
+        g2 = parts_sum<P_::WN, P_::LPE>(g2);
+        const float4 u = x[pl.k];
+        const float sn = pl.node ? (g0 * g0 + g1 * g1 + g2 * g2) * u.w : 0.f;
+        const float ssum = lanes_sum<P_::WN>(sn);
+        const float stiff = (m == 0) ? mt.lambda : mt.mu;
+        const float alpha = 4.f * C / (stiff * dt * dt);
+        const float beta = C < 1e-12f ? 0.f : -2.f * C / (ssum + alpha);
+        wave_lds_sync();   // every lane has read x
+        if (pl.node) {
+            const float s = beta * u.w;
+            x[pl.k] = make_float4(u.x + s * g0, u.y + s * g1, u.z + s * g2, u.w);
+        }
+        wave_lds_sync();
+    }
+}
+
+// One group of LPE lanes per element, one-wave blocks (an element's lanes
+// never span waves, so no workgroup barrier is needed and the blocks spread
+// over the chip).  Bound by one wave's chain: launch 1.6 us, three dependent
+// loads, then about 950 instructions (27 nodes).  us per colour of the
+// 32 x 8 x 8 beams, before (256-thread blocks, rolled sums, 4-byte LDS reads)
+// and now: see the launcher.
+template <int S, int Q>
+__global__ __launch_bounds__(64) void k_xpbd_v2(XpbdArgs a) {
+    using P_ = V2Plan<S, Q>;
+    constexpr int EPB = 64 / P_::LPE;
+    __shared__ float4 sx[EPB][S];
+    __shared__ float4 sP[EPB][Q * 3];
+    const int le = threadIdx.x / P_::LPE, lane = threadIdx.x % P_::LPE;
     const int ei = blockIdx.x * EPB + le;
     const bool valid = ei < a.count;
-    const int eid = valid ? a.eids[a.first + ei] : 0;
-    const int* __restrict__ tp = a.fem.topo + static_cast<size_t>(eid) * S;
-    int vid = 0;
-    float wv = 0.f;
-    if (valid && lane < S) {
-        vid = tp[lane];
-        const float4 x = a.ps.p[vid];
-        sx[le][lane][0] = x.x; sx[le][lane][1] = x.y; sx[le][lane][2] = x.z;
-        wv = a.ps.w[vid];
-    }
+    // a group past the colour's end works on its last element and stores nothing
+    const int eid = gload(a.eids, a.first + (valid ? ei : a.count - 1));
+    P_ pl;
+    pl.init(a.fem.dN, lane);
+    const int vid = gload(a.fem.topo, static_cast<size_t>(eid) * S + pl.k);
     float JXi[9], V;
-    load_element_record(a.fem, eid, sub < Q ? sub : Q - 1, JXi, V);
-    __syncthreads();
-    // constant bounds without a split, so that those loops unroll fully
-    const int k_begin = SPLIT == 1 ? 0 : part * KH;
-    const int k_end = SPLIT == 1 ? S : ((part + 1) * KH < S ? (part + 1) * KH : S);
-    const int q_begin = SPLIT == 1 ? 0 : part * QH;
-    const int q_end = SPLIT == 1 ? Q : ((part + 1) * QH < Q ? (part + 1) * QH : Q);
-    for (int m = 0; m < 2; ++m) {
-        float e_loc = 0.f;
-        {
-            const int q = sub < Q ? sub : Q - 1;
-            const float* dn = dnt + q * S * 3;
-            float Jx[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) Jx[i] = 0.f;
-#pragma unroll
-            for (int k = k_begin; k < k_end; ++k) {
-                const float d0 = dn[3 * k], d1 = dn[3 * k + 1], d2 = dn[3 * k + 2];
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const float xr = sx[le][k][r];
-                    Jx[r] += xr * d0; Jx[3 + r] += xr * d1; Jx[6 + r] += xr * d2;
-                }
-            }
-            if constexpr (SPLIT == 2) {
-#pragma unroll
-                for (int i = 0; i < 9; ++i) Jx[i] += __shfl_xor(Jx[i], 32);
-            }
-            if (valid && part == 0 && sub < Q) {
-                float F[9], P[9], Ps[9], e;
-                deformation_gradient(Jx, JXi, F);
-                xpbd_material(a.mt.material, m, 1.f + a.mt.mu / a.mt.lambda, F, P, e);
-                scale_stress(P, JXi, V, Ps);
-                e_loc = e * V;
-#pragma unroll
-                for (int i = 0; i < 9; ++i) sP[le][q][i] = Ps[i];
-            }
-        }
-        const float C = group_sum<LPE>(e_loc);
-        __syncthreads();
-        float g0 = 0.f, g1 = 0.f, g2 = 0.f, sn = 0.f;
-        {
-            const int k = sub < S ? sub : S - 1;
-#pragma unroll
-            for (int q = q_begin; q < q_end; ++q) {
-                const float* dn = dnt + (q * S + k) * 3;
-                const float* Ps = sP[le][q];
-                g0 += Ps[0] * dn[0] + Ps[3] * dn[1] + Ps[6] * dn[2];
-                g1 += Ps[1] * dn[0] + Ps[4] * dn[1] + Ps[7] * dn[2];
-                g2 += Ps[2] * dn[0] + Ps[5] * dn[1] + Ps[8] * dn[2];
-            }
-            if constexpr (SPLIT == 2) {
-                g0 += __shfl_xor(g0, 32);
-                g1 += __shfl_xor(g1, 32);
-                g2 += __shfl_xor(g2, 32);
-            }
-            if (valid && lane < S) sn = (g0 * g0 + g1 * g1 + g2 * g2) * wv;
-        }
-        const float ssum = group_sum<LPE>(sn);
-        const float stiff = (m == 0) ? a.mt.lambda : a.mt.mu;
-        const float alpha = 4.f * C / (stiff * a.dt * a.dt);
-        const float beta = C < 1e-12f ? 0.f : -2.f * C / (ssum + alpha);
-        if (valid && lane < S) {
-            const float nx = sx[le][lane][0] + beta * wv * g0;
-            const float ny = sx[le][lane][1] + beta * wv * g1;
-            const float nz = sx[le][lane][2] + beta * wv * g2;
-            sx[le][lane][0] = nx; sx[le][lane][1] = ny; sx[le][lane][2] = nz;
-            const float4 old = a.ps.p[vid];
-            a.ps.p[vid] = make_float4(nx, ny, nz, old.w);
-        }
-        __syncthreads();
+    load_element_record(a.fem, eid, pl.q, JXi, V);
+    float4 u = gload(static_cast<const float4*>(a.ps.p), vid);
+    const float keep = u.w;
+    u.w = gload(a.ps.w, vid);
+    if (lane < S) sx[le][lane] = u;
+    wave_lds_sync();
+    v2_project<S, Q>(a.mt, a.dt, pl, JXi, V, sx[le], sP[le]);
+    if (valid && lane < S) {
+        const float4 r = sx[le][lane];
+        gstore(a.ps.p, vid, make_float4(r.x, r.y, r.z, keep));
     }
 }
 
@@ -243,11 +286,10 @@ void launch_v0(const XpbdArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_xpbd_v0<S, Q>), dim3(grid), dim3(256), 0, s, a);
 }
 
-template <int S, int Q, int LPE>
+template <int S, int Q>
 void launch_v2(const XpbdArgs& a, hipStream_t s) {
-    constexpr int EPB = 256 / LPE;
-    const int grid = (a.count + EPB - 1) / EPB;
-    hipLaunchKernelGGL((k_xpbd_v2<S, Q, LPE>), dim3(grid), dim3(256), 0, s, a);
+    constexpr int EPB = 64 / V2Plan<S, Q>::LPE;
+    hipLaunchKernelGGL((k_xpbd_v2<S, Q>), dim3((a.count + EPB - 1) / EPB), dim3(64), 0, s, a);
 }
 
 }  // namespace
@@ -262,11 +304,11 @@ bool launch_xpbd(int S, int Q, bool v0_form, const XpbdArgs& a, hipStream_t s) {
         if (S == 27 && Q == 27) { launch_v0<27, 27>(a, s); return true; }
         return false;
     }
-    if (S == 4 && Q == 1) { launch_v2<4, 1, 4>(a, s); return true; }
-    if (S == 8 && Q == 8) { launch_v2<8, 8, 8>(a, s); return true; }
-    if (S == 10 && Q == 4) { launch_v2<10, 4, 16>(a, s); return true; }
-    if (S == 20 && Q == 11) { launch_v2<20, 11, 32>(a, s); return true; }
-    if (S == 27 && Q == 27) { launch_v2<27, 27, 64>(a, s); return true; }
+    if (S == 4 && Q == 1) { launch_v2<4, 1>(a, s); return true; }
+    if (S == 8 && Q == 8) { launch_v2<8, 8>(a, s); return true; }
+    if (S == 10 && Q == 4) { launch_v2<10, 4>(a, s); return true; }
+    if (S == 20 && Q == 11) { launch_v2<20, 11>(a, s); return true; }
+    if (S == 27 && Q == 27) { launch_v2<27, 27>(a, s); return true; }
     return false;
 }
 
