@@ -131,17 +131,19 @@ __global__ __launch_bounds__(256) void k_xpbd_v0(XpbdArgs a) {
 // holds a few hundred elements, far too few to fill the chip, so a pass lasts
 // as long as one wave's chain of instructions: the sums are split over as many
 // lanes as an element can use, and LDS is read 16 bytes at a time.
-template <int S, int Q>
+// NARROW (8-node hexahedra, 8 lanes): colours that fill the chip by themselves.
+template <int S, int Q, bool NARROW = false>
 struct V2Lanes;
+template <> struct V2Lanes<8, 8, true> { static constexpr int WP = 8, PP = 1, WN = 8, PN = 1; };
 template <> struct V2Lanes<4, 1> { static constexpr int WP = 4, PP = 1, WN = 4, PN = 1; };
 template <> struct V2Lanes<8, 8> { static constexpr int WP = 8, PP = 4, WN = 8, PN = 4; };
 template <> struct V2Lanes<10, 4> { static constexpr int WP = 4, PP = 4, WN = 16, PN = 1; };
 template <> struct V2Lanes<20, 11> { static constexpr int WP = 16, PP = 4, WN = 32, PN = 2; };
 template <> struct V2Lanes<27, 27> { static constexpr int WP = 32, PP = 2, WN = 32, PN = 2; };
 
-template <int S, int Q>
+template <int S, int Q, bool NARROW = false>
 struct V2Plan {
-    using L = V2Lanes<S, Q>;
+    using L = V2Lanes<S, Q, NARROW>;
     static constexpr int WP = L::WP, WN = L::WN, LPE = L::WP * L::PP;
     static_assert(LPE == L::WN * L::PN && LPE <= 64 && Q <= WP && S <= WN, "lanes of one element");
     static constexpr int KP = (S + L::PP - 1) / L::PP;   // nodes a part sums (point stage)
@@ -186,10 +188,9 @@ struct V2Plan {
 // Both constraints of the element whose node values are x[0 .. S) in LDS (xyz;
 // w the inverse mass), moved in place.  sP: Q rows of 3 float4 of scratch of
 // the lane group.  Every lane of the wave must call it.
-template <int S, int Q>
-__device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, const V2Plan<S, Q>& pl, const float JXi[9],
-                                           float V, float4* x, float4* sP) {
-    using P_ = V2Plan<S, Q>;
+template <class P_>
+__device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, const P_& pl, const float JXi[9], float V,
+                                           float4* x, float4* sP) {
     const float alpha_nh = 1.f + mt.mu / mt.lambda;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -249,12 +250,13 @@ __device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, con
 // One group of LPE lanes per element, one-wave blocks (an element's lanes
 // never span waves, so no workgroup barrier is needed and the blocks spread
 // over the chip).  Bound by one wave's chain: launch 1.6 us, three dependent
-// loads, then about 950 instructions (27 nodes).  us per colour of the
-// 32 x 8 x 8 beams, before (256-thread blocks, rolled sums, 4-byte LDS reads)
-// and now: see the launcher.
-template <int S, int Q>
+// loads, then about 950 instructions (27 nodes).  A frame of 50 substeps of the
+// 32 x 8 x 8 beams: 27-node hexahedra 4.84 -> 3.05 ms (227 elements per
+// colour), 20-node tetrahedra 10.16 -> 7.45 ms (424 per colour), against
+// 256-thread blocks with workgroup barriers, rolled sums and 4-byte LDS reads.
+template <int S, int Q, bool NARROW>
 __global__ __launch_bounds__(64) void k_xpbd_v2(XpbdArgs a) {
-    using P_ = V2Plan<S, Q>;
+    using P_ = V2Plan<S, Q, NARROW>;
     constexpr int EPB = 64 / P_::LPE;
     __shared__ float4 sx[EPB][S];
     __shared__ float4 sP[EPB][Q * 3];
@@ -273,7 +275,7 @@ __global__ __launch_bounds__(64) void k_xpbd_v2(XpbdArgs a) {
     u.w = gload(a.ps.w, vid);
     if (lane < S) sx[le][lane] = u;
     wave_lds_sync();
-    v2_project<S, Q>(a.mt, a.dt, pl, JXi, V, sx[le], sP[le]);
+    v2_project(a.mt, a.dt, pl, JXi, V, sx[le], sP[le]);
     if (valid && lane < S) {
         const float4 r = sx[le][lane];
         gstore(a.ps.p, vid, make_float4(r.x, r.y, r.z, keep));
@@ -286,10 +288,10 @@ void launch_v0(const XpbdArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_xpbd_v0<S, Q>), dim3(grid), dim3(256), 0, s, a);
 }
 
-template <int S, int Q>
+template <int S, int Q, bool NARROW = false>
 void launch_v2(const XpbdArgs& a, hipStream_t s) {
-    constexpr int EPB = 64 / V2Plan<S, Q>::LPE;
-    hipLaunchKernelGGL((k_xpbd_v2<S, Q>), dim3((a.count + EPB - 1) / EPB), dim3(64), 0, s, a);
+    constexpr int EPB = 64 / V2Plan<S, Q, NARROW>::LPE;
+    hipLaunchKernelGGL((k_xpbd_v2<S, Q, NARROW>), dim3((a.count + EPB - 1) / EPB), dim3(64), 0, s, a);
 }
 
 }  // namespace
@@ -305,7 +307,14 @@ bool launch_xpbd(int S, int Q, bool v0_form, const XpbdArgs& a, hipStream_t s) {
         return false;
     }
     if (S == 4 && Q == 1) { launch_v2<4, 1>(a, s); return true; }
-    if (S == 8 && Q == 8) { launch_v2<8, 8>(a, s); return true; }
+    if (S == 8 && Q == 8) {
+        // 32 lanes per element up to two waves per SIMD (4,096 elements), 8 past
+        // that: a substep of the 64x16x16 beam (2,048 elements per colour) takes
+        // 51.9 us with 32 lanes and 62 with 8, of 128x32x32 (16,384) 118 and 78
+        if (a.count <= 1024) launch_v2<8, 8>(a, s);
+        else launch_v2<8, 8, true>(a, s);
+        return true;
+    }
     if (S == 10 && Q == 4) { launch_v2<10, 4>(a, s); return true; }
     if (S == 20 && Q == 11) { launch_v2<20, 11>(a, s); return true; }
     if (S == 27 && Q == 27) { launch_v2<27, 27>(a, s); return true; }
