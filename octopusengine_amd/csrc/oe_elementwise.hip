@@ -24,14 +24,11 @@ inline int grid_for(long long n) { return static_cast<int>((n + kBlock - 1) / kB
 
 __device__ __forceinline__ float4 f4(float x, float y, float z, float w) { return make_float4(x, y, z, w); }
 
-// y = p + ((p - last_p) / dt + (g + f w) dt) dt ; last_p = p ; p = y ; f = 0,
-// on the compensated state in FP64.
-__device__ __forceinline__ void vbd_predict_one(const PSView& ps, float4* y, int i, float dt, float gx, float gy,
-                                                float gz, float4* prev_it_p) {
-    const float4 p = ps.p[i];
-    const float4 f = ps.f[i];
-    const float w = ps.w[i];
-    const dvec3 P = dunpack(p, ps.lo_unit), LP = dunpack(ps.last_p[i], ps.lo_unit);
+// y = p + ((p - last_p) / dt + (g + f w) dt) dt ; last_p = p ; p = y, on the
+// compensated state in FP64.
+__device__ __forceinline__ void vbd_predict_from(const PSView& ps, float4* y, int i, float4 p, float4 last_p, float4 f,
+                                                 float w, float dt, float gx, float gy, float gz, float4* prev_it_p) {
+    const dvec3 P = dunpack(p, ps.lo_unit), LP = dunpack(last_p, ps.lo_unit);
     if (prev_it_p) prev_it_p[i] = p;
     const double ddt = dt;
     const double ax = gx + static_cast<double>(f.x) * w, ay = gy + static_cast<double>(f.y) * w,
@@ -42,6 +39,14 @@ __device__ __forceinline__ void vbd_predict_one(const PSView& ps, float4* y, int
     y[i] = Y;
     ps.last_p[i] = p;
     ps.p[i] = Y;
+}
+
+// the same from the stored state; f = 0 after it
+__device__ __forceinline__ void vbd_predict_one(const PSView& ps, float4* y, int i, float dt, float gx, float gy,
+                                                float gz, float4* prev_it_p) {
+    const float4 p = ps.p[i], f = ps.f[i];
+    const float w = ps.w[i];
+    vbd_predict_from(ps, y, i, p, ps.last_p[i], f, w, dt, gx, gy, gz, prev_it_p);
     ps.f[i] = f4(0.f, 0.f, 0.f, 0.f);
 }
 
@@ -53,33 +58,11 @@ __global__ __launch_bounds__(kBlock) void k_vbd_predict(PSView ps, float4* y, fl
 }
 
 // v = (p - last_p) / dt
-__device__ __forceinline__ void vbd_velocity_one(const PSView& ps, int i, float dt) {
-    const dvec3 P = dunpack(ps.p[i], ps.lo_unit), LP = dunpack(ps.last_p[i], ps.lo_unit);
+__device__ __forceinline__ void vbd_velocity_from(const PSView& ps, int i, float4 p, float4 last_p, float dt) {
+    const dvec3 P = dunpack(p, ps.lo_unit), LP = dunpack(last_p, ps.lo_unit);
     const double ddt = dt;
     ps.v[i] = f4(static_cast<float>((P.x - LP.x) / ddt), static_cast<float>((P.y - LP.y) / ddt),
                  static_cast<float>((P.z - LP.z) / ddt), 0.f);
-}
-
-__global__ __launch_bounds__(kBlock) void k_vbd_velocity(PSView ps, float dt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ps.n) return;
-    vbd_velocity_one(ps, i, dt);
-}
-
-// p = prev2 + omega (p - prev2) from the third iteration on; prev2 = prev1, prev1 = p
-__global__ __launch_bounds__(kBlock) void k_chebyshev(PSView ps, float4* prev_it_p, float4* prev_it2_p, int it,
-                                                      float omega) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ps.n) return;
-    float4 p = ps.p[i];
-    if (it >= 2) {
-        const dvec3 P = dunpack(p, ps.lo_unit), Q = dunpack(prev_it2_p[i], ps.lo_unit);
-        const double om = omega;
-        p = dpack(dvec3{Q.x + om * (P.x - Q.x), Q.y + om * (P.y - Q.y), Q.z + om * (P.z - Q.z)}, ps.lo_inv);
-        ps.p[i] = p;
-    }
-    prev_it2_p[i] = prev_it_p[i];
-    prev_it_p[i] = p;
 }
 
 // last_p = p ; v += (g + f w) dt ; p += v dt ; f = 0
@@ -102,21 +85,22 @@ __global__ __launch_bounds__(kBlock) void k_semi_implicit(PSView ps, float dt, f
     ps.f[i] = f4(0.f, 0.f, 0.f, 0.f);
 }
 
-__global__ __launch_bounds__(kBlock) void k_pbd_velocity(PSView ps, float dt, float global_damping) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ps.n) return;
-    const float4 p = ps.p[i], lp = ps.last_p[i];
+// v = (p - last_p) / dt, damped
+__device__ __forceinline__ void pbd_velocity_of(float4 p, float4 lp, float w, float dt, float global_damping,
+                                                float v[3]) {
     float vx = (p.x - lp.x) / dt, vy = (p.y - lp.y) / dt, vz = (p.z - lp.z) / dt;
     const float nv = sqrtf(vx * vx + vy * vy + vz * vz);
     if (nv > 1e-7f) {
-        const float coef = global_damping * dt * ps.w[i];
+        const float coef = global_damping * dt * w;
         const float damp = -nv * (coef > 1.f ? 1.f : coef);
         const float inv = 1.f / nv;
         vx += vx * inv * damp;
         vy += vy * inv * damp;
         vz += vz * inv * damp;
     }
-    ps.v[i] = f4(vx, vy, vz, 0.f);
+    v[0] = vx;
+    v[1] = vy;
+    v[2] = vz;
 }
 
 // target = offset + com + R (X - com), X = init_p (rest position);  p = target,
@@ -154,11 +138,10 @@ __device__ __forceinline__ bool box_clamp(float4& u, float4 X, const float pmin[
 }
 
 // The compensated form: the absolute position X + (hi + lo) in FP64 against the
-// box; a clamped component becomes bound - X (packed again); written only when
-// a component is clamped.
-__device__ __forceinline__ void box_clamp_comp(const PSView& ps, int i, float4 X, const float pmin[3],
+// box; a clamped component becomes bound - X (packed again).  True when a
+// component is clamped.
+__device__ __forceinline__ bool box_clamp_comp(float4& h, float unit, float inv, float4 X, const float pmin[3],
                                                const float pmax[3]) {
-    const float4 h = ps.p[i];
     // the low-order part (|lo| <= half an ulp of hi) can only matter within a
     // relative 1e-4 of a bound: elsewhere the float sum decides alone
     const float xf[3] = {X.x + h.x, X.y + h.y, X.z + h.z};
@@ -167,15 +150,106 @@ __device__ __forceinline__ void box_clamp_comp(const PSView& ps, int i, float4 X
     for (int k = 0; k < 3; ++k)
         near = near || xf[k] < pmin[k] + 1e-4f * (1.f + fabsf(pmin[k])) ||
                xf[k] > pmax[k] - 1e-4f * (1.f + fabsf(pmax[k]));
-    if (!near) return;
-    dvec3 U = dunpack(h, ps.lo_unit);
+    if (!near) return false;
+    dvec3 U = dunpack(h, unit);
     const double x = X.x + U.x, y = X.y + U.y, z = X.z + U.z;
     const bool cx = x < pmin[0] || x > pmax[0], cy = y < pmin[1] || y > pmax[1], cz = z < pmin[2] || z > pmax[2];
-    if (!(cx || cy || cz)) return;
+    if (!(cx || cy || cz)) return false;
     if (cx) U.x = fmin(fmax(x, static_cast<double>(pmin[0])), static_cast<double>(pmax[0])) - X.x;
     if (cy) U.y = fmin(fmax(y, static_cast<double>(pmin[1])), static_cast<double>(pmax[1])) - X.y;
     if (cz) U.z = fmin(fmax(z, static_cast<double>(pmin[2])), static_cast<double>(pmax[2])) - X.z;
-    ps.p[i] = dpack(U, ps.lo_inv);
+    h = dpack(U, inv);
+    return true;
+}
+
+// Fixation then box limit of one vertex whose record is u: a fixed vertex
+// (flag set) is snapped and masked, every other vertex with mask 1 is clamped -
+// the same result as k_fix then k_box, since the box skips masked vertices.
+// True when u changed; v, f and mask of a fixed vertex are stored here.
+__device__ __forceinline__ bool constrain(const PSView& ps, int i, float4& u, bool is_fixed, int mask, float4 X,
+                                          const float com[3], const float off[3], const float R[9], int has_box,
+                                          const float lo[3], const float hi[3]) {
+    if (is_fixed) {
+        u = fix_displacement(X, com, off, R);
+        gstore(ps.v, i, f4(0.f, 0.f, 0.f, 0.f));
+        gstore(ps.f, i, f4(0.f, 0.f, 0.f, 0.f));
+        gstore(ps.mask, i, 0);
+        return true;
+    }
+    if (!has_box || mask == 0) return false;
+    return ps.comp ? box_clamp_comp(u, ps.lo_unit, ps.lo_inv, X, lo, hi) : box_clamp(u, X, lo, hi);
+}
+
+// The same for one scene's constraints; the flag, the mask and the rest
+// position are loaded together (waiting on one another they cost three
+// round trips).
+__device__ __forceinline__ bool constrain(const PSView& ps, int i, float4& u, const VertexConstraints& c) {
+    if (!c.fixed && !c.has_box) return false;
+    const bool is_fixed = c.fixed && gload(c.fixed, i) != 0;
+    const int mask = gload(static_cast<const int*>(ps.mask), i);
+    const float4 X = gload(static_cast<const float4*>(ps.init_p), i);
+    return constrain(ps, i, u, is_fixed, mask, X, c.t.com, c.t.offset, c.t.R, c.has_box, c.lo, c.hi);
+}
+
+// One pass over the vertices after a VBD sweep (see VbdTailArgs).  Each of its
+// parts needs only the vertex's own records; as passes of their own they were
+// 2-3 us of launch each (two of six launches of an iteration of the P1
+// 64x16x16 beam with Chebyshev).  The predictor finds f = 0: the one that
+// opened the step cleared it, and only a fixation writes it since (zero).
+__global__ __launch_bounds__(kBlock) void k_vbd_tail(VbdTailArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const PSView& ps = a.ps;
+    if (i >= ps.n) return;
+    float4 p = gload(static_cast<const float4*>(ps.p), i);
+    float4 last = f4(0.f, 0.f, 0.f, 0.f), h1 = last, h2 = last;
+    if (a.velocity || a.predict) last = gload(static_cast<const float4*>(ps.last_p), i);
+    if (a.prev1) {
+        h1 = gload(static_cast<const float4*>(a.prev1), i);
+        h2 = gload(static_cast<const float4*>(a.prev2), i);
+    }
+    bool moved = constrain(ps, i, p, a.c);
+    if (a.prev1) {
+        // p = prev2 + omega (p - prev2) from the third iteration on; prev2 = prev1, prev1 = p
+        if (a.it >= 2) {
+            const dvec3 P = dunpack(p, ps.lo_unit), Q = dunpack(h2, ps.lo_unit);
+            const double om = a.omega;
+            p = dpack(dvec3{Q.x + om * (P.x - Q.x), Q.y + om * (P.y - Q.y), Q.z + om * (P.z - Q.z)}, ps.lo_inv);
+            moved = true;
+        }
+        gstore(a.prev2, i, h1);
+        gstore(a.prev1, i, p);
+    }
+    if (a.velocity) vbd_velocity_from(ps, i, p, last, a.dt);
+    if (a.predict)
+        vbd_predict_from(ps, a.y, i, p, last, f4(0.f, 0.f, 0.f, 0.f), 0.f, a.dt, a.g[0], a.g[1], a.g[2], a.prev1);
+    else if (moved)
+        gstore(ps.p, i, p);
+}
+
+// One pass over the vertices after the XPBD projections: constraints, velocity
+// and the next substep's k_semi_implicit (f = 0 since the last one; the
+// velocity in between is not stored).  Three passes of 2-3 us of launch each
+// before, of 12 in a substep of the 27-node 32x8x8 beam.
+__global__ __launch_bounds__(kBlock) void k_pbd_tail(PSView ps, VertexConstraints c, float dt, float global_damping,
+                                                     int next, float gx, float gy, float gz) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ps.n) return;
+    float4 p = gload(static_cast<const float4*>(ps.p), i);
+    const float4 lp = gload(static_cast<const float4*>(ps.last_p), i);
+    const float w = gload(ps.w, i);
+    const bool moved = constrain(ps, i, p, c);
+    float v[3];
+    pbd_velocity_of(p, lp, w, dt, global_damping, v);
+    if (!next) {
+        if (moved) gstore(ps.p, i, p);
+        gstore(ps.v, i, f4(v[0], v[1], v[2], 0.f));
+        return;
+    }
+    gstore(ps.last_p, i, p);
+    p.x += (v[0] + gx * dt) * dt;
+    p.y += (v[1] + gy * dt) * dt;
+    p.z += (v[2] + gz * dt) * dt;
+    gstore(ps.p, i, p);
 }
 
 __global__ __launch_bounds__(kBlock) void k_box(PSView ps, float3 pmin, float3 pmax) {
@@ -183,40 +257,10 @@ __global__ __launch_bounds__(kBlock) void k_box(PSView ps, float3 pmin, float3 p
     if (i >= ps.n) return;
     if (ps.mask[i] == 0) return;
     const float lo[3] = {pmin.x, pmin.y, pmin.z}, hi[3] = {pmax.x, pmax.y, pmax.z};
-    if (ps.comp) {
-        box_clamp_comp(ps, i, ps.init_p[i], lo, hi);
-        return;
-    }
     float4 u = ps.p[i];
-    if (box_clamp(u, ps.init_p[i], lo, hi)) ps.p[i] = u;   // written only when clamped
-}
-
-// Fixation then box limit over one scene's vertices, fused as in the batched
-// form: a fixed vertex (flag set) is snapped and masked, every other vertex
-// with mask 1 is clamped; the same result as k_fix then k_box, since the box
-// skips masked vertices.
-__global__ __launch_bounds__(kBlock) void k_fix_box(PSView ps, const unsigned char* fixed, FixTransform t, float3 pmin,
-                                                    float3 pmax) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ps.n) return;
-    const bool is_fixed = gload(fixed, i) != 0;
-    const int mask = gload(static_cast<const int*>(ps.mask), i);
-    float4 u = gload(static_cast<const float4*>(ps.p), i);
-    const float4 X = gload(static_cast<const float4*>(ps.init_p), i);
-    if (is_fixed) {
-        gstore(ps.p, i, fix_displacement(X, t.com, t.offset, t.R));
-        gstore(ps.v, i, f4(0.f, 0.f, 0.f, 0.f));
-        gstore(ps.f, i, f4(0.f, 0.f, 0.f, 0.f));
-        gstore(ps.mask, i, 0);
-        return;
-    }
-    if (mask == 0) return;
-    const float lo[3] = {pmin.x, pmin.y, pmin.z}, hi[3] = {pmax.x, pmax.y, pmax.z};
-    if (ps.comp) {
-        box_clamp_comp(ps, i, X, lo, hi);
-        return;
-    }
-    if (box_clamp(u, X, lo, hi)) gstore(ps.p, i, u);   // written only when clamped
+    const float4 X = ps.init_p[i];
+    if (ps.comp ? box_clamp_comp(u, ps.lo_unit, ps.lo_inv, X, lo, hi) : box_clamp(u, X, lo, hi))
+        ps.p[i] = u;   // written only when clamped
 }
 
 __global__ __launch_bounds__(kBlock) void k_copy_colour(PSView ps, const int* slot_vid, int first, int count,
@@ -236,12 +280,14 @@ __global__ __launch_bounds__(kBlock) void k_copy_colour(PSView ps, const int* sl
 // incidences are loaded at a time so that their loads overlap.  With
 // integrate set (a semi-implicit integrator whose only dynamic is this force
 // pass) the thread then runs k_semi_implicit's update of its vertex, the same
-// operations on the same values, and the separate pass is skipped.
+// operations on the same values, and the constraints; the separate passes are
+// skipped (2.9 us each of the 17.5 us of a 27-node 32x8x8 substep).
 constexpr int kExplicitVertexBlock = 64;
 __global__ __launch_bounds__(kExplicitVertexBlock) void k_explicit_vertex(PSView ps, OwnersView own,
                                                                           const float* partial, int count,
                                                                           float damping, int integrate, float dt,
-                                                                          float gx, float gy, float gz) {
+                                                                          float gx, float gy, float gz,
+                                                                          VertexConstraints c) {
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= count) return;
     const int vid = gload(own.slot_vid, slot);
@@ -280,9 +326,13 @@ __global__ __launch_bounds__(kExplicitVertexBlock) void k_explicit_vertex(PSView
     p.x += v.x * dt;
     p.y += v.y * dt;
     p.z += v.z * dt;
-    ps.v[vid] = v;
+    const bool is_fixed = c.fixed && gload(c.fixed, vid) != 0;   // constrain() stores v and f of a fixed vertex
+    if (!is_fixed) {
+        ps.v[vid] = v;
+        ps.f[vid] = f4(0.f, 0.f, 0.f, 0.f);
+    }
+    constrain(ps, vid, p, c);
     ps.p[vid] = p;
-    ps.f[vid] = f4(0.f, 0.f, 0.f, 0.f);
 }
 
 // Packed xyz of a run of records for the host.  The output is pinned host
@@ -353,19 +403,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_fix_box(BatchVArgs b) {
     const int mask = gload(static_cast<const int*>(ps.mask), i);
     float4 u = gload(static_cast<const float4*>(ps.p), i);
     const float4 X = gload(static_cast<const float4*>(ps.init_p), i);
-    if (is_fixed) {
-        gstore(ps.p, i, fix_displacement(X, sd.fix_com, sd.fix_offset, sd.fix_R));
-        gstore(ps.v, i, f4(0.f, 0.f, 0.f, 0.f));
-        gstore(ps.f, i, f4(0.f, 0.f, 0.f, 0.f));
-        gstore(ps.mask, i, 0);
-        return;
-    }
-    if (!sd.has_box || mask == 0) return;
-    if (ps.comp) {
-        box_clamp_comp(ps, i, X, sd.box_min, sd.box_max);
-        return;
-    }
-    if (box_clamp(u, X, sd.box_min, sd.box_max)) gstore(ps.p, i, u);   // written only when clamped
+    if (constrain(ps, i, u, is_fixed, mask, X, sd.fix_com, sd.fix_offset, sd.fix_R, sd.has_box, sd.box_min, sd.box_max))
+        gstore(ps.p, i, u);   // written only when it changed
 }
 
 __global__ __launch_bounds__(kBlock) void k_batch_velocity(BatchVArgs b) {
@@ -373,7 +412,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_velocity(BatchVArgs b) {
     const SceneDev& sd = vseg_scene(b, i, ok);
     if (!ok) return;
     const PSView ps = sd.ps;
-    vbd_velocity_one(ps, i, b.dt);
+    vbd_velocity_from(ps, i, gload(static_cast<const float4*>(ps.p), i), gload(static_cast<const float4*>(ps.last_p), i),
+                      b.dt);
 }
 
 }  // namespace
@@ -398,14 +438,9 @@ void launch_vbd_predict(const PSView& ps, float4* y, float4* prev_it_p, float dt
     hipLaunchKernelGGL(k_vbd_predict, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, y, prev_it_p, dt, g[0], g[1], g[2]);
 }
 
-void launch_vbd_velocity(const PSView& ps, float dt, hipStream_t s) {
-    if (ps.n <= 0) return;
-    hipLaunchKernelGGL(k_vbd_velocity, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, dt);
-}
-
-void launch_chebyshev(const PSView& ps, float4* prev_it_p, float4* prev_it2_p, int it, float omega, hipStream_t s) {
-    if (ps.n <= 0) return;
-    hipLaunchKernelGGL(k_chebyshev, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, prev_it_p, prev_it2_p, it, omega);
+void launch_vbd_tail(const VbdTailArgs& a, hipStream_t s) {
+    if (a.ps.n <= 0) return;
+    hipLaunchKernelGGL(k_vbd_tail, dim3(grid_for(a.ps.n)), dim3(kBlock), 0, s, a);
 }
 
 void launch_semi_implicit(const PSView& ps, float dt, const float g[3], hipStream_t s) {
@@ -413,21 +448,16 @@ void launch_semi_implicit(const PSView& ps, float dt, const float g[3], hipStrea
     hipLaunchKernelGGL(k_semi_implicit, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, dt, g[0], g[1], g[2]);
 }
 
-void launch_pbd_velocity(const PSView& ps, float dt, float global_damping, hipStream_t s) {
+void launch_pbd_tail(const PSView& ps, const VertexConstraints& c, float dt, float global_damping, bool next,
+                     const float g[3], hipStream_t s) {
     if (ps.n <= 0) return;
-    hipLaunchKernelGGL(k_pbd_velocity, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, dt, global_damping);
+    hipLaunchKernelGGL(k_pbd_tail, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, c, dt, global_damping, next ? 1 : 0,
+                       g[0], g[1], g[2]);
 }
 
 void launch_fix(const PSView& ps, const int* ids, int n, const FixTransform& t, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_fix, dim3(grid_for(n)), dim3(kBlock), 0, s, ps, ids, n, t);
-}
-
-void launch_fix_box(const PSView& ps, const unsigned char* fixed, const FixTransform& t, const float pmin[3],
-                    const float pmax[3], hipStream_t s) {
-    if (ps.n <= 0) return;
-    hipLaunchKernelGGL(k_fix_box, dim3(grid_for(ps.n)), dim3(kBlock), 0, s, ps, fixed, t,
-                       make_float3(pmin[0], pmin[1], pmin[2]), make_float3(pmax[0], pmax[1], pmax[2]));
 }
 
 void launch_box(const PSView& ps, const float pmin[3], const float pmax[3], hipStream_t s) {
@@ -437,12 +467,12 @@ void launch_box(const PSView& ps, const float pmin[3], const float pmax[3], hipS
 }
 
 void launch_explicit_vertex(const PSView& ps, const OwnersView& own, const float* partial, int count, float damping,
-                            const float* gravity, float dt, hipStream_t s) {
+                            const float* gravity, const VertexConstraints& c, float dt, hipStream_t s) {
     if (count <= 0) return;
     const float g0 = gravity ? gravity[0] : 0.f, g1 = gravity ? gravity[1] : 0.f, g2 = gravity ? gravity[2] : 0.f;
     hipLaunchKernelGGL(k_explicit_vertex, dim3((count + kExplicitVertexBlock - 1) / kExplicitVertexBlock),
                        dim3(kExplicitVertexBlock), 0, s, ps, own, partial, count, damping, gravity ? 1 : 0, dt, g0,
-                       g1, g2);
+                       g1, g2, c);
 }
 
 void launch_copy_colour(const PSView& ps, const int* slot_vid, int first, int count, const float4* p_new,

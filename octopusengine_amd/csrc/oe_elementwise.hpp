@@ -14,22 +14,47 @@ struct FixTransform {
     float R[9];   // column-major
 };
 
+// The constraints of an integrator that act on each vertex by itself: a
+// fixation (per-vertex flag, null = none) and a box limit after it.
+struct VertexConstraints {
+    const unsigned char* fixed = nullptr;
+    FixTransform t{};
+    int has_box = 0;
+    float lo[3] = {0.f, 0.f, 0.f}, hi[3] = {0.f, 0.f, 0.f};
+    bool any() const { return fixed || has_box; }
+};
+
 void launch_vbd_predict(const PSView& ps, float4* y, float4* prev_it_p, float dt, const float g[3], hipStream_t s);
-void launch_vbd_velocity(const PSView& ps, float dt, hipStream_t s);
-void launch_chebyshev(const PSView& ps, float4* prev_it_p, float4* prev_it2_p, int it, float omega, hipStream_t s);
+// What follows a VBD sweep, in one pass over the vertices and in this order:
+// the constraints; the Chebyshev step (prev1 / prev2 set, iteration it); the
+// velocity; the next substep's predictor.
+struct VbdTailArgs {
+    PSView ps;
+    float4* y;
+    float4* prev1;   // Chebyshev history, null = off
+    float4* prev2;
+    VertexConstraints c;
+    int it;
+    float omega;
+    int velocity;
+    int predict;
+    float dt;
+    float g[3];
+};
+void launch_vbd_tail(const VbdTailArgs& a, hipStream_t s);
 void launch_semi_implicit(const PSView& ps, float dt, const float g[3], hipStream_t s);
-void launch_pbd_velocity(const PSView& ps, float dt, float global_damping, hipStream_t s);
+// What follows the XPBD projections: constraints, velocity with the global
+// damping, and (next) the semi-implicit step of the next substep.
+void launch_pbd_tail(const PSView& ps, const VertexConstraints& c, float dt, float global_damping, bool next,
+                     const float g[3], hipStream_t s);
 void launch_fix(const PSView& ps, const int* ids, int n, const FixTransform& t, hipStream_t s);
 void launch_box(const PSView& ps, const float pmin[3], const float pmax[3], hipStream_t s);
-// launch_fix then launch_box in one pass over all vertices; fixed = per-vertex flag
-void launch_fix_box(const PSView& ps, const unsigned char* fixed, const FixTransform& t, const float pmin[3],
-                    const float pmax[3], hipStream_t s);
 // Explicit integrator: each vertex's internal force from the element partials
 // (9 floats per (element, local node), owners order) and the damping term.
 // With gravity set, the semi-implicit update (launch_semi_implicit) of the
-// vertex follows in the same thread.
+// vertex and the constraints follow in the same thread.
 void launch_explicit_vertex(const PSView& ps, const OwnersView& own, const float* partial, int count, float damping,
-                            const float* gravity, float dt, hipStream_t s);
+                            const float* gravity, const VertexConstraints& c, float dt, hipStream_t s);
 void launch_copy_colour(const PSView& ps, const int* slot_vid, int first, int count, const float4* p_new,
                         hipStream_t s);
 // Read-back: out[0 .. 3 count) = packed xyz of records first .. first + count

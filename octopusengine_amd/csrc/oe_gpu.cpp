@@ -189,32 +189,49 @@ void GPU_Integrator::eval_dynamics(GPU_ParticleSystem* ps, float dt) {
     for (auto& d : _dynamics)
         if (d->active) d->step(ps, dt);
 }
-// A fixation directly followed by a box limit (the order a scene adds them in)
-// runs as one fused pass; everything else in insertion order.
 void GPU_Integrator::eval_constraints(GPU_ParticleSystem* ps, float dt) {
-    for (size_t i = 0; i < _constraints.size(); ++i) {
-        GPU_Dynamic* c = _constraints[i].get();
-        if (!c->active) continue;
-        if (i + 1 < _constraints.size() && _constraints[i + 1]->active) {
-            auto* fix = dynamic_cast<GPU_Fix_Constraint*>(c);
-            auto* box = dynamic_cast<GPU_Box_Limit*>(_constraints[i + 1].get());
-            if (fix && box) {
-                launch_fix_box(ps->get_parameters(), fix->d_flags.get(), fix->t, box->pmin, box->pmax, fix->stream);
-                ++i;
-                continue;
-            }
-        }
-        c->step(ps, dt);
+    VbdTailArgs t{};   // constraints only: a fixation and a box limit in one pass
+    if (vertex_constraints(t.c) && t.c.fixed && t.c.has_box) {
+        t.ps = ps->get_parameters();
+        launch_vbd_tail(t, stream);
+        return;
     }
+    for (auto& c : _constraints)
+        if (c->active) c->step(ps, dt);
+}
+
+bool GPU_Integrator::vertex_constraints(VertexConstraints& out) const {
+    out = VertexConstraints{};
+    for (const auto& c : _constraints) {
+        if (!c->active) continue;
+        if (const auto* fix = dynamic_cast<const GPU_Fix_Constraint*>(c.get())) {
+            if (out.any()) return false;
+            out.fixed = fix->d_flags.get();
+            out.t = fix->t;
+        } else if (const auto* box = dynamic_cast<const GPU_Box_Limit*>(c.get())) {
+            if (out.has_box) return false;
+            out.has_box = 1;
+            std::copy(box->pmin, box->pmin + 3, out.lo);
+            std::copy(box->pmax, box->pmax + 3, out.hi);
+        } else {
+            return false;
+        }
+    }
+    return true;
 }
 
 void GPU_SemiExplicit::step(GPU_ParticleSystem* ps, float dt) {
     // A lone element-centric explicit force pass integrates in its own vertex
-    // pass (the same update as launch_semi_implicit, one launch fewer).
+    // pass (the same update as launch_semi_implicit, one launch fewer), and
+    // constrains there too when the constraints allow it.
     if (_dynamics.size() == 1 && _dynamics[0]->active)
-        if (auto* fe = dynamic_cast<GPU_FEM_Explicit*>(_dynamics[0].get()); fe && fe->step_integrate(ps, dt, gravity)) {
-            if (apply_constraints) eval_constraints(ps, dt);
-            return;
+        if (auto* fe = dynamic_cast<GPU_FEM_Explicit*>(_dynamics[0].get())) {
+            VertexConstraints c;
+            const bool fused = vertex_constraints(c) && apply_constraints;
+            if (fe->step_integrate(ps, dt, gravity, fused ? c : VertexConstraints{})) {
+                if (apply_constraints && !fused) eval_constraints(ps, dt);
+                return;
+            }
         }
     eval_dynamics(ps, dt);
     launch_semi_implicit(ps->get_parameters(), dt, gravity, stream);
@@ -242,31 +259,60 @@ void GPU_VBD::add_dynamics(GPU_Dynamic* d) {
     GPU_Integrator::add_dynamics(d);
 }
 
-void GPU_VBD::step(GPU_ParticleSystem* ps, float dt) {
-    const PSView v = ps->get_parameters();
+void GPU_VBD::run(GPU_ParticleSystem* ps, float dt, int n) {
     // rho > eps with the reference's eps = FLT_MIN * 1e6 (include/Core/Base.h:11)
     const bool cheb = _rho > std::numeric_limits<float>::min() * 1e6f;
-    init_dynamics(ps, dt);
-    launch_vbd_predict(v, y.get(), cheb ? prev_it_p.get() : nullptr, dt, gravity, stream);
-    float omega = 1.f;
-    for (int j = 0; j < iteration; ++j) {
-        eval_dynamics(ps, dt);
-        eval_constraints(ps, dt);
-        if (cheb) {
-            if (j == 1) omega = 2.f / (2.f - _rho * _rho);
-            else if (j > 1) omega = 4.f / (4.f - _rho * _rho * omega);
-            launch_chebyshev(v, prev_it_p.get(), prev_it2_p.get(), j, omega, stream);
+    VbdTailArgs t{};
+    t.ps = ps->get_parameters();
+    t.y = y.get();
+    t.dt = dt;
+    for (int d = 0; d < 3; ++d) t.g[d] = gravity[d];
+    const bool fused = vertex_constraints(t.c);
+    if (!fused) t.c = VertexConstraints{};
+    for (int k = 0; k < n; ++k) {
+        init_dynamics(ps, dt);
+        if (k == 0) launch_vbd_predict(t.ps, y.get(), cheb ? prev_it_p.get() : nullptr, dt, gravity, stream);
+        t.prev1 = cheb ? prev_it_p.get() : nullptr;
+        t.prev2 = cheb ? prev_it2_p.get() : nullptr;
+        float omega = 1.f;
+        for (int j = 0; j < iteration; ++j) {
+            eval_dynamics(ps, dt);
+            if (!fused) eval_constraints(ps, dt);
+            if (cheb) {
+                if (j == 1) omega = 2.f / (2.f - _rho * _rho);
+                else if (j > 1) omega = 4.f / (4.f - _rho * _rho * omega);
+            }
+            const bool last = j + 1 == iteration;
+            t.it = j;
+            t.omega = omega;
+            t.velocity = last;
+            t.predict = last && k + 1 < n;
+            if (cheb || last || t.c.any()) launch_vbd_tail(t, stream);
+        }
+        if (iteration == 0) {   // no sweep, no constraints: the predictor's positions are the step's
+            VbdTailArgs bare = t;
+            bare.prev1 = bare.prev2 = nullptr;
+            bare.c = VertexConstraints{};
+            bare.velocity = 1;
+            bare.predict = 0;
+            launch_vbd_tail(bare, stream);
+            if (k + 1 < n)
+                launch_vbd_predict(t.ps, y.get(), cheb ? prev_it_p.get() : nullptr, dt, gravity, stream);
         }
     }
-    launch_vbd_velocity(v, dt, stream);
 }
 
-void GPU_PBD::step(GPU_ParticleSystem* ps, float dt) {
+void GPU_PBD::run(GPU_ParticleSystem* ps, float dt, int n) {
     const PSView v = ps->get_parameters();
-    launch_semi_implicit(v, dt, gravity, stream);
-    eval_dynamics(ps, dt);
-    eval_constraints(ps, dt);
-    launch_pbd_velocity(v, dt, _global_damping, stream);
+    VertexConstraints c;
+    const bool fused = vertex_constraints(c);
+    if (!fused) c = VertexConstraints{};
+    if (n > 0) launch_semi_implicit(v, dt, gravity, stream);
+    for (int k = 0; k < n; ++k) {
+        eval_dynamics(ps, dt);
+        if (!fused) eval_constraints(ps, dt);
+        launch_pbd_tail(v, c, dt, _global_damping, k + 1 < n, gravity, stream);
+    }
 }
 
 // ---------------------------------------------------------------- GPU_FEM
@@ -635,19 +681,21 @@ void GPU_FEM_Explicit::step(GPU_ParticleSystem* ps, float dt) {
     if (tile.mode == PASS_TASKS) {
         ExplicitElemArgs ea{a.ps, a.fem, a.mt, d_inc_at.get(), d_partial.get()};
         if (!launch_explicit_elem(S, Q, ea, eng->stream)) throw std::invalid_argument("unsupported element");
-        launch_explicit_vertex(a.ps, a.own, d_partial.get(), n_vertices, _damping, nullptr, dt, eng->stream);
+        launch_explicit_vertex(a.ps, a.own, d_partial.get(), n_vertices, _damping, nullptr, VertexConstraints{}, dt,
+                               eng->stream);
         return;
     }
     if (!launch_gather(S, Q, tile.L, tile.QL, a, eng->stream)) throw std::invalid_argument("unsupported gather tile");
 }
 
-bool GPU_FEM_Explicit::step_integrate(GPU_ParticleSystem* ps, float dt, const float gravity[3]) {
+bool GPU_FEM_Explicit::step_integrate(GPU_ParticleSystem* ps, float dt, const float gravity[3],
+                                      const VertexConstraints& c) {
     if (tile.mode != PASS_TASKS || ps->n != n_vertices) return false;
     const PSView v = ps->get_parameters();
     ExplicitElemArgs ea{v, fem_view(), mt, d_inc_at.get(), d_partial.get()};
     if (!launch_explicit_elem(S, Q, ea, eng->stream)) throw std::invalid_argument("unsupported element");
     launch_explicit_vertex(v, OwnersView{d_slot_vid.get(), d_slot_nbo.get(), d_own.get()}, d_partial.get(), n_vertices,
-                           _damping, gravity, dt, eng->stream);
+                           _damping, gravity, c, dt, eng->stream);
     return true;
 }
 

@@ -114,6 +114,15 @@ struct GPU_Integrator : GPU_Dynamic {
     virtual void init_dynamics(GPU_ParticleSystem* ps, float dt);
     virtual void eval_dynamics(GPU_ParticleSystem* ps, float dt);
     virtual void eval_constraints(GPU_ParticleSystem* ps, float dt);
+    // n steps of dt.  The VBD and XPBD integrators run a step's last vertex
+    // pass and the next step's first one in one launch.
+    virtual void run(GPU_ParticleSystem* ps, float dt, int n) {
+        for (int i = 0; i < n; ++i) step(ps, dt);
+    }
+    // The active constraints as a per-vertex description (a fixation, a box
+    // limit, or a fixation and then a box limit, the order a scene adds them
+    // in); false for any other list, which eval_constraints runs one by one.
+    bool vertex_constraints(VertexConstraints& out) const;
 
     bool apply_constraints;
     float gravity[3] = {0.f, -9.81f, 0.f};
@@ -128,7 +137,8 @@ struct GPU_SemiExplicit final : GPU_Integrator {
 
 struct GPU_VBD final : GPU_Integrator {
     GPU_VBD(GPU_ParticleSystem* ps, int it, float rho);
-    void step(GPU_ParticleSystem* ps, float dt) override;
+    void step(GPU_ParticleSystem* ps, float dt) override { run(ps, dt, 1); }
+    void run(GPU_ParticleSystem* ps, float dt, int n) override;
     void add_dynamics(GPU_Dynamic* d) override;
     int iteration;
     float _rho;
@@ -137,7 +147,8 @@ struct GPU_VBD final : GPU_Integrator {
 
 struct GPU_PBD final : GPU_Integrator {
     explicit GPU_PBD(float global_damping = 0.f) : _global_damping(global_damping) {}
-    void step(GPU_ParticleSystem* ps, float dt) override;
+    void step(GPU_ParticleSystem* ps, float dt) override { run(ps, dt, 1); }
+    void run(GPU_ParticleSystem* ps, float dt, int n) override;
     float _global_damping;
 };
 
@@ -281,9 +292,9 @@ struct GPU_FEM_Explicit final : GPU_FEM {
     GPU_FEM_Explicit(Engine* eng, Element element, const HostMesh& mesh, float young, float poisson,
                      Material material, float damping);
     void step(GPU_ParticleSystem* ps, float dt) override;
-    // The element-centric pass followed by the semi-implicit update in its
-    // vertex pass; false (nothing launched) in the gather mode.
-    bool step_integrate(GPU_ParticleSystem* ps, float dt, const float gravity[3]);
+    // The element-centric pass followed by the semi-implicit update and the
+    // constraints in its vertex pass; false (nothing launched) in the gather mode.
+    bool step_integrate(GPU_ParticleSystem* ps, float dt, const float gravity[3], const VertexConstraints& c);
     float _damping;
     // mode PASS_TASKS (the default): element-centric force pass (one element
     // per 32 lanes, then a per-vertex sum of the element partials);
@@ -303,7 +314,7 @@ struct GPU_Fix_Constraint final : GPU_Dynamic {
     FixTransform t;
     std::vector<int> ids;
     DBuf<int> d_ids;
-    DBuf<unsigned char> d_flags;   // per vertex: 1 when fixed (the fused fix + box pass)
+    DBuf<unsigned char> d_flags;   // per vertex: 1 when fixed (the passes that constrain a vertex by itself)
     hipStream_t stream;
 };
 

@@ -86,7 +86,7 @@ void Scene::box_limit(const float pmin[3], const float pmax[3]) {
 
 void Scene::run_substeps(float dt, int substeps) {
     const float sub_dt = dt / static_cast<float>(substeps);
-    for (int i = 0; i < substeps; ++i) integrator->step(ps.get(), sub_dt);
+    integrator->run(ps.get(), sub_dt, substeps);
 }
 
 void Scene::set_graph(bool on) {
