@@ -307,6 +307,10 @@ void GPU_PBD::run(GPU_ParticleSystem* ps, float dt, int n) {
     VertexConstraints c;
     const bool fused = vertex_constraints(c);
     if (!fused) c = VertexConstraints{};
+    if (fused && n > 0 && _dynamics.size() == 1 && _dynamics[0]->active)
+        if (auto* fem = dynamic_cast<GPU_PBD_FEM*>(_dynamics[0].get());
+            fem && fem->run_resident(ps, c, dt, _global_damping, gravity, n))
+            return;
     if (n > 0) launch_semi_implicit(v, dt, gravity, stream);
     for (int k = 0; k < n; ++k) {
         eval_dynamics(ps, dt);
@@ -627,6 +631,44 @@ GPU_PBD_FEM::GPU_PBD_FEM(Engine* e, Element el, const HostMesh& mesh, float youn
     if (count_conflicts(g, colors) != 0) throw std::logic_error("element colouring has conflicts");
     sched = build_element_schedule(colors, E);
     d_eids = DBuf<int>(&eng->pool, std::vector<int>(sched.eids.begin(), sched.eids.end()));
+    if (el == Tetra) {
+        std::vector<float> host_rec, host_wq;   // one point: the same index in both record layouts
+        jxv.download(host_rec, eng->stream);
+        wq.download(host_wq, eng->stream);
+        std::vector<int4> nodes(E);
+        std::vector<float4> rec(3 * static_cast<size_t>(E));
+        for (int i = 0; i < E; ++i) {
+            const size_t e = static_cast<size_t>(sched.eids[i]);
+            const int32_t* t = &mesh.topo[4 * e];
+            nodes[i] = make_int4(t[0], t[1], t[2], t[3]);
+            const float* r = &host_rec[10 * e];
+            rec[3 * i] = make_float4(r[0], r[1], r[2], r[3]);
+            rec[3 * i + 1] = make_float4(r[4], r[5], r[6], r[7]);
+            rec[3 * i + 2] = make_float4(r[8], r[9] * host_wq[0], 0.f, 0.f);
+        }
+        d_p1_nodes = DBuf<int4>(&eng->pool, nodes);
+        d_p1_rec = DBuf<float4>(&eng->pool, rec);
+        d_color_begin = DBuf<int>(&eng->pool, std::vector<int>(sched.color_begin.begin(), sched.color_begin.end()));
+    }
+}
+
+bool GPU_PBD_FEM::run_resident(GPU_ParticleSystem* ps, const VertexConstraints& c, float dt, float global_damping,
+                               const float gravity[3], int n) {
+    if (S != 4 || ps->n > kXpbdResidentVertices) return false;
+    XpbdResidentArgs a{};
+    a.ps = ps->get_parameters();
+    a.mt = mt;
+    a.nodes = d_p1_nodes.get();
+    a.rec = d_p1_rec.get();
+    a.color_begin = d_color_begin.get();
+    a.n_colors = colors.nb_color;
+    a.c = c;
+    a.dt = dt;
+    a.global_damping = global_damping;
+    for (int d = 0; d < 3; ++d) a.g[d] = gravity[d];
+    a.substeps = n;
+    launch_xpbd_p1_resident(a, eng->stream);
+    return true;
 }
 
 void GPU_PBD_FEM::step(GPU_ParticleSystem* ps, float dt) {
@@ -639,6 +681,8 @@ void GPU_PBD_FEM::step(GPU_ParticleSystem* ps, float dt) {
     a.fem = fem_view();
     a.mt = mt;
     a.eids = d_eids.get();
+    a.p1_nodes = d_p1_nodes.get();
+    a.p1_rec = d_p1_rec.get();
     a.dt = dt;
     for (int c = 0; c < colors.nb_color; ++c) {
         a.first = sched.color_begin[c];

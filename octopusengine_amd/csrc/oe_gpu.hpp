@@ -282,10 +282,20 @@ struct GPU_PBD_FEM final : GPU_FEM {
     GPU_PBD_FEM(Engine* eng, Element element, const HostMesh& mesh, float young, float poisson, Material material,
                 XPBD_FEM_VERSION v = OptiShared);
     void step(GPU_ParticleSystem* ps, float dt) override;
+    // n substeps (predictor to velocity, constraints c) in one launch of one
+    // workgroup, for linear-tetrahedron scenes whose vertices fit its LDS;
+    // false (nothing launched) for any other scene.
+    bool run_resident(GPU_ParticleSystem* ps, const VertexConstraints& c, float dt, float global_damping,
+                      const float gravity[3], int n);
     Coloration colors;   // element colours
     ElementSchedule sched;
     XPBD_FEM_VERSION version;
     DBuf<int> d_eids;
+    // linear tetrahedra: the elements' node ids and records in schedule order
+    // (a colour's elements consecutive), and the colours' first elements
+    DBuf<int4> d_p1_nodes;
+    DBuf<float4> d_p1_rec;   // 3 per element: JX_inv (9), V
+    DBuf<int> d_color_begin;
 };
 
 struct GPU_FEM_Explicit final : GPU_FEM {

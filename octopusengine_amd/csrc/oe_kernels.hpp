@@ -137,13 +137,21 @@ __device__ __forceinline__ void jx_from_nodes(const float (&xs)[S][3], const flo
     }
 }
 
+// a0 b0 + a1 b1 + a2 b2 and a b - c d with their roundings written out: which
+// product of a sum the compiler fuses depends on what else uses the products,
+// so the same source would round differently from kernel to kernel.
+__device__ __forceinline__ float dot3(float a0, float b0, float a1, float b1, float a2, float b2) {
+    return fmaf(a2, b2, fmaf(a1, b1, a0 * b0));
+}
+__device__ __forceinline__ float diff2(float a, float b, float c, float d) { return fmaf(a, b, -(c * d)); }
+
 // F = Jx * JX_inv (both column-major)
 __device__ __forceinline__ void mat_mul(const float A[9], const float B[9], float C[9]) {
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int r = 0; r < 3; ++r)
-            C[c * 3 + r] = A[0 * 3 + r] * B[c * 3 + 0] + A[1 * 3 + r] * B[c * 3 + 1] + A[2 * 3 + r] * B[c * 3 + 2];
+            C[c * 3 + r] = dot3(A[r], B[c * 3], A[3 + r], B[c * 3 + 1], A[6 + r], B[c * 3 + 2]);
 }
 
 // Deformation gradient from nodal displacements u = x - X:
@@ -162,21 +170,21 @@ __device__ __forceinline__ void cofactor(const float F[9], float C[9]) {
     const float* a = F;       // column 0
     const float* b = F + 3;   // column 1
     const float* c = F + 6;   // column 2
-    C[0] = b[1] * c[2] - b[2] * c[1];
-    C[1] = b[2] * c[0] - b[0] * c[2];
-    C[2] = b[0] * c[1] - b[1] * c[0];
-    C[3] = c[1] * a[2] - c[2] * a[1];
-    C[4] = c[2] * a[0] - c[0] * a[2];
-    C[5] = c[0] * a[1] - c[1] * a[0];
-    C[6] = a[1] * b[2] - a[2] * b[1];
-    C[7] = a[2] * b[0] - a[0] * b[2];
-    C[8] = a[0] * b[1] - a[1] * b[0];
+    C[0] = diff2(b[1], c[2], b[2], c[1]);
+    C[1] = diff2(b[2], c[0], b[0], c[2]);
+    C[2] = diff2(b[0], c[1], b[1], c[0]);
+    C[3] = diff2(c[1], a[2], c[2], a[1]);
+    C[4] = diff2(c[2], a[0], c[0], a[2]);
+    C[5] = diff2(c[0], a[1], c[1], a[0]);
+    C[6] = diff2(a[1], b[2], a[2], b[1]);
+    C[7] = diff2(a[2], b[0], a[0], b[2]);
+    C[8] = diff2(a[0], b[1], a[1], b[0]);
 }
 
 // det F = column0 . cof column0.  Elements close to inversion (J < 0.1) get
 // the determinant re-evaluated in double precision.
 __device__ __forceinline__ float det_from_cof(const float F[9], const float C[9]) {
-    float J = F[0] * C[0] + F[1] * C[1] + F[2] * C[2];
+    float J = dot3(F[0], C[0], F[1], C[1], F[2], C[2]);
     if (J < 0.1f) {
         const double a0 = F[0], a1 = F[1], a2 = F[2], b0 = F[3], b1 = F[4], b2 = F[5], c0 = F[6], c1 = F[7], c2 = F[8];
         const double d = a0 * (b1 * c2 - b2 * c1) + a1 * (b2 * c0 - b0 * c2) + a2 * (b0 * c1 - b1 * c0);

@@ -13,6 +13,7 @@
 //    the node positions and per-quadrature stresses are staged in LDS.
 // Energies per material: src/GPU/PBD/GPU_PBD_FEM_Materials.cu:31-66,97-118.
 #include "oe_kernels.hpp"
+#include "oe_vertex.hpp"
 #include "oe_xpbd.hpp"
 
 namespace oe {
@@ -36,8 +37,8 @@ __device__ __forceinline__ void xpbd_material(int material, int m, float alpha, 
         } else {
             float n2 = 0.f;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) n2 += F[i] * F[i];
-            e = n2 - 3.f - 2.f * (J - 1.f);
+            for (int i = 0; i < 9; ++i) n2 = fmaf(F[i], F[i], n2);
+            e = fmaf(-2.f, J - 1.f, n2 - 3.f);
 #pragma unroll
             for (int i = 0; i < 9; ++i) P[i] = 2.f * F[i] - 2.f * C[i];
         }
@@ -50,7 +51,7 @@ __device__ __forceinline__ void xpbd_material(int material, int m, float alpha, 
         } else {
             float n2 = 0.f;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) n2 += F[i] * F[i];
+            for (int i = 0; i < 9; ++i) n2 = fmaf(F[i], F[i], n2);
             e = n2 - 3.f;
 #pragma unroll
             for (int i = 0; i < 9; ++i) P[i] = 2.f * F[i];
@@ -64,7 +65,7 @@ __device__ __forceinline__ void scale_stress(const float P[9], const float JXi[9
     for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int r = 0; r < 3; ++r)
-            Ps[c * 3 + r] = (P[0 * 3 + r] * JXi[0 * 3 + c] + P[1 * 3 + r] * JXi[1 * 3 + c] + P[2 * 3 + r] * JXi[2 * 3 + c]) * V;
+            Ps[c * 3 + r] = dot3(P[r], JXi[c], P[3 + r], JXi[3 + c], P[6 + r], JXi[6 + c]) * V;
 }
 
 template <int S, int Q>
@@ -131,11 +132,206 @@ __global__ __launch_bounds__(256) void k_xpbd_v0(XpbdArgs a) {
 // holds a few hundred elements, far too few to fill the chip, so a pass lasts
 // as long as one wave's chain of instructions: the sums are split over as many
 // lanes as an element can use, and LDS is read 16 bytes at a time.
+// One linear tetrahedron, both constraints: x the nodes' values, w their
+// inverse masses, free whether a node may move.  dN is (-1,-1,-1) and the unit
+// vectors, so Jx holds edge differences and the gradient of node k > 0 is
+// column k - 1 of the scaled stress: the sums of the general form with its zero
+// terms left out, the same bits.
+struct P1Element {
+    float JXi[9], V;
+};
+__device__ __forceinline__ P1Element p1_element(float4 r0, float4 r1, float4 r2) {
+    return P1Element{{r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x}, r2.y};
+}
+__device__ __forceinline__ void p1_project(const MaterialView& mt, float dt, const P1Element& el, const float (&w)[4],
+                                           const bool (&free)[4], float (&x)[4][3]) {
+    const float alpha_nh = 1.f + mt.mu / mt.lambda;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        float Jx[9], F[9], P[9], Ps[9], e;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) Jx[3 * c + r] = x[c + 1][r] - x[0][r];
+        deformation_gradient(Jx, el.JXi, F);
+        xpbd_material(mt.material, m, alpha_nh, F, P, e);
+        scale_stress(P, el.JXi, el.V, Ps);
+        const float C = sqrtf(fabsf(e * el.V));
+        const float Cinv = C < 1e-12f ? 0.f : 1.f / (2.f * C);
+        float grad[4][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            grad[0][r] = (-Ps[r] - Ps[3 + r] - Ps[6 + r]) * Cinv;
+            grad[1][r] = Ps[r] * Cinv;
+            grad[2][r] = Ps[3 + r] * Cinv;
+            grad[3][r] = Ps[6 + r] * Cinv;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            sum = fmaf(dot3(grad[k][0], grad[k][0], grad[k][1], grad[k][1], grad[k][2], grad[k][2]), w[k], sum);
+        const float stiff = (m == 0) ? mt.lambda : mt.mu;
+        const float alpha = 1.f / (stiff * dt * dt);
+        const float dl = -C / (sum + alpha);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float s = dl * w[k];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) x[k][r] = free[k] ? fmaf(s, grad[k][r], x[k][r]) : x[k][r];
+        }
+    }
+}
+
+// One thread per linear tetrahedron of a colour; the element's four nodes are
+// read once and written once for its two constraints.  Bound by the launch and
+// the chain nodes -> positions -> ~450 instructions; reading the nodes again
+// for the second constraint, after an element id and an index load, it took
+// 5.9 us per colour.
+__global__ __launch_bounds__(64) void k_xpbd_p1(XpbdArgs a) {
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= a.count) return;
+    const size_t i = static_cast<size_t>(a.first) + t;
+    const int4 n4 = gload(a.p1_nodes, i);
+    const float4 r0 = gload(a.p1_rec, 3 * i), r1 = gload(a.p1_rec, 3 * i + 1), r2 = gload(a.p1_rec, 3 * i + 2);
+    const int n[4] = {n4.x, n4.y, n4.z, n4.w};
+    float4 u[4];
+    float w[4], x[4][3];
+    bool free[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        u[k] = gload(static_cast<const float4*>(a.ps.p), n[k]);
+        w[k] = gload(a.ps.w, n[k]);
+        free[k] = gload(static_cast<const int*>(a.ps.mask), n[k]) != 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        x[k][0] = u[k].x;
+        x[k][1] = u[k].y;
+        x[k][2] = u[k].z;
+    }
+    p1_project(a.mt, a.dt, p1_element(r0, r1, r2), w, free, x);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (free[k]) gstore(a.ps.p, n[k], make_float4(x[k][0], x[k][1], x[k][2], u[k].w));
+}
+
+// The workgroup's LDS operations ordered for all of its waves.  Unlike
+// __syncthreads it names LDS alone, so loads in flight stay in flight.
+__device__ __forceinline__ void block_lds_sync() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// A run of substeps of a small linear-tetrahedron scene in one workgroup.  A
+// colour of such a scene is a wave or a few of work (59 elements on the
+// 16x4x4 beam), and a substep has ~28 of them: as launches the frame is the
+// launches.  Here the positions stay in LDS (xyz and the inverse mass, its
+// sign set on masked vertices), a colour boundary is a workgroup barrier, and
+// the next colour's element is loaded while the current one computes.  One
+// compute unit does all the work, so the form is for scenes whose positions fit
+// LDS (kXpbdResidentVertices), where a colour is at most ~6 waves.  The
+// arithmetic is that of k_xpbd_p1 and the vertex passes, in their order.
+constexpr int kXpbdResidentThreads = 512;
+__global__ __launch_bounds__(kXpbdResidentThreads) void k_xpbd_p1_resident(XpbdResidentArgs a) {
+    constexpr int T = kXpbdResidentThreads;
+    __shared__ float4 pos[kXpbdResidentVertices];
+    __shared__ float last[kXpbdResidentVertices * 3];
+    const int tid = threadIdx.x, n = a.ps.n;
+    // load, then the first semi-implicit step (k_semi_implicit)
+    for (int i = tid; i < n; i += T) {
+        float4 p = gload(static_cast<const float4*>(a.ps.p), i), v = gload(static_cast<const float4*>(a.ps.v), i);
+        const float4 f = gload(static_cast<const float4*>(a.ps.f), i);
+        const float w = gload(a.ps.w, i);
+        const int mask = gload(static_cast<const int*>(a.ps.mask), i);
+        last[3 * i] = p.x;
+        last[3 * i + 1] = p.y;
+        last[3 * i + 2] = p.z;
+        semi_implicit(p, v, f, w, a.dt, a.g[0], a.g[1], a.g[2]);
+        pos[i] = make_float4(p.x, p.y, p.z, mask != 0 ? w : -w);
+        gstore(a.ps.f, i, make_float4(0.f, 0.f, 0.f, 0.f));
+    }
+    // the thread's element of the next colour to come, loaded ahead
+    int4 nn = make_int4(0, 0, 0, 0);
+    float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
+    auto fetch = [&](int i) {
+        nn = gload(a.nodes, i);
+        r0 = gload(a.rec, 3 * i);
+        r1 = gload(a.rec, 3 * i + 1);
+        r2 = gload(a.rec, 3 * i + 2);
+    };
+    if (tid < a.color_begin[1]) fetch(tid);
+    for (int sub = 0; sub < a.substeps; ++sub) {
+        int begin = 0, end = a.color_begin[1];
+        for (int c = 0; c < a.n_colors; ++c) {
+            block_lds_sync();
+            const int nc = c + 1 < a.n_colors ? c + 1 : 0;   // after the last colour, the first of the next substep
+            const int nb = a.color_begin[nc], ne = a.color_begin[nc + 1];
+            for (int i = begin + tid; i < end; i += T) {
+                if (i >= begin + T) fetch(i);
+                const int nd[4] = {nn.x, nn.y, nn.z, nn.w};
+                const P1Element el = p1_element(r0, r1, r2);
+                if (i + T >= end && nb + tid < ne) fetch(nb + tid);
+                float w[4], x[4][3], ws[4];
+                bool free[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float4 u = pos[nd[k]];
+                    x[k][0] = u.x;
+                    x[k][1] = u.y;
+                    x[k][2] = u.z;
+                    ws[k] = u.w;
+                    w[k] = fabsf(u.w);
+                    free[k] = u.w > 0.f;
+                }
+                p1_project(a.mt, a.dt, el, w, free, x);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (free[k]) pos[nd[k]] = make_float4(x[k][0], x[k][1], x[k][2], ws[k]);
+            }
+            if (begin + tid >= end && nb + tid < ne) fetch(nb + tid);   // a thread without work in this colour
+            begin = nb;
+            end = ne;
+        }
+        block_lds_sync();
+        // k_pbd_tail
+        const bool next = sub + 1 < a.substeps;
+        for (int i = tid; i < n; i += T) {
+            const float4 q = pos[i];
+            const float4 lp = make_float4(last[3 * i], last[3 * i + 1], last[3 * i + 2], 0.f);
+            float4 p = make_float4(q.x, q.y, q.z, 0.f);
+            const float w = fabsf(q.w);
+            float ws = q.w;
+            if (a.c.fixed || a.c.has_box) {
+                const bool is_fixed = a.c.fixed && gload(a.c.fixed, i) != 0;
+                const float4 X = gload(static_cast<const float4*>(a.ps.init_p), i);
+                constrain(a.ps, i, p, is_fixed, q.w > 0.f ? 1 : 0, X, a.c.t.com, a.c.t.offset, a.c.t.R, a.c.has_box,
+                          a.c.lo, a.c.hi);
+                if (is_fixed) ws = -w;
+            }
+            float v[3];
+            pbd_velocity_of(p, lp, w, a.dt, a.global_damping, v);
+            if (!next) {
+                gstore(a.ps.p, i, make_float4(p.x, p.y, p.z, 0.f));
+                gstore(a.ps.last_p, i, lp);
+                gstore(a.ps.v, i, make_float4(v[0], v[1], v[2], 0.f));
+                continue;
+            }
+            last[3 * i] = p.x;
+            last[3 * i + 1] = p.y;
+            last[3 * i + 2] = p.z;
+            float4 vel = make_float4(v[0], v[1], v[2], 0.f);
+            semi_implicit(p, vel, make_float4(0.f, 0.f, 0.f, 0.f), 0.f, a.dt, a.g[0], a.g[1], a.g[2]);
+            pos[i] = make_float4(p.x, p.y, p.z, ws);
+        }
+    }
+}
+
 // NARROW (8-node hexahedra, 8 lanes): colours that fill the chip by themselves.
 template <int S, int Q, bool NARROW = false>
 struct V2Lanes;
 template <> struct V2Lanes<8, 8, true> { static constexpr int WP = 8, PP = 1, WN = 8, PN = 1; };
-template <> struct V2Lanes<4, 1> { static constexpr int WP = 4, PP = 1, WN = 4, PN = 1; };
 template <> struct V2Lanes<8, 8> { static constexpr int WP = 8, PP = 4, WN = 8, PN = 4; };
 template <> struct V2Lanes<10, 4> { static constexpr int WP = 4, PP = 4, WN = 16, PN = 1; };
 template <> struct V2Lanes<20, 11> { static constexpr int WP = 16, PP = 4, WN = 32, PN = 2; };
@@ -296,17 +492,23 @@ void launch_v2(const XpbdArgs& a, hipStream_t s) {
 
 }  // namespace
 
+void launch_xpbd_p1_resident(const XpbdResidentArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_xpbd_p1_resident, dim3(1), dim3(kXpbdResidentThreads), 0, s, a);
+}
+
 bool launch_xpbd(int S, int Q, bool v0_form, const XpbdArgs& a, hipStream_t s) {
     if (a.count <= 0) return true;
     if (v0_form) {
-        if (S == 4 && Q == 1) { launch_v0<4, 1>(a, s); return true; }
+        if (S == 4 && Q == 1) {
+            hipLaunchKernelGGL(k_xpbd_p1, dim3((a.count + 63) / 64), dim3(64), 0, s, a);
+            return true;
+        }
         if (S == 8 && Q == 8) { launch_v0<8, 8>(a, s); return true; }
         if (S == 10 && Q == 4) { launch_v0<10, 4>(a, s); return true; }
         if (S == 20 && Q == 11) { launch_v0<20, 11>(a, s); return true; }
         if (S == 27 && Q == 27) { launch_v0<27, 27>(a, s); return true; }
         return false;
     }
-    if (S == 4 && Q == 1) { launch_v2<4, 1>(a, s); return true; }
     if (S == 8 && Q == 8) {
         // 32 lanes per element up to two waves per SIMD (4,096 elements), 8 past
         // that: a substep of the 64x16x16 beam (2,048 elements per colour) takes

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "oe_device.hpp"
+#include "oe_elementwise.hpp"
 
 namespace oe {
 
@@ -19,7 +20,29 @@ struct XpbdArgs {
     int first;         // first element of the colour
     int count;         // elements in the colour
     float dt;
+    // linear tetrahedra: node ids and records (3 float4: JX_inv, V) of the
+    // elements in the order of eids
+    const int4* p1_nodes;
+    const float4* p1_rec;
 };
+
+// A whole run of substeps of a small linear-tetrahedron scene in one launch of
+// one workgroup (k_xpbd_p1_resident).
+constexpr int kXpbdResidentVertices = 2304;   // 28 bytes of LDS each, 63 KB
+struct XpbdResidentArgs {
+    PSView ps;
+    MaterialView mt;
+    const int4* nodes;        // as XpbdArgs::p1_nodes / p1_rec
+    const float4* rec;
+    const int* color_begin;   // n_colors + 1
+    int n_colors;
+    int substeps;
+    VertexConstraints c;
+    float dt;
+    float global_damping;
+    float g[3];
+};
+void launch_xpbd_p1_resident(const XpbdResidentArgs& a, hipStream_t s);
 
 // v0_form selects the sqrt-constraint formulation with the fixed-vertex mask
 // (reference kernel_XPBD_V0); otherwise the energy formulation of V1/V2.

@@ -67,3 +67,39 @@ def test_substeps_equal_single_steps(engine, kind, constraints):
             assert np.array_equal(a, b)
     for s in (many, one):
         s.close()
+
+
+def _disjoint_tetrahedra(n):
+    """n unit-corner tetrahedra apart from each other: one colour of n elements."""
+    ref = np.float32([(0, 0, 0), (0.02, 0, 0), (0, 0.02, 0), (0, 0, 0.02)])
+    at = np.stack(np.meshgrid(np.arange(24), np.arange(24), [0.0], indexing="ij"), -1).reshape(-1, 3)[:n]
+    xyz = (at[:, None, :] * 0.04 + ref[None]).reshape(-1, 3).astype(np.float32)
+    return xyz, np.arange(4 * n, dtype=np.int32).reshape(n, 4)
+
+
+@pytest.mark.parametrize("material", [oe.NEOHOOKE, oe.STABLE_NEOHOOKE])
+@pytest.mark.parametrize("mesh", [(1, 1, 1), (16, 4, 4), (35, 8, 6), (36, 8, 6), "disjoint"], ids=str)
+def test_small_linear_xpbd_equals_its_launches(engine, mesh, material):
+    """The one-workgroup run of a small linear XPBD scene (up to 2,304 vertices:
+    35x8x6 has 2,268, 36x8x6 has 2,331 and is launched colour by colour; 576
+    disjoint tetrahedra give one colour of more elements than threads) against
+    the launches of the same scene with its box limit added twice."""
+    xyz, topo = _disjoint_tetrahedra(576) if mesh == "disjoint" else oe.beam_mesh(oe.TETRA, mesh, (1.0, 0.25, 0.25))
+    scenes = []
+    for boxes in (1, 2):
+        s = oe.Scene(engine, oe.TETRA, xyz, topo, material=material, young=1e6, poisson=0.45, solver=oe.SOLVER_XPBD,
+                     global_damping=0.5)
+        s.fix_plane((1e-6, 0.0, 0.0), (-1.0, 0.0, 0.0))
+        for _ in range(boxes):
+            s.box_limit(LO, HI)
+        rng = np.random.default_rng(5)
+        p = (xyz + rng.uniform(-1e-3, 1e-3, xyz.shape)).astype(np.float32)
+        s.set_state(p=p, last_p=p, v=rng.standard_normal(xyz.shape).astype(np.float32))
+        for n in (1, 7, 20):
+            s.step(1e-3 * n, n)
+        scenes.append(s)
+    for a, b in zip(state(scenes[0]), state(scenes[1])):
+        assert np.array_equal(a, b)
+    assert np.isfinite(scenes[0].positions()).all()
+    for s in scenes:
+        s.close()
