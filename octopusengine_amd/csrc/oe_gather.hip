@@ -25,6 +25,10 @@
 //
 // This file is compiled once per element type (OE_GATHER_S / OE_GATHER_Q set
 // on the command line) so that the template instances build in parallel.
+#include <cmath>
+#include <stdexcept>
+#include <type_traits>
+
 #include "oe_gather.hpp"
 #include "oe_host.hpp"
 #include "oe_kernels.hpp"
@@ -305,33 +309,8 @@ __global__ __launch_bounds__(256) void k_batch_ju_refresh(BatchRefreshArgs b) {
 // takes the incidences t, t + kFusedThreads, ... of the vertex block.  Fixed
 // vertices are not skipped there: phase 2 skips them.
 //
-// The shape-derivative table is read through an accessor.  Tables of up to
-// 3 KB travel by value in the kernel arguments, so the Jx contraction (the
-// same point q on every lane) reads them with scalar loads; larger ones stay
-// in device memory.  dN_r(q) differs between lanes and always comes from the
-// table in device memory.
-template <int S, int Q>
-struct ShapeGrad {
-    float dN[Q * S * 3];
-};
-template <int S, int Q>
-constexpr bool grad_by_value() {
-    return Q * S * 3 * sizeof(float) <= 3072;
-}
-template <int S, int Q>
-struct GradByValue {
-    const ShapeGrad<S, Q>& g;
-    __device__ __forceinline__ float at(int i) const { return g.dN[i]; }
-};
-struct GradInMemory {
-    const float* dN;
-    __device__ __forceinline__ float at(int i) const { return gload(dN, i); }
-};
-// the kernel-argument table: the element's own, or a 1-point stand-in for
-// types whose table stays in device memory
-template <int S, int Q>
-using ShapeGradArg = ShapeGrad<S, (grad_by_value<S, Q>() ? Q : 1)>;
-
+// The Jx contraction reads the shape-derivative table from device memory, except
+// for quadratic tetrahedra, whose gradients follow from two scalars (P2Factors).
 template <int S, class Grad>
 __device__ __forceinline__ void jx_from_grad(const float (&xs)[S][3], const Grad& grad, int base, float Jx[9]) {
 #pragma unroll
@@ -347,6 +326,54 @@ __device__ __forceinline__ void jx_from_grad(const float (&xs)[S][3], const Grad
         }
     }
 }
+struct GradInMemory {
+    const float* dN;
+    __device__ __forceinline__ float at(int i) const { return gload(dN, i); }
+};
+
+// Quadratic tetrahedra.  With M_ii the corner and M_ij the edge values, u =
+// sum_i l_i (2 l_i - 1) M_ii + 4 sum_{i<j} l_i l_j M_ij in the barycentric
+// coordinates l, so the derivative along xi_c (l_c against l_0) is
+//   D_c = 4 sum_j l_j (M_cj - M_0j) - (M_cc - M_00).
+// The 4-point rule's points have three coordinates a and one b, the b at
+// corner q* = 1, 2, 3, 0, so with E_cj = M_cj - M_0j
+//   D_c(q) = 4a sum_j E_cj - E_cc - E_c0 + 4(b - a) E_c,q*
+// - 9 multiply-adds per point on a base shared by the four, against 90 per
+// point for the sum over the nodes (a third of the table is zero), and no
+// table reads in the point loop.
+struct P2Factors {
+    float a4, k4;   // 4a, 4(b - a)
+};
+constexpr int kP2Edge[4][4] = {{0, 4, 6, 7}, {4, 1, 5, 8}, {6, 5, 2, 9}, {7, 8, 9, 3}};   // node of M_ij
+constexpr int kP2Corner[4] = {1, 2, 3, 0};                                              // q* of point q
+struct P2Gradients {
+    float E[3][4][3];   // E_cj, c = 1..3
+    float base[9];      // column-major, column c - 1
+    __device__ __forceinline__ void init(const float (&x)[10][3], const P2Factors& f) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                float sum = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    E[c][j][k] = x[kP2Edge[c + 1][j]][k] - x[kP2Edge[0][j]][k];
+                    sum = j == 0 ? E[c][j][k] : sum + E[c][j][k];
+                }
+                base[3 * c + k] = fmaf(f.a4, sum, -(E[c][c + 1][k] + E[c][0][k]));
+            }
+    }
+    __device__ __forceinline__ void at(int corner, const P2Factors& f, float Jx[9]) const {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) Jx[3 * c + k] = fmaf(f.k4, E[c][corner][k], base[3 * c + k]);
+    }
+};
+// what a fused kernel takes besides its arguments: the P2 factors, or nothing
+struct NoFactors {};
+template <int S>
+using ShapeArg = std::conditional_t<S == 10, P2Factors, NoFactors>;
 
 // In the throughput form of the fused blocks, shape-derivative tables of at
 // most kDnLdsFloats floats (P1, P2, Q1) are copied to LDS, one copy per wave,
@@ -376,40 +403,54 @@ __device__ __forceinline__ void dnr_at(const FemView& f, const float* dnw, int q
 
 // Partial (force, Hessian) of local node r of element eid over its Q points.
 // dnw: the wave's LDS copy of the shape-derivative table (DNL only).
-template <int S, int Q, bool DNL, class Grad>
-__device__ __forceinline__ void elem_partial(const FemView& f, const MaterialView& mt, const Grad& grad, int eid,
-                                             int r, const float (&xs)[S][3], const float* dnw, Acc9& acc) {
+template <int S, int Q, bool DNL>
+__device__ __forceinline__ void elem_partial(const FemView& f, const MaterialView& mt, const ShapeArg<S>& shape,
+                                             int eid, int r, const float (&xs)[S][3], const float* dnw, Acc9& acc) {
     acc_zero(acc);
+    // affine: one record per element, JX_inv and |det B|, V_q = |det B| w_q
+    float JXi[9], detB = 0.f;
     if (f.affine) {
-        // one record per element: JX_inv and |det B|, V_q = |det B| w_q
-        float JXi[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) JXi[i] = gload(f.jxv, static_cast<size_t>(eid) * 10 + i);
-        const float detB = gload(f.jxv, static_cast<size_t>(eid) * 10 + 9);
-        // one point at a time: its 3S table entries fit the scalar registers
-#pragma unroll 1
+        detB = gload(f.jxv, static_cast<size_t>(eid) * 10 + 9);
+    }
+    float Ju[9], V = 0.f;
+    if constexpr (S == 10) {
+        // dN_r at the four points: issued here with the record's loads when it
+        // comes from memory (in the point loop each would be waited for)
+        float dnr[Q][3];
+        if constexpr (!DNL) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) load_dnr(f.dN, (q * S + r) * 3, dnr[q]);
+        }
+        V = detB * gload(f.wq, 0);   // the rule's four weights are equal (shape_arg)
+        P2Gradients g;
+        g.init(xs, shape);
+#pragma unroll
         for (int q = 0; q < Q; ++q) {
-            float Ju[9], dnr[3];
-            jx_from_grad<S>(xs, grad, q * S * 3, Ju);
-            dnr_at<S, Q, DNL>(f, dnw, q, r, dnr);
-            nh_contrib(Ju, JXi, detB * gload(f.wq, q), dnr, mt, acc);
+            g.at(kP2Corner[q], shape, Ju);
+            if constexpr (DNL) dnr_at<S, Q, DNL>(f, dnw, q, r, dnr[q]);
+            if (!f.affine) load_element_record(f, eid, q, JXi, V);
+            nh_contrib(Ju, JXi, V, dnr[q], mt, acc);
+            acc_settle(acc);   // or the four points' sums are formed together at the end (138 VGPRs, 3 waves)
         }
     } else {
 #pragma unroll 1
         for (int q = 0; q < Q; ++q) {
-            float Ju[9], JXi[9], V, dnr[3];
-            load_element_record(f, eid, q, JXi, V);
-            jx_from_grad<S>(xs, grad, q * S * 3, Ju);
+            float dnr[3];
+            jx_from_grad<S>(xs, GradInMemory{f.dN}, q * S * 3, Ju);
             dnr_at<S, Q, DNL>(f, dnw, q, r, dnr);
+            if (f.affine) V = detB * gload(f.wq, q);
+            else load_element_record(f, eid, q, JXi, V);
             nh_contrib(Ju, JXi, V, dnr, mt, acc);
         }
     }
 }
 
 // Phase 1 of a fused block: the partials of the block's incidences into LDS.
-template <int S, int Q, bool DNL, class Grad>
+template <int S, int Q, bool DNL>
 __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f, const OwnersView& own,
-                                             const MaterialView& mt, const Grad& grad, const int4 blk,
+                                             const MaterialView& mt, const ShapeArg<S>& grad, const int4 blk,
                                              float (*part)[9], float* dnw) {
     const int first_own = blk.z, n_inc = blk.w;
     const int t0 = threadIdx.x;
@@ -464,9 +505,9 @@ __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f,
 // every load in flight, the slot state's included.  (The throughput form keeps
 // the loop above: this form's prologue cost it 2%, 86.7 against 84.5 us per P2
 // batch pass on one GPU.)
-template <int S, int Q, class Grad, class AfterOwner, class AfterTopo>
+template <int S, int Q, class AfterOwner, class AfterTopo>
 __device__ __forceinline__ void fused_phase1_lat(const PSView& ps, const FemView& f, const OwnersView& own,
-                                                 const MaterialView& mt, const Grad& grad, const int4 blk,
+                                                 const MaterialView& mt, const ShapeArg<S>& grad, const int4 blk,
                                                  float (*part)[9], AfterOwner&& after_owner, AfterTopo&& after_topo) {
     static_assert(kFusedRuns == 1, "one incidence per thread");
     const int first_own = blk.z, n_inc = blk.w;
@@ -495,10 +536,10 @@ __device__ __forceinline__ void fused_phase1_lat(const PSView& ps, const FemView
     }
 }
 
-template <int S, int Q, bool LAT, class Grad>
+template <int S, int Q, bool LAT>
 __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, const OwnersView& own,
-                                            const MaterialView& mt, const Grad& grad, const float4* y, float damping,
-                                            float dt, const int4 blk, float (*part)[9], float* dnw) {
+                                            const MaterialView& mt, const ShapeArg<S>& grad, const float4* y,
+                                            float damping, float dt, const int4 blk, float (*part)[9], float* dnw) {
     const int first_slot = blk.x, n_slots = blk.y, first_own = blk.z;
     const int t0 = threadIdx.x;
     if constexpr (LAT) {
@@ -530,27 +571,16 @@ __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, 
 }
 
 template <int S, int Q, bool LAT>
-__device__ __forceinline__ void fused_dispatch(const PSView& ps, const FemView& f, const OwnersView& own,
-                                               const MaterialView& mt, const ShapeGradArg<S, Q>& g, const float4* y,
-                                               float damping, float dt, const int4 blk, float (*part)[9],
-                                               float* dnw) {
-    if constexpr (grad_by_value<S, Q>())
-        fused_block<S, Q, LAT>(ps, f, own, mt, GradByValue<S, Q>{g}, y, damping, dt, blk, part, dnw);
-    else
-        fused_block<S, Q, LAT>(ps, f, own, mt, GradInMemory{f.dN}, y, damping, dt, blk, part, dnw);
-}
-
-template <int S, int Q, bool LAT>
-__global__ __launch_bounds__(kFusedThreads) void k_fused_tasks(FusedTaskArgs a, ShapeGradArg<S, Q> g) {
+__global__ __launch_bounds__(kFusedThreads) void k_fused_tasks(FusedTaskArgs a, ShapeArg<S> g) {
     __shared__ float part[LAT ? kFusedIncPerBlockLat : kFusedIncPerBlock][9];
     __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, LAT>()];
     const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
-    fused_dispatch<S, Q, LAT>(a.ps, a.fem, a.own, a.mt, g, a.y, a.damping, a.dt, blk, part,
+    fused_block<S, Q, LAT>(a.ps, a.fem, a.own, a.mt, g, a.y, a.damping, a.dt, blk, part,
                               dn_lds[threadIdx.x >> 6]);
 }
 
 template <int S, int Q, bool LAT>
-__global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedArgs b, ShapeGradArg<S, Q> g) {
+__global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedArgs b, ShapeArg<S> g) {
     __shared__ float part[LAT ? kFusedIncPerBlockLat : kFusedIncPerBlock][9];
     __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, LAT>()];
     const int bid = xcd_block(blockIdx.x, gridDim.x);
@@ -565,7 +595,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedA
     const float4* y = sd.y;
     const float damping = sd.damping;
     const int4 blk = gload(LAT ? sd.fblocks_lat : sd.fblocks, seg.first + (bid - seg.block_begin));
-    fused_dispatch<S, Q, LAT>(ps, fem, own, mt, g, y, damping, b.dt, blk, part, dn_lds[threadIdx.x >> 6]);
+    fused_block<S, Q, LAT>(ps, fem, own, mt, g, y, damping, b.dt, blk, part, dn_lds[threadIdx.x >> 6]);
 }
 
 #endif
@@ -812,18 +842,32 @@ int OE_FN(refresh_elements_per_block_)() { return refresh_epb<OE_GATHER_Q>(); }
 
 #if OE_GATHER_S != 27
 namespace {
-// The element type's shape-derivative table as float, the values the scenes
-// upload as their dN (FemConstants), built once.
-const ShapeGradArg<OE_GATHER_S, OE_GATHER_Q>& shape_grad_arg() {
-    constexpr int S = OE_GATHER_S, Q = OE_GATHER_Q;
-    static const ShapeGradArg<S, Q> g = [] {
-        ShapeGradArg<S, Q> t{};
-        if constexpr (grad_by_value<S, Q>()) {
-            const Element el = S == 4 ? Tetra : S == 8 ? Hexa : S == 10 ? Tetra10 : S == 20 ? Tetra20 : Hexa27;
-            const ShapeTable& st = shape_table(el);
-            if (static_cast<int>(st.dN.size()) != Q * S * 3) throw std::logic_error("shape table size mismatch");
-            for (int i = 0; i < Q * S * 3; ++i) t.dN[i] = static_cast<float>(st.dN[i]);
-        }
+// The P2 factors from the element's quadrature points, checked against its
+// shape-derivative table (to float rounding: the reference's points are floats
+// whose coordinates add to 1 within an ulp).  Nothing for the other types.
+const ShapeArg<OE_GATHER_S>& shape_arg() {
+    static const ShapeArg<OE_GATHER_S> g = [] {
+        ShapeArg<OE_GATHER_S> t{};
+#if OE_GATHER_S == 10
+        const ShapeTable& st = shape_table(Tetra10);
+        const double b = st.qpoints[0], a = (1.0 - b) / 3.0;
+        for (int q = 0; q < 4; ++q)
+            for (int c = 1; c < 4; ++c) {
+                double want[10] = {};
+                for (int j = 0; j < 4; ++j) {
+                    const double l = j == kP2Corner[q] ? b : a;
+                    want[kP2Edge[c][j]] += 4.0 * l;
+                    want[kP2Edge[0][j]] -= 4.0 * l;
+                }
+                want[c] -= 1.0;
+                want[0] += 1.0;
+                for (int k = 0; k < 10; ++k)
+                    if (st.weights[q] != st.weights[0] || std::fabs(want[k] - st.dN[(q * 10 + k) * 3 + c - 1]) > 5e-7)
+                        throw std::logic_error("the P2 table does not have the 4-point rule's form");
+            }
+        t.a4 = static_cast<float>(4.0 * a);
+        t.k4 = static_cast<float>(4.0 * (b - a));
+#endif
         return t;
     }();
     return g;
@@ -834,20 +878,20 @@ void OE_FN(launch_fused_tasks_)(const FusedTaskArgs& a, hipStream_t s) {
     if (a.count <= 0) return;
     if (a.latency)
         hipLaunchKernelGGL((k_fused_tasks<OE_GATHER_S, OE_GATHER_Q, true>), dim3(a.count), dim3(kFusedThreads), 0, s, a,
-                           shape_grad_arg());
+                           shape_arg());
     else
         hipLaunchKernelGGL((k_fused_tasks<OE_GATHER_S, OE_GATHER_Q, false>), dim3(a.count), dim3(kFusedThreads), 0, s,
-                           a, shape_grad_arg());
+                           a, shape_arg());
 }
 
 void OE_FN(launch_batch_fused_tasks_)(const BatchFusedArgs& b, int nblocks, hipStream_t s) {
     if (nblocks <= 0) return;
     if (b.latency)
         hipLaunchKernelGGL((k_batch_fused_tasks<OE_GATHER_S, OE_GATHER_Q, true>), dim3(nblocks), dim3(kFusedThreads), 0,
-                           s, b, shape_grad_arg());
+                           s, b, shape_arg());
     else
         hipLaunchKernelGGL((k_batch_fused_tasks<OE_GATHER_S, OE_GATHER_Q, false>), dim3(nblocks), dim3(kFusedThreads),
-                           0, s, b, shape_grad_arg());
+                           0, s, b, shape_arg());
 }
 
 #endif

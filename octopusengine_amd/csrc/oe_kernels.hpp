@@ -62,6 +62,15 @@ __device__ __forceinline__ void acc_zero(Acc9& a) {
     for (int i = 0; i < 9; ++i) a.v[i] = 0.f;
 }
 
+// The sums as they are here: the empty asm takes them as inputs and outputs,
+// so the compiler cannot move the additions past this point (and hold their
+// terms in registers until then).
+__device__ __forceinline__ void acc_settle(Acc9& a) {
+    asm volatile(""
+                 : "+v"(a.v[0]), "+v"(a.v[1]), "+v"(a.v[2]), "+v"(a.v[3]), "+v"(a.v[4]), "+v"(a.v[5]), "+v"(a.v[6]),
+                   "+v"(a.v[7]), "+v"(a.v[8]));
+}
+
 // Sum over groups of L consecutive lanes (L a power of two, L <= 64).
 template <int L>
 __device__ __forceinline__ float group_sum(float x) {
@@ -139,9 +148,11 @@ __device__ __forceinline__ void jx_from_nodes(const float (&xs)[S][3], const flo
 
 // a0 b0 + a1 b1 + a2 b2 and a b - c d with their roundings written out: which
 // product of a sum the compiler fuses depends on what else uses the products,
-// so the same source would round differently from kernel to kernel.
+// so the same source would round differently from kernel to kernel.  dot3 adds
+// its first product last: with the largest product there (the diagonal of F or
+// cof F, near 1) the sum is rounded once at that size.
 __device__ __forceinline__ float dot3(float a0, float b0, float a1, float b1, float a2, float b2) {
-    return fmaf(a2, b2, fmaf(a1, b1, a0 * b0));
+    return fmaf(a0, b0, fmaf(a1, b1, a2 * b2));
 }
 __device__ __forceinline__ float diff2(float a, float b, float c, float d) { return fmaf(a, b, -(c * d)); }
 
@@ -202,8 +213,8 @@ __device__ __forceinline__ float det_from_cof(const float F[9], const float C[9]
 // The reference assembles H_r from six 3x3 blocks of d2W/dF2; the
 // lambda (J - alpha) d2J/dF2 blocks are antisymmetric and cancel in the
 // symmetric assembly, which leaves the closed form above.
-__device__ __forceinline__ void nh_node(const float F[9], const float C[9], float s, float V, const float g[3],
-                                        const MaterialView& mt, Acc9& a);
+// The two parts of P g nearly cancel in a relaxed stable Neo-Hookean element:
+// they are added before V scales them and before the sum over the points.
 __device__ __forceinline__ void nh_contrib(const float Jx[9], const float JXi[9], float V, const float* __restrict__ dnr,
                                            const MaterialView& mt, Acc9& a) {
     float F[9];
@@ -211,37 +222,29 @@ __device__ __forceinline__ void nh_contrib(const float Jx[9], const float JXi[9]
     // g_c = sum_l JX_inv(l, c) dN_r[l]
     float g[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) g[c] = JXi[c * 3 + 0] * dnr[0] + JXi[c * 3 + 1] * dnr[1] + JXi[c * 3 + 2] * dnr[2];
+    for (int c = 0; c < 3; ++c) g[c] = dot3(JXi[c * 3], dnr[0], JXi[c * 3 + 1], dnr[1], JXi[c * 3 + 2], dnr[2]);
     float C[9];
     cofactor(F, C);
     const float J = det_from_cof(F, C);
-    const float s = mt.lambda * (J - mt.alpha);
-    nh_node(F, C, s, V, g, mt, a);
-}
-
-// The part of nh_contrib that depends on node r (through g = JX_inv^T dN_r),
-// given the point's F, cof F and s = lambda (J - alpha): element-centric
-// callers form those once per point and add every node's terms.
-__device__ __forceinline__ void nh_node(const float F[9], const float C[9], float s, float V, const float g[3],
-                                        const MaterialView& mt, Acc9& a) {
+    const float sl = mt.lambda * (J - mt.alpha), Vmu = V * mt.mu, Vl = V * mt.lambda;
     // P g = mu F g + s C g ; c = C g
     float cg[3], Fg[3];
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
-        cg[r] = C[r] * g[0] + C[3 + r] * g[1] + C[6 + r] * g[2];
-        Fg[r] = F[r] * g[0] + F[3 + r] * g[1] + F[6 + r] * g[2];
+        const int s = (r + 1) % 3, t = (r + 2) % 3;
+        cg[r] = dot3(C[4 * r], g[r], C[3 * s + r], g[s], C[3 * t + r], g[t]);
+        Fg[r] = dot3(F[4 * r], g[r], F[3 * s + r], g[s], F[3 * t + r], g[t]);
     }
 #pragma unroll
-    for (int r = 0; r < 3; ++r) a.v[r] -= V * (mt.mu * Fg[r] + s * cg[r]);
-    const float gg = g[0] * g[0] + g[1] * g[1] + g[2] * g[2];
-    const float d = V * mt.mu * gg;
-    const float l = V * mt.lambda;
-    a.v[3] += d + l * cg[0] * cg[0];
-    a.v[4] += l * cg[1] * cg[0];
-    a.v[5] += l * cg[2] * cg[0];
-    a.v[6] += d + l * cg[1] * cg[1];
-    a.v[7] += l * cg[2] * cg[1];
-    a.v[8] += d + l * cg[2] * cg[2];
+    for (int r = 0; r < 3; ++r) a.v[r] = fmaf(-V, fmaf(mt.mu, Fg[r], sl * cg[r]), a.v[r]);
+    const float gg = dot3(g[0], g[0], g[1], g[1], g[2], g[2]);
+    const float l0 = Vl * cg[0], l1 = Vl * cg[1], l2 = Vl * cg[2];
+    a.v[3] = fmaf(l0, cg[0], fmaf(Vmu, gg, a.v[3]));
+    a.v[4] = fmaf(l1, cg[0], a.v[4]);
+    a.v[5] = fmaf(l2, cg[0], a.v[5]);
+    a.v[6] = fmaf(l1, cg[1], fmaf(Vmu, gg, a.v[6]));
+    a.v[7] = fmaf(l2, cg[1], a.v[7]);
+    a.v[8] = fmaf(l2, cg[2], fmaf(Vmu, gg, a.v[8]));
 }
 
 // Residual force of the local VBD problem at the current position
