@@ -64,11 +64,13 @@ SceneDev make_scene_dev(Scene& s, const unsigned char* fixed, const std::map<int
     if (t.mode == PASS_TASKS && s.mesh.element == Hexa27 && !s.vbd_fem->has_q2_basis)
         throw std::invalid_argument("no tensor factors for this 27-node hexahedron");
     d.ju = t.mode == PASS_CACHE ? s.vbd_fem->ensure_ju() : nullptr;
-    d.fblocks = d.fblocks_lat = nullptr;
+    d.fblocks = d.fblocks_lat = d.fblocks_split = nullptr;
     if (t.mode == PASS_TASKS) {
         d.fblocks = s.vbd_fem->throughput_tables(t.inc).blocks.get();
         const TaskTables* lt = s.vbd_fem->latency_tables();
         d.fblocks_lat = lt ? lt->blocks.get() : nullptr;
+        const TaskTables* sp = s.vbd_fem->split_form();
+        d.fblocks_split = sp ? sp->blocks.get() : nullptr;
     }
     d.ps = s.ps->get_parameters();
     d.fem = s.fem->fem_view();
@@ -138,13 +140,15 @@ void Schedule::build(const std::vector<Scene*>& scenes, const std::vector<int>& 
             const GatherTile et = tile_of(tiles, el);
             if (want_latency && et.mode == PASS_TASKS) {
                 bool all = true;
-                int64_t through_blocks = 0;
+                int64_t through_blocks = 0, incidences = 0;
                 for (Scene* s : scenes) {
                     if (s->mesh.element != el || c >= s->vbd_fem->nb_colors()) continue;
                     if (!s->vbd_fem->latency_tables()) all = false;
                     through_blocks += s->vbd_fem->throughput_tables(et.inc).color_blocks(c);
+                    incidences += s->vbd_fem->owners.color_incidences[c];
                 }
-                gl.latency = all && through_blocks < et.lat_blocks;
+                if (all && through_blocks < et.lat_blocks)
+                    gl.form = el == Tetra10 && incidences <= kSplitIncidences ? TASKS_SPLIT : TASKS_LATENCY;
             }
             bool any = false;
             for (size_t i = 0; i < scenes.size(); ++i) {
@@ -166,8 +170,9 @@ void Schedule::build(const std::vector<Scene*>& scenes, const std::vector<int>& 
                 }
                 if (gl.mode == PASS_TASKS) {
                     // fused tasks: one block per vertex block of the colour
-                    const TaskTables* tt =
-                        gl.latency ? s->vbd_fem->latency_tables() : &s->vbd_fem->throughput_tables(t.inc);
+                    const TaskTables* tt = gl.form == TASKS_SPLIT     ? s->vbd_fem->split_form()
+                                           : gl.form == TASKS_LATENCY ? s->vbd_fem->latency_tables()
+                                                                      : &s->vbd_fem->throughput_tables(t.inc);
                     if (!tt) throw std::logic_error("vertex blocks not prepared");
                     const int nfb = tt->color_blocks(c);
                     segs.push_back(BatchSeg{table_index[i], tt->color_begin[c], nfb, gl.nblocks});
@@ -314,15 +319,15 @@ void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const Scene
                 if (gl.mode == PASS_TASKS && is_q2(gl)) {
                     tk.seg_first = gl.seg_first;
                     tk.seg_count = gl.seg_count;
-                    tk.latency = gl.latency ? 1 : 0;
-                    if (!gl.latency && q2_pencil(gl.inc))
+                    tk.latency = gl.form == TASKS_LATENCY ? 1 : 0;
+                    if (gl.form == TASKS_THROUGHPUT && q2_pencil(gl.inc))
                         launch_batch_q2_pencil(tk, gl.nblocks, ls);
                     else
                         launch_batch_q2_fused(tk, gl.nblocks, ls);
                 } else if (gl.mode == PASS_TASKS) {
                     ft.seg_first = gl.seg_first;
                     ft.seg_count = gl.seg_count;
-                    ft.latency = gl.latency ? 1 : 0;
+                    ft.form = gl.form;
                     if (!launch_batch_fused_tasks(gl.S, gl.Q, ft, gl.nblocks, ls))
                         throw std::invalid_argument("unsupported element in batch");
                 } else if (!launch_batch_gather(gl.S, gl.Q, gl.L, gl.QL, gl.mode == PASS_CACHE, g, gl.nblocks, ls)) {

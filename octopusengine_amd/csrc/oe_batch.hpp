@@ -35,7 +35,7 @@ struct Schedule {
     struct GLaunch {
         int color, element, S, Q, L, QL;
         int mode;                         // PassMode
-        bool latency;                     // task pass in the kernels' latency form
+        int form;                         // of a task pass: TaskForm (27-node hexahedra: throughput or latency)
         int inc = 0;                      // task pass: the tile's incidences per throughput-form block
         int seg_first, seg_count, nblocks;   // gather: slot ranges; tasks: vertex-block ranges
         int64_t slots;   // vertex slots covered (all scenes)

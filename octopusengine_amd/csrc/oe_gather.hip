@@ -304,11 +304,207 @@ __global__ __launch_bounds__(256) void k_batch_ju_refresh(BatchRefreshArgs b) {
     ju_refresh_block<S, Q>(sd.ps.p, sd.ps.lo_unit, sd.fem, sd.ju, e0, ne);
 }
 
-#if !defined(OE_GATHER_S) || OE_GATHER_S != 27   // 27-node hexahedra have their own task kernels
+#if OE_GATHER_S != 27   // 27-node hexahedra have their own task kernels
 // Fused element tasks (see FusedTaskArgs).  Phase 1: thread t of the block
 // takes the incidences t, t + kFusedThreads, ... of the vertex block.  Fixed
 // vertices are not skipped there: phase 2 skips them.
 //
+// Point tasks: the task form with an incidence's points spread over LQ lanes
+// (LQ PPL >= Q), for linear tetrahedra (1 lane), 8-node hexahedra (8), 20-node
+// tetrahedra (4 lanes, 3 points each) and, in launches too small to fill the
+// chip, quadratic tetrahedra (4).  A pass of a single scene lasts as long as one
+// wave's chain of loads and instructions (about 2 ns each): the gather runs
+// ceil(incidences Q / L) work items per lane in turn, each loading and unpacking
+// all S nodes; here a lane loads S / LQ nodes, passes them to its group through
+// LDS, and runs one point.  Against the gather (the former default): a frame of
+// 4 steps of the 64x16x16 beam Q1 4.35 -> 2.72 ms, P1 1.24 -> 1.18 ms; 16 P3
+// beams of 32x8x8 in a batch 22.6 -> 8.2 ms a step.  Against a thread per
+// incidence: a step of the quadratic 16x4x4 beam 721 -> 627 us.
+// A block takes a vertex block's incidences kFusedThreads / LQ at a time (more
+// than one round only for vertices of very many elements).
+template <int S>
+constexpr int point_lanes() { return S == 4 ? 1 : S == 8 ? 8 : 4; }
+
+template <int S, int Q>
+struct PointLDS {
+    static constexpr int LQ = point_lanes<S>(), G = kFusedThreads / LQ;
+    // node values per group; the odd row stride spreads the groups over the banks
+    float4 xs[LQ > 1 ? G : 1][LQ > 1 ? (S | 1) : 1];
+    float part[kFusedIncPerBlock][9];
+    float dn[LQ > 1 ? Q * S * 3 : 1];   // (k Q + q) 3 + c: neighbouring lanes read neighbouring words
+};
+
+// lane 0 of each group of LQ lanes, in every lane of the group
+template <int LQ>
+__device__ __forceinline__ float group_first(float x) {
+    const int v = __float_as_int(x);
+    if constexpr (LQ == 4) return __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x00, 0xF, 0xF, false));
+    if constexpr (LQ == 8) {
+        // row_newbcast 0 and 8: lanes 0 and 8 of each 16-lane row
+        const int a = __builtin_amdgcn_update_dpp(0, v, 0x150, 0xF, 0xF, false);
+        const int b = __builtin_amdgcn_update_dpp(0, v, 0x158, 0xF, 0xF, false);
+        return __int_as_float((threadIdx.x & 8) ? b : a);
+    }
+    return x;
+}
+
+template <int S, int Q>
+__device__ __forceinline__ void point_block(const PSView& ps, const FemView& f, const OwnersView& own,
+                                            const MaterialView& mt, const float4* y, float damping, float dt,
+                                            const int4 blk, PointLDS<S, Q>& sh) {
+    constexpr int LQ = PointLDS<S, Q>::LQ, G = PointLDS<S, Q>::G;
+    constexpr int PPL = (Q + LQ - 1) / LQ, NPL = (S + LQ - 1) / LQ;
+    const int first_slot = blk.x, n_slots = blk.y, first_own = blk.z, n_inc = blk.w;
+    const int t0 = threadIdx.x, g = t0 / LQ, sub = t0 % LQ;
+    // loads in the order of the chain owners entry -> node ids -> positions; the
+    // slot's state rides along (see slot_state_level1)
+    int pk = gload(own.own, first_own + min(g, n_inc - 1));
+    SlotState st{};
+    slot_state_level1(own, first_slot + min(t0, n_slots - 1), st);
+    constexpr int kStage = LQ > 1 ? (Q * S * 3 + kFusedThreads - 1) / kFusedThreads : 1;
+    float stage[kStage];
+    if constexpr (LQ > 1) {
+#pragma unroll
+        for (int j = 0; j < kStage; ++j) {
+            const int i = min(t0 + kFusedThreads * j, Q * S * 3 - 1);
+            const int k = i / (3 * Q), q = i / 3 % Q, c = i % 3;
+            stage[j] = gload(f.dN, (q * S + k) * 3 + c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int nid[NPL];
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) nid[j] = gload(f.topo, static_cast<size_t>(pk >> 5) * S + min(sub + LQ * j, S - 1));
+    slot_state_level2(ps, y, st);
+    const bool busy = __builtin_amdgcn_readfirstlane(g) < n_inc;   // the wave has an incidence in the first round
+    if constexpr (LQ > 1) {
+#pragma unroll
+        for (int j = 0; j < kStage; ++j) sh.dn[min(t0 + kFusedThreads * j, Q * S * 3 - 1)] = stage[j];
+    }
+    for (int base = 0; base < n_inc; base += G) {
+        const bool has = base + g < n_inc;
+        if (base > 0) {
+            pk = gload(own.own, first_own + min(base + g, n_inc - 1));
+#pragma unroll
+            for (int j = 0; j < NPL; ++j)
+                nid[j] = gload(f.topo, static_cast<size_t>(pk >> 5) * S + min(sub + LQ * j, S - 1));
+        }
+        const int eid = pk >> 5, r = pk & 31;
+        float xs[LQ > 1 ? 1 : S][3];
+        float JXi[9], detB = 0.f, V = 0.f, dnr[3];
+        if (busy) {
+            float4 h[NPL];
+#pragma unroll
+            for (int j = 0; j < NPL; ++j) h[j] = gload(static_cast<const float4*>(ps.p), nid[j]);
+            if (f.affine) {
+#pragma unroll
+                for (int i = 0; i < 9; ++i) JXi[i] = gload(f.jxv, static_cast<size_t>(eid) * 10 + i);
+                detB = gload(f.jxv, static_cast<size_t>(eid) * 10 + 9);
+                V = detB * gload(f.wq, min(sub, Q - 1));
+            } else {
+                load_element_record(f, eid, min(sub, Q - 1), JXi, V);
+            }
+            if constexpr (LQ == 1) load_dnr(f.dN, 3 * r, dnr);
+            float4 ref = h[0];   // node 0 is lane 0's first
+            ref.x = group_first<LQ>(ref.x);
+            ref.y = group_first<LQ>(ref.y);
+            ref.z = group_first<LQ>(ref.z);
+            if constexpr (LQ == 1) {
+#pragma unroll
+                for (int k = 0; k < S; ++k) rel_node(h[k], ref, ps.lo_unit, xs[k]);
+            } else {
+                if (base > 0) wave_lds_sync();   // the group has read the last round's values
+#pragma unroll
+                for (int j = 0; j < NPL; ++j) {
+                    float d[3];
+                    rel_node(h[j], ref, ps.lo_unit, d);
+                    sh.xs[g][min(sub + LQ * j, S - 1)] = make_float4(d[0], d[1], d[2], 0.f);
+                }
+                if (base > 0) wave_lds_sync();
+            }
+        }
+        if constexpr (LQ > 1)
+            if (base == 0) __syncthreads();   // the shape derivatives are every wave's
+        if (!busy) continue;
+        Acc9 acc;
+        acc_zero(acc);
+        if constexpr (LQ == 1) {
+            // dN of a linear tetrahedron is (-1,-1,-1) and the unit vectors
+            float Ju[9];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) Ju[3 * c + k] = xs[c + 1][k] - xs[0][k];
+            nh_contrib(Ju, JXi, V, dnr, mt, acc);
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < PPL; ++i) {
+                const int q = min(sub + LQ * i, Q - 1);
+                if (i > 0) {
+                    if (f.affine) V = detB * gload(f.wq, q);
+                    else load_element_record(f, eid, q, JXi, V);
+                }
+                const float Vq = sub + LQ * i < Q ? V : 0.f;
+                float Ju[9];
+#pragma unroll
+                for (int k = 0; k < 9; ++k) Ju[k] = 0.f;
+                const float* dn = &sh.dn[q * 3];
+#pragma unroll
+                for (int k = 0; k < S; ++k) {
+                    const float4 x = sh.xs[g][k];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const float d = dn[k * Q * 3 + c];
+                        Ju[3 * c] = fmaf(x.x, d, Ju[3 * c]);
+                        Ju[3 * c + 1] = fmaf(x.y, d, Ju[3 * c + 1]);
+                        Ju[3 * c + 2] = fmaf(x.z, d, Ju[3 * c + 2]);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) dnr[c] = dn[r * Q * 3 + c];
+                nh_contrib(Ju, JXi, Vq, dnr, mt, acc);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 9; ++i) acc.v[i] = lanes_sum<LQ>(acc.v[i]);
+        if (has && sub == 0) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) sh.part[base + g][i] = acc.v[i];
+        }
+    }
+    __syncthreads();
+    if (t0 < n_slots) {
+        slot_state_settle(st);
+        if (st.free != 0) solve_slot_from_lds(ps, st, sh.part, first_own, damping, dt);
+    }
+}
+
+template <int S, int Q>
+__global__ __launch_bounds__(kFusedThreads) void k_point_tasks(FusedTaskArgs a) {
+    __shared__ PointLDS<S, Q> sh;
+    const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
+    point_block<S, Q>(a.ps, a.fem, a.own, a.mt, a.y, a.damping, a.dt, blk, sh);
+}
+
+template <int S, int Q>
+__global__ __launch_bounds__(kFusedThreads) void k_batch_point_tasks(BatchFusedArgs b) {
+    __shared__ PointLDS<S, Q> sh;
+    const int bid = xcd_block(blockIdx.x, gridDim.x);
+    const BatchSeg seg = find_seg(b.segs, b.seg_first, b.seg_count, bid);
+    const SceneDev& sd = b.scenes[seg.scene];
+    if (b.iteration >= sd.iterations) return;
+    // the scene's views, read before the first store
+    const PSView ps = sd.ps;
+    const FemView fem = sd.fem;
+    const OwnersView own = sd.own;
+    const MaterialView mt = sd.mt;
+    const float4* y = sd.y;
+    const float damping = sd.damping;
+    const int4 blk = gload(S == 10 ? sd.fblocks_split : sd.fblocks, seg.first + (bid - seg.block_begin));
+    point_block<S, Q>(ps, fem, own, mt, y, damping, b.dt, blk, sh);
+}
+
+#if OE_GATHER_S == 10   // one thread per incidence: quadratic tetrahedra in larger launches
 // The Jx contraction reads the shape-derivative table from device memory, except
 // for quadratic tetrahedra, whose gradients follow from two scalars (P2Factors).
 template <int S, class Grad>
@@ -598,6 +794,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedA
     fused_block<S, Q, LAT>(ps, fem, own, mt, g, y, damping, b.dt, blk, part, dn_lds[threadIdx.x >> 6]);
 }
 
+#endif   // OE_GATHER_S == 10
 #endif
 
 namespace {
@@ -840,7 +1037,7 @@ void OE_FN(launch_ju_refresh_)(const PSView& ps, const FemView& f, float* ju, hi
 
 int OE_FN(refresh_elements_per_block_)() { return refresh_epb<OE_GATHER_Q>(); }
 
-#if OE_GATHER_S != 27
+#if OE_GATHER_S == 10
 namespace {
 // The P2 factors from the element's quadrature points, checked against its
 // shape-derivative table (to float rounding: the reference's points are floats
@@ -848,7 +1045,6 @@ namespace {
 const ShapeArg<OE_GATHER_S>& shape_arg() {
     static const ShapeArg<OE_GATHER_S> g = [] {
         ShapeArg<OE_GATHER_S> t{};
-#if OE_GATHER_S == 10
         const ShapeTable& st = shape_table(Tetra10);
         const double b = st.qpoints[0], a = (1.0 - b) / 3.0;
         for (int q = 0; q < 4; ++q)
@@ -867,33 +1063,48 @@ const ShapeArg<OE_GATHER_S>& shape_arg() {
             }
         t.a4 = static_cast<float>(4.0 * a);
         t.k4 = static_cast<float>(4.0 * (b - a));
-#endif
         return t;
     }();
     return g;
 }
 }  // namespace
 
+#endif
+
+#if OE_GATHER_S != 27
 void OE_FN(launch_fused_tasks_)(const FusedTaskArgs& a, hipStream_t s) {
+    constexpr int S = OE_GATHER_S, Q = OE_GATHER_Q;
     if (a.count <= 0) return;
-    if (a.latency)
-        hipLaunchKernelGGL((k_fused_tasks<OE_GATHER_S, OE_GATHER_Q, true>), dim3(a.count), dim3(kFusedThreads), 0, s, a,
-                           shape_arg());
-    else
-        hipLaunchKernelGGL((k_fused_tasks<OE_GATHER_S, OE_GATHER_Q, false>), dim3(a.count), dim3(kFusedThreads), 0, s,
-                           a, shape_arg());
+#if OE_GATHER_S == 10
+    if (a.form == TASKS_THROUGHPUT) {
+        hipLaunchKernelGGL((k_fused_tasks<S, Q, false>), dim3(a.count), dim3(kFusedThreads), 0, s, a, shape_arg());
+        return;
+    }
+    if (a.form == TASKS_LATENCY) {
+        hipLaunchKernelGGL((k_fused_tasks<S, Q, true>), dim3(a.count), dim3(kFusedThreads), 0, s, a, shape_arg());
+        return;
+    }
+#endif
+    hipLaunchKernelGGL((k_point_tasks<S, Q>), dim3(a.count), dim3(kFusedThreads), 0, s, a);
 }
 
 void OE_FN(launch_batch_fused_tasks_)(const BatchFusedArgs& b, int nblocks, hipStream_t s) {
+    constexpr int S = OE_GATHER_S, Q = OE_GATHER_Q;
     if (nblocks <= 0) return;
-    if (b.latency)
-        hipLaunchKernelGGL((k_batch_fused_tasks<OE_GATHER_S, OE_GATHER_Q, true>), dim3(nblocks), dim3(kFusedThreads), 0,
-                           s, b, shape_arg());
-    else
-        hipLaunchKernelGGL((k_batch_fused_tasks<OE_GATHER_S, OE_GATHER_Q, false>), dim3(nblocks), dim3(kFusedThreads),
-                           0, s, b, shape_arg());
+#if OE_GATHER_S == 10
+    if (b.form == TASKS_THROUGHPUT) {
+        hipLaunchKernelGGL((k_batch_fused_tasks<S, Q, false>), dim3(nblocks), dim3(kFusedThreads), 0, s, b,
+                           shape_arg());
+        return;
+    }
+    if (b.form == TASKS_LATENCY) {
+        hipLaunchKernelGGL((k_batch_fused_tasks<S, Q, true>), dim3(nblocks), dim3(kFusedThreads), 0, s, b,
+                           shape_arg());
+        return;
+    }
+#endif
+    hipLaunchKernelGGL((k_batch_point_tasks<S, Q>), dim3(nblocks), dim3(kFusedThreads), 0, s, b);
 }
-
 #endif
 
 void OE_FN(launch_explicit_elem_)(const ExplicitElemArgs& a, hipStream_t s) {

@@ -50,6 +50,7 @@ struct SceneDev {
     float* ju;        // cached displacement gradients, or null
     const int4* fblocks;       // vertex blocks of the fused element tasks (throughput form), or null
     const int4* fblocks_lat;   // the same for the latency form
+    const int4* fblocks_split; // quadratic tetrahedra: the same for the point-task form
     float damping;
     int iterations;
     float g[3];
@@ -85,18 +86,17 @@ struct BatchGatherArgs {
 // element types other than the 27-node hexahedron.  A block takes a run of
 // consecutive slots of one colour (a "vertex block", int4 {first slot, slot
 // count, first owners index, incidence count}) whose incidences fit
-// kFusedIncPerBlock.  Its threads first take one incidence (element e, local
-// node r) each, kFusedThreads apart, and put the force / Hessian partial of
-// node r over all Q points of e in LDS; then one thread per slot adds its
-// vertex's partials in the owners order and runs the local solve.
-// Two forms share the kernels: the throughput form (each thread takes up to
-// kFusedRuns incidences in turn) and the latency form for launches too small
-// to fill the GPU (one incidence per thread, so a block's critical path holds
-// one element; the vertex state is loaded along the element chain).  Each
-// form has its own vertex blocks.  One run per thread measured fastest for the
-// throughput form too (P2 batch: 11.25 ms per step against 11.50 ms for two,
-// with no loads run ahead: those held 12 VGPRs and cost a wave per SIMD), so
-// the two forms differ only in when the vertex state is loaded.
+// kFusedIncPerBlock.  Its threads first take the incidences (element e, local
+// node r) and put the force / Hessian partial of node r over the points of e in
+// LDS; then one thread per slot adds its vertex's partials in the owners order
+// and runs the local solve.  Quadratic tetrahedra have three forms, each with
+// vertex blocks of its own:
+//   throughput  one thread per incidence;
+//   latency     the same, the vertex state loaded along the element chain, for
+//               launches too small to fill the GPU;
+//   split       point tasks, a lane per point, for launches smaller still.
+// The other types have point tasks only (oe_gather.hip, k_point_tasks).
+enum TaskForm : int { TASKS_THROUGHPUT = 0, TASKS_LATENCY = 1, TASKS_SPLIT = 2 };
 constexpr int kFusedThreads = 256;
 constexpr int kFusedRuns = 1;
 constexpr int kFusedIncPerBlock = kFusedThreads * kFusedRuns;
@@ -106,6 +106,12 @@ constexpr int kFusedMaxSlots = kFusedThreads;
 // fill the GPU: single scenes, and batches built for latency, use the latency
 // form there.
 constexpr int64_t kLatencyBlocks = 512;
+// Incidences that a point-task block of an element type takes at a time.
+constexpr int point_task_groups(int S) { return S == 4 ? kFusedThreads : S == 8 ? kFusedThreads / 8 : kFusedThreads / 4; }
+// Quadratic tetrahedra take point tasks up to this many incidences in a launch:
+// one wave per SIMD.  Past that a lane per point repeats the element's loads for
+// nothing (a pass of the 16x4x4 beam, 1,400 incidences, 6.0 -> 5.2 us).
+constexpr int64_t kSplitIncidences = 16384;
 
 struct FusedTaskArgs {
     PSView ps;
@@ -118,7 +124,7 @@ struct FusedTaskArgs {
     float dt;
     int first_block;      // the colour's vertex blocks: [first_block, first_block + count)
     int count;
-    int latency;          // 1: latency form (blocks are the latency-form vertex blocks)
+    int form;             // TaskForm; the blocks are that form's vertex blocks
 };
 // Batched: BatchSeg.first / count are a range of one scene's vertex blocks,
 // one block each.
@@ -129,7 +135,7 @@ struct BatchFusedArgs {
     int seg_count;
     int iteration;
     float dt;
-    int latency;   // 1: latency form and the scenes' latency vertex blocks
+    int form;   // TaskForm and that form's vertex blocks of the scenes
 };
 
 // Batched refresh of the cached displacement gradients: VSeg.count is the

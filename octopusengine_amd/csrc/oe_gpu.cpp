@@ -364,10 +364,12 @@ FemView GPU_FEM::fem_view() const {
 
 GatherTile default_tile(Element e) {
     switch (e) {
-        case Tetra: return {8, 1, PASS_GATHER};
-        case Hexa: return {16, 1, PASS_GATHER};
+        // lanes and points per lane: the gather of a Jacobi sweep, of the
+        // residual and of a mesh whose vertices do not fit the task blocks
+        case Tetra: return {8, 1, PASS_TASKS};
+        case Hexa: return {16, 1, PASS_TASKS};
         case Tetra10: return {64, 1, PASS_TASKS};
-        case Tetra20: return {64, 1, PASS_GATHER};
+        case Tetra20: return {64, 1, PASS_TASKS};
         case Hexa27: return {64, 1, PASS_TASKS, kQ2PencilIncLatency};
         default: return {16, 1, PASS_GATHER};
     }
@@ -408,7 +410,8 @@ GPU_VBD_FEM::GPU_VBD_FEM(Engine* e, Element el, const HostMesh& mesh, Material m
         } catch (const std::invalid_argument&) {
             // a vertex with more incidences than a task block holds: the
             // default pass falls back to the gather kernel
-            tile = element == Hexa27 ? GatherTile{64, 1, PASS_GATHER} : GatherTile{16, 2, PASS_GATHER};
+            if (element == Tetra10) tile = GatherTile{16, 2, PASS_GATHER};
+            else tile.mode = PASS_GATHER;
         }
     }
 }
@@ -433,7 +436,9 @@ void upload_vertex_blocks(Engine* eng, const OwnersCSR& o, int max_inc, int max_
 
 int GPU_VBD_FEM::fit_inc(int inc) const {
     const int n = inc > 0 ? inc : (element == Hexa27 ? kQ2FusedIncPerBlock : max_task_inc(element));
-    return element == Hexa27 ? q2_pencil_fit(n, max_incidences) : n;
+    if (element == Hexa27) return q2_pencil_fit(n, max_incidences);
+    if (element == Tetra10) return n;
+    return std::min(n, std::max(point_task_groups(S), max_incidences));
 }
 
 const TaskTables& GPU_VBD_FEM::throughput_tables(int inc) {
@@ -455,7 +460,7 @@ const TaskTables& GPU_VBD_FEM::built_tables(int inc) const {
 }
 
 const TaskTables* GPU_VBD_FEM::latency_tables() {
-    if (!lat_built) {
+    if (!lat_built && (element == Hexa27 || element == Tetra10)) {
         lat_built = true;
         const bool q2 = element == Hexa27;
         try {
@@ -469,9 +474,18 @@ const TaskTables* GPU_VBD_FEM::latency_tables() {
     return lat_tables.blocks.get() ? &lat_tables : nullptr;
 }
 
+const TaskTables* GPU_VBD_FEM::split_form() {
+    if (element != Tetra10) return nullptr;
+    if (!split_tables.blocks.get())
+        upload_vertex_blocks(eng, owners, std::max(point_task_groups(S), max_incidences), kFusedMaxSlots,
+                             split_tables.blocks, split_tables.color_begin);
+    return &split_tables;
+}
+
 void GPU_VBD_FEM::prepare_tasks() {
     throughput_tables(tile.inc);
     latency_tables();
+    split_form();
 }
 
 float* GPU_VBD_FEM::ensure_ju() {
@@ -585,7 +599,8 @@ void GPU_VBD_FEM::step(GPU_ParticleSystem* ps, float dt) {
             // the latency form for colours with few throughput-form blocks
             // (by default under 2 per CU)
             const bool lat = lt && thr->color_blocks(c) < tile.lat_blocks;
-            const TaskTables& tt = lat ? *lt : *thr;
+            const bool split = lat && element == Tetra10 && owners.color_incidences[c] <= kSplitIncidences;
+            const TaskTables& tt = split ? split_tables : lat ? *lt : *thr;
             const int4* blocks = tt.blocks.get();
             const int b0 = tt.color_begin[c], nb = tt.color_blocks(c);
             if (element == Hexa27) {
@@ -596,7 +611,7 @@ void GPU_VBD_FEM::step(GPU_ParticleSystem* ps, float dt) {
                     launch_q2_fused(qa, s);
             }
             else if (!launch_fused_tasks(S, Q, FusedTaskArgs{a.ps, a.fem, a.own, a.mt, y, blocks, damping, dt, b0, nb,
-                                                             lat ? 1 : 0},
+                                                             split ? TASKS_SPLIT : lat ? TASKS_LATENCY : TASKS_THROUGHPUT},
                                          s))
                 throw std::invalid_argument("unsupported element");
         } else if (!launch_gather(S, Q, tile.L, tile.QL, a, s)) {

@@ -247,18 +247,21 @@ struct GPU_VBD_FEM final : GPU_FEM {
     // half-wave); empty when a vertex has more incidences than one holds.
     TaskTables lat_tables;
     bool lat_built = false;
+    TaskTables split_tables;   // quadratic tetrahedra: vertex blocks of the point-task form
     // Build (if needed) and return the throughput tables for `inc`
     // incidences per block (0 = the kernel's maximum); throws
     // std::invalid_argument when a vertex has more incidences than a block.
     const TaskTables& throughput_tables(int inc);
     // the incidences per throughput-form block a tile of inc gets on this mesh
-    // (q2_pencil_fit for 27-node hexahedra; 0 = the kernel's maximum)
+    // (q2_pencil_fit for 27-node hexahedra; what a point-task block takes at a
+    // time for the types that have no other form; 0 = the kernel's maximum)
     int fit_inc(int inc) const;
     int max_incidences = 0;   // most incident elements of one vertex
     // The tables already built for `inc` (std::logic_error if not): for
     // step(), which may run under HIP graph capture and must not allocate.
     const TaskTables& built_tables(int inc) const;
     const TaskTables* latency_tables();   // null when absent
+    const TaskTables* split_form();       // null for other types than quadratic tetrahedra
     void prepare_tasks();                 // the tables of the current tile
     bool tasks() const {
         return tile.mode == PASS_TASKS && version != Better_Coloration && (element != Hexa27 || has_q2_basis);

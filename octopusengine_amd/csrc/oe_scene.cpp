@@ -133,7 +133,8 @@ size_t Scene::device_bytes() const {
     size_t b = ps->device_bytes() + fem->topo.bytes() + fem->jxv.bytes() + fem->dN.bytes() + fem->wq.bytes();
     if (vbd_fem) {
         b += vbd_fem->d_slot_vid.bytes() + vbd_fem->d_slot_nbo.bytes() + vbd_fem->d_own.bytes() +
-             vbd_fem->p_new.bytes() + vbd_fem->ju.bytes() + vbd_fem->lat_tables.blocks.bytes();
+             vbd_fem->p_new.bytes() + vbd_fem->ju.bytes() + vbd_fem->lat_tables.blocks.bytes() +
+             vbd_fem->split_tables.blocks.bytes();
         for (const auto& kv : vbd_fem->thr_tables) b += kv.second.blocks.bytes();
     }
     return b;

@@ -222,7 +222,7 @@ TuneRecord autotune_scene(Scene& sc, bool force) {
             continue;
         }
         try {
-            std::pair<int, std::vector<bool>> sig{t.inc, latency_pattern(*sc.vbd_fem, t)};
+            std::pair<int, std::vector<bool>> sig{sc.vbd_fem->fit_inc(t.inc), latency_pattern(*sc.vbd_fem, t)};
             if (std::find(seen.begin(), seen.end(), sig) != seen.end()) continue;
             seen.push_back(std::move(sig));
             unique.push_back(t);
