@@ -172,41 +172,66 @@ __global__ __launch_bounds__(kBlock) void k_copy_colour(PSView ps, const int* sl
 }
 
 // Internal force of each vertex from the element partials of k_explicit_elem
-// (9 floats per (element, local node), in owners order, so a vertex's partials
-// are contiguous): they are added in owners order, then the damping term of
-// the reference's force pass, f = sum(-V P g) - k H v
-// (src/GPU/Explicit/GPU_FEM_Explicit.cu:45-62), overwrites ps.f.  Four
-// incidences are loaded at a time so that their loads overlap.  With
-// integrate set (a semi-implicit integrator whose only dynamic is this force
-// pass) the thread then runs k_semi_implicit's update of its vertex, the same
-// operations on the same values, and the constraints; the separate passes are
-// skipped (2.9 us each of the 17.5 us of a 27-node 32x8x8 substep).
-constexpr int kExplicitVertexBlock = 64;
-__global__ __launch_bounds__(kExplicitVertexBlock) void k_explicit_vertex(PSView ps, OwnersView own,
-                                                                          const float* partial, int count,
-                                                                          float damping, int integrate, float dt,
-                                                                          float gx, float gy, float gz,
-                                                                          VertexConstraints c) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= count) return;
-    const int vid = gload(own.slot_vid, slot);
-    const int2 nbo = gload(own.slot_nbo, slot);
-    const float* __restrict__ src = partial + static_cast<size_t>(nbo.y) * 9;
-    float a[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int j = 0;
-    for (; j + 4 <= nbo.x; j += 4) {
-        float t[36];
-#pragma unroll
-        for (int k = 0; k < 36; ++k) t[k] = gload(src, j * 9 + k);
-#pragma unroll
-        for (int k = 0; k < 36; ++k) a[k % 9] += t[k];
+// (3 floats per (element, local node), with damping 9, in owners order, so a
+// vertex's partials are contiguous): they are added in owners order, then the
+// damping term of the reference's force pass, f = sum(-V P g) - k H v
+// (src/GPU/Explicit/GPU_FEM_Explicit.cu:45-62), overwrites ps.f.  Eight
+// incidences are loaded at a time, and the vertex's own records before them, so
+// that the chain is {range, records} -> partials.  With damping three lanes take
+// a vertex's nine sums, three neighbouring floats each, and one of them finishes:
+// 36 floats a round in one lane took 7.7 us, nine lanes of one float 6.5, this
+// 5.5 us on the damped 20-node 32x8x8 beam.  With integrate set (a semi-implicit
+// integrator whose only dynamic is this force pass) the thread then runs
+// k_semi_implicit's update of its vertex and the constraints; those passes are
+// skipped (2.9 us each).  Undamped 27-node 32x8x8 beam: 3.3 us, 3.8 us when the
+// undamped partials had nine floats too.
+constexpr int kExplicitVertices = 64;   // per block
+template <bool DAMP>
+__global__ __launch_bounds__(kExplicitVertices * (DAMP ? 3 : 1)) void k_explicit_vertex(
+    PSView ps, const int2* nbo, const float* partial, int count, float damping, int integrate, float dt, float gx,
+    float gy, float gz, VertexConstraints c) {
+    constexpr int NP = explicit_partial(DAMP), LANES = NP / 3, NV = kExplicitVertices, N = 8;
+    const int t = threadIdx.x;
+    const int2 range = gload(nbo, min(static_cast<int>(blockIdx.x) * NV + t / LANES, count - 1));
+    const int vid = blockIdx.x * NV + t;
+    const bool mine = t < NV && vid < count;
+    float4 p = f4(0.f, 0.f, 0.f, 0.f), v = p, X = p;
+    float w = 0.f;
+    bool is_fixed = false;
+    int mask = 0;
+    if (mine) {
+        p = gload(static_cast<const float4*>(ps.p), vid);
+        v = gload(static_cast<const float4*>(ps.v), vid);
+        w = gload(ps.w, vid);
+        is_fixed = c.fixed && gload(c.fixed, vid) != 0;
+        if (c.has_box) mask = gload(static_cast<const int*>(ps.mask), vid);
+        if (c.fixed || c.has_box) X = gload(static_cast<const float4*>(ps.init_p), vid);
     }
-    for (; j < nbo.x; ++j)
+    const float* __restrict__ src = partial + static_cast<size_t>(range.y) * NP + t % LANES * 3;
+    float part[3] = {0.f, 0.f, 0.f};
+    for (int j = 0; j < range.x; j += N) {
+        float x[3 * N];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) a[i] += gload(src, j * 9 + i);
-    float4 f = make_float4(a[0], a[1], a[2], 0.f);
-    if (damping != 0.f) {
-        const float4 v = ps.v[vid];
+        for (int k = 0; k < 3 * N; ++k) x[k] = gload(src, NP * min(j + k / 3, range.x - 1) + k % 3);
+#pragma unroll
+        for (int k = 0; k < 3 * N; ++k) part[k % 3] += j + k / 3 < range.x ? x[k] : 0.f;
+    }
+    float a[NP];
+    if constexpr (DAMP) {
+        __shared__ float sums[NV * NP];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sums[3 * t + i] = part[i];
+        __syncthreads();
+        if (!mine) return;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) a[i] = sums[NP * t + i];
+    } else {
+        if (!mine) return;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) a[i] = part[i];
+    }
+    float4 f = f4(a[0], a[1], a[2], 0.f);
+    if constexpr (DAMP) {
         f.x -= damping * (a[3] * v.x + a[4] * v.y + a[5] * v.z);
         f.y -= damping * (a[4] * v.x + a[6] * v.y + a[7] * v.z);
         f.z -= damping * (a[5] * v.x + a[7] * v.y + a[8] * v.z);
@@ -215,18 +240,14 @@ __global__ __launch_bounds__(kExplicitVertexBlock) void k_explicit_vertex(PSView
         ps.f[vid] = f;
         return;
     }
-    float4 p = ps.p[vid];
-    float4 v = ps.v[vid];
-    const float w = ps.w[vid];
-    ps.last_p[vid] = p;
+    gstore(ps.last_p, vid, p);
     semi_implicit(p, v, f, w, dt, gx, gy, gz);
-    const bool is_fixed = c.fixed && gload(c.fixed, vid) != 0;   // constrain() stores v and f of a fixed vertex
-    if (!is_fixed) {
-        ps.v[vid] = v;
-        ps.f[vid] = f4(0.f, 0.f, 0.f, 0.f);
+    if (!is_fixed) {   // constrain() stores v and f of a fixed vertex
+        gstore(ps.v, vid, v);
+        gstore(ps.f, vid, f4(0.f, 0.f, 0.f, 0.f));
     }
-    constrain(ps, vid, p, c);
-    ps.p[vid] = p;
+    constrain(ps, vid, p, is_fixed, mask, X, c.t.com, c.t.offset, c.t.R, c.has_box, c.lo, c.hi);
+    gstore(ps.p, vid, p);
 }
 
 // Packed xyz of a run of records for the host.  The output is pinned host
@@ -360,13 +381,18 @@ void launch_box(const PSView& ps, const float pmin[3], const float pmax[3], hipS
                        make_float3(pmax[0], pmax[1], pmax[2]));
 }
 
-void launch_explicit_vertex(const PSView& ps, const OwnersView& own, const float* partial, int count, float damping,
+void launch_explicit_vertex(const PSView& ps, const int2* nbo, const float* partial, int count, float damping,
                             const float* gravity, const VertexConstraints& c, float dt, hipStream_t s) {
     if (count <= 0) return;
     const float g0 = gravity ? gravity[0] : 0.f, g1 = gravity ? gravity[1] : 0.f, g2 = gravity ? gravity[2] : 0.f;
-    hipLaunchKernelGGL(k_explicit_vertex, dim3((count + kExplicitVertexBlock - 1) / kExplicitVertexBlock),
-                       dim3(kExplicitVertexBlock), 0, s, ps, own, partial, count, damping, gravity ? 1 : 0, dt, g0,
-                       g1, g2, c);
+    const dim3 grid((count + kExplicitVertices - 1) / kExplicitVertices);
+    const dim3 block(kExplicitVertices * (damping != 0.f ? 3 : 1));
+    if (damping != 0.f)
+        hipLaunchKernelGGL((k_explicit_vertex<true>), grid, block, 0, s, ps, nbo, partial, count, damping,
+                           gravity ? 1 : 0, dt, g0, g1, g2, c);
+    else
+        hipLaunchKernelGGL((k_explicit_vertex<false>), grid, block, 0, s, ps, nbo, partial, count, damping,
+                           gravity ? 1 : 0, dt, g0, g1, g2, c);
 }
 
 void launch_copy_colour(const PSView& ps, const int* slot_vid, int first, int count, const float4* p_new,

@@ -50,10 +50,12 @@ void launch_pbd_tail(const PSView& ps, const VertexConstraints& c, float dt, flo
 void launch_fix(const PSView& ps, const int* ids, int n, const FixTransform& t, hipStream_t s);
 void launch_box(const PSView& ps, const float pmin[3], const float pmax[3], hipStream_t s);
 // Explicit integrator: each vertex's internal force from the element partials
-// (9 floats per (element, local node), owners order) and the damping term.
-// With gravity set, the semi-implicit update (launch_semi_implicit) of the
-// vertex and the constraints follow in the same thread.
-void launch_explicit_vertex(const PSView& ps, const OwnersView& own, const float* partial, int count, float damping,
+// (explicit_partial(damping != 0) floats per (element, local node), owners
+// order; nbo: incidence count and first partial of every vertex) and the
+// damping term.  With gravity set, the semi-implicit update
+// (launch_semi_implicit) of the vertex and the constraints follow in the same
+// thread.
+void launch_explicit_vertex(const PSView& ps, const int2* nbo, const float* partial, int count, float damping,
                             const float* gravity, const VertexConstraints& c, float dt, hipStream_t s);
 void launch_copy_colour(const PSView& ps, const int* slot_vid, int first, int count, const float4* p_new,
                         hipStream_t s);

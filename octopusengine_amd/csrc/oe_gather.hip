@@ -841,151 +841,164 @@ bool launch_L(int L, const GatherArgs& a, hipStream_t s) {
 // Element-centric internal forces of the explicit integrator.  The reference
 // computes them per vertex (kernel_fem_eval_force,
 // src/GPU/Explicit/GPU_FEM_Explicit.cu:5-64), so a vertex rebuilds F at every
-// point of each incident element: S times over per (element, point).  Here LPE
-// lanes (32, or a whole wave for 27-point elements) take one element:
-//   nodes:  lane k < S puts node k's displacement relative to node 0 in LDS;
-//   points: lane q < Q forms Ju = sum_k x_k (x) dN_k(q), F, cof F and
+// point of each incident element: S times over per (element, point).  Here a
+// block takes NE elements in three stages, each dealt evenly over its threads
+// (as many elements as make the points, or the nodes, fill whole waves):
+//   nodes:  thread (e, k) puts node k's displacement relative to node 0 in LDS;
+//   points: thread (e, q) forms Ju = sum_k x_k (x) dN_k(q), F, cof F and
 //           s = lambda (J - alpha) once, and from them (M = JX_inv^T, so that
-//           g = M dN_r):
+//           g = M dN_r)
 //             Pm = V (mu F + s C) M    force  -V (mu F g + s C g) = -Pm dN_r
+//           and with damping
 //             G  = V mu M^T M          V mu |g|^2 = dN_r^T G dN_r
 //             K  = C M                 C g = K dN_r
-//           and V lambda, in LDS point-major per component (lanes write
-//           consecutive words);
-//   nodes:  lane r < S of each 32-lane half adds the force and Hessian block
-//           V mu |g|^2 I + V lambda (C g)(C g)^T of node r over its half of
-//           the points (every lane reads the same point words, a broadcast);
-//           the halves are added and lane r stores the 9 floats at the
-//           owners position of (e, r), so that each vertex's partials are
-//           contiguous.
-// k_explicit_vertex then adds each vertex's partials in owners order.
+//           and V lambda, in LDS;
+//   nodes:  thread (e, r) adds node r's terms over the points: the force, and
+//           with damping the Hessian block V mu |g|^2 I + V lambda (C g)(C g)^T
+//           of the reference's -k H v.  They go to the owners position of
+//           (e, r), so that each vertex's partials are contiguous.
+// k_explicit_vertex then adds each vertex's partials in owners order.  Explicit
+// substeps carry every rounding of the force on (high modes are undamped), so
+// each sum keeps its order.  With one element per 32 or 64 lanes (11 of 32 in
+// the point stage of a 20-node element), scalar LDS reads and the Hessian also
+// where nothing reads it, the pass took 11.1 us on the 27-node 32x8x8 beam and
+// 18.5 us on the damped 20-node one; now 7.1 us and 13.3 us.
+// Damped it is bound by the 47 VALU instructions per (node, point),
+// 6.8 us on that beam, undamped by the three stages' latencies.
 constexpr int kExplicitThreads = 256;
-constexpr int kExplicitPt = 25;      // Pm 9, K 9, G 6, V lambda
-
-template <int Q>
-constexpr int explicit_lanes() {
-    return Q >= 16 ? 64 : 32;
-}
-
 template <int S, int Q>
+constexpr int explicit_elements() { return S == 4 ? 64 : S == 8 ? 32 : S == 10 ? 25 : S == 20 ? 11 : 9; }
+
+template <int S, int Q, bool DAMP>
 __global__ __launch_bounds__(kExplicitThreads) void k_explicit_elem(ExplicitElemArgs a) {
-    static_assert(S <= 32 && Q <= 32, "one element per 32 or 64 lanes");
-    constexpr int LPE = explicit_lanes<Q>();
-    constexpr int EPB = kExplicitThreads / LPE;
-    constexpr int QH = (Q + LPE / 32 - 1) / (LPE / 32);   // points per 32-lane half
-    __shared__ float dn_s[Q * S * 3];
-    __shared__ float xs_s[EPB][S * 3];
-    __shared__ float pt_s[EPB][kExplicitPt][Q];
-    const int tid = threadIdx.x;
-    const int h = tid / LPE, lane = tid % LPE;
-    const int r = (lane & 31) < S ? (lane & 31) : S - 1;
-    const int half = lane >> 5;
-    const int E = a.fem.E;
-    const int e = blockIdx.x * EPB + h;
-    const int ec = e < E ? e : E - 1;
-    const int at = gload(a.inc_at, static_cast<size_t>(ec) * S + r);
-    for (int i = tid; i < Q * S * 3; i += kExplicitThreads) dn_s[i] = gload(a.fem.dN, i);
-    {
-        const int k = lane < S ? lane : S - 1;
-        const int node = gload(a.fem.topo, static_cast<size_t>(ec) * S + k);
-        const float4 u = gload(static_cast<const float4*>(a.ps.p), node);
-        float4 ref;
-        ref.x = __shfl(u.x, 0, LPE);
-        ref.y = __shfl(u.y, 0, LPE);
-        ref.z = __shfl(u.z, 0, LPE);
-        ref.w = __shfl(u.w, 0, LPE);
-        float x[3];
-        rel_node(u, ref, a.ps.lo_unit, x);
-        if (lane < S) {
-            xs_s[h][3 * lane] = x[0];
-            xs_s[h][3 * lane + 1] = x[1];
-            xs_s[h][3 * lane + 2] = x[2];
-        }
-    }
-    const int q = lane < Q ? lane : Q - 1;
+    constexpr int T = kExplicitThreads, NE = explicit_elements<S, Q>();
+    static_assert(NE * S <= T && NE * Q <= T, "one round per stage");
+    constexpr int R = (Q * 3) | 1;              // row of dn: node k's 3 Q values; odd, so nodes spread over the banks
+    constexpr int W = DAMP ? 7 : 3;             // float4 per point: Pm (9), then K (9), G (6), V lambda
+    __shared__ float dn[S * R];
+    __shared__ float4 xs[NE][S | 1];
+    __shared__ float4 pt[NE * Q][W];
+    const int t = threadIdx.x;
+    const int E = a.fem.E, e0 = blockIdx.x * NE;
+    // the thread's node (threads past the last work on it and store nothing)
+    const int nt = min(t, NE * S - 1), ne = nt / S, r = nt % S;
+    const int ec = min(e0 + ne, E - 1);
+    const size_t inc = static_cast<size_t>(ec) * S + r;
+    const int node = gload(a.fem.topo, inc);
+    const int at = gload(a.inc_at, inc);
+    // the thread's point
+    const int qt = min(t, NE * Q - 1), qe = qt / Q, q = qt % Q;
     float JXi[9], V;
-    load_element_record(a.fem, ec, q, JXi, V);
+    load_element_record(a.fem, min(e0 + qe, E - 1), q, JXi, V);
+    constexpr int kStage = (S * Q * 3 + T - 1) / T;
+    float stage[kStage];
+#pragma unroll
+    for (int j = 0; j < kStage; ++j) stage[j] = gload(a.fem.dN, min(t + T * j, S * Q * 3 - 1));
+    const float4 u = gload(static_cast<const float4*>(a.ps.p), node);
+#pragma unroll
+    for (int j = 0; j < kStage; ++j) {
+        const int i = min(t + T * j, S * Q * 3 - 1);   // (q S + k) 3 + c
+        dn[i / 3 % S * R + i / (3 * S) * 3 + i % 3] = stage[j];
+    }
+    if (t < NE * S) xs[ne][r] = u;
     __syncthreads();
-    {
+    if (t < NE * Q) {
         float Ju[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) Ju[i] = 0.f;
-        const float* __restrict__ dn = dn_s + q * S * 3;
+        const float4 ref = xs[qe][0];
 #pragma unroll
         for (int k = 0; k < S; ++k) {
-            const float d0 = dn[3 * k], d1 = dn[3 * k + 1], d2 = dn[3 * k + 2];
+            const float4 h = xs[qe][k];
+            const float x[3] = {h.x - ref.x, h.y - ref.y, h.z - ref.z};   // an explicit state has no low-order parts
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const float xk = xs_s[h][3 * k + c];
-                Ju[0 + c] = fmaf(xk, d0, Ju[0 + c]);
-                Ju[3 + c] = fmaf(xk, d1, Ju[3 + c]);
-                Ju[6 + c] = fmaf(xk, d2, Ju[6 + c]);
+                const float d = dn[k * R + q * 3 + c];
+                Ju[3 * c] = fmaf(x[0], d, Ju[3 * c]);
+                Ju[3 * c + 1] = fmaf(x[1], d, Ju[3 * c + 1]);
+                Ju[3 * c + 2] = fmaf(x[2], d, Ju[3 * c + 2]);
             }
         }
-        float F[9], C[9];
+        float F[9], C[9], P[9];
         deformation_gradient(Ju, JXi, F);
         cofactor(F, C);
-        const float J = det_from_cof(F, C);
+        const float J = det_fixup(dot3_plain(F[0], C[0], F[1], C[1], F[2], C[2]), F);
         const float sl = a.mt.lambda * (J - a.mt.alpha);
-        if (lane < Q) {
-            // F, C, JX_inv column-major: X(row, col) = X[col * 3 + row]; M(c, l) = JX_inv[c * 3 + l]
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
+        for (int i = 0; i < 9; ++i) P[i] = fmaf(a.mt.mu, F[i], sl * C[i]);
+        // X(row, col) = X[col * 3 + row]; M(c, l) = JX_inv[c * 3 + l]
+        float w[4 * W];
 #pragma unroll
-                for (int l = 0; l < 3; ++l) {
-                    float pm = 0.f, km = 0.f;
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        pm += (a.mt.mu * F[c * 3 + i] + sl * C[c * 3 + i]) * JXi[c * 3 + l];
-                        km += C[c * 3 + i] * JXi[c * 3 + l];
-                    }
-                    pt_s[h][i * 3 + l][lane] = V * pm;
-                    pt_s[h][9 + i * 3 + l][lane] = km;
-                }
+            for (int l = 0; l < 3; ++l) {
+                w[i * 3 + l] = V * fmaf(P[6 + i], JXi[6 + l], fmaf(P[3 + i], JXi[3 + l], P[i] * JXi[l]));
+                if constexpr (DAMP)
+                    w[9 + i * 3 + l] = fmaf(C[6 + i], JXi[6 + l], fmaf(C[3 + i], JXi[3 + l], C[i] * JXi[l]));
+            }
+        if constexpr (DAMP) {
             const float vm = V * a.mt.mu;
             constexpr int gl[6] = {0, 0, 0, 1, 1, 2}, gm[6] = {0, 1, 2, 1, 2, 2};
 #pragma unroll
             for (int i = 0; i < 6; ++i)
-                pt_s[h][18 + i][lane] = vm * (JXi[gl[i]] * JXi[gm[i]] + JXi[3 + gl[i]] * JXi[3 + gm[i]] +
-                                              JXi[6 + gl[i]] * JXi[6 + gm[i]]);
-            pt_s[h][24][lane] = V * a.mt.lambda;
+                w[18 + i] = vm * dot3_plain(JXi[gl[i]], JXi[gm[i]], JXi[3 + gl[i]], JXi[3 + gm[i]], JXi[6 + gl[i]],
+                                            JXi[6 + gm[i]]);
+            w[24] = V * a.mt.lambda;
+            w[25] = w[26] = w[27] = 0.f;
+        } else {
+            w[9] = w[10] = w[11] = 0.f;
         }
+#pragma unroll
+        for (int i = 0; i < W; ++i) pt[qt][i] = make_float4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
     }
     __syncthreads();
-    float acc[9];
+    if (t >= NE * S || e0 + ne >= E) return;
+    // force, and with damping the Hessian block xx xy xz yy yz zz; a 27-node
+    // hexahedron's points in two partial sums
+    constexpr int NP = explicit_partial(DAMP);
+    constexpr int QH = Q >= 16 ? (Q + 1) / 2 : Q;
+    float acc[NP], lo[NP];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) acc[i] = 0.f;
-    const int p_end = (half + 1) * QH < Q ? (half + 1) * QH : Q;
-    for (int p = half * QH; p < p_end; ++p) {
-        const float* __restrict__ dn = dn_s + (p * S + r) * 3;
-        const float d0 = dn[0], d1 = dn[1], d2 = dn[2];
-        float w[kExplicitPt];
+    for (int i = 0; i < NP; ++i) acc[i] = lo[i] = 0.f;
+#pragma unroll 3
+    for (int p = 0; p < Q; ++p) {
+        if (QH < Q && p == QH) {
 #pragma unroll
-        for (int i = 0; i < kExplicitPt; ++i) w[i] = pt_s[h][i][p];
-        float c[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            acc[i] -= w[i * 3] * d0 + w[i * 3 + 1] * d1 + w[i * 3 + 2] * d2;
-            c[i] = w[9 + i * 3] * d0 + w[9 + i * 3 + 1] * d1 + w[9 + i * 3 + 2] * d2;
+            for (int i = 0; i < NP; ++i) {
+                lo[i] = acc[i];
+                acc[i] = 0.f;
+            }
         }
-        const float gd = w[18] * d0 * d0 + w[21] * d1 * d1 + w[23] * d2 * d2 +
-                         2.f * (w[19] * d0 * d1 + w[20] * d0 * d2 + w[22] * d1 * d2);
-        const float vl = w[24];
-        acc[3] += gd + vl * c[0] * c[0];
-        acc[4] += vl * c[1] * c[0];
-        acc[5] += vl * c[2] * c[0];
-        acc[6] += gd + vl * c[1] * c[1];
-        acc[7] += vl * c[2] * c[1];
-        acc[8] += gd + vl * c[2] * c[2];
-    }
-    if constexpr (LPE == 64) {
+        const float d0 = dn[r * R + p * 3], d1 = dn[r * R + p * 3 + 1], d2 = dn[r * R + p * 3 + 2];
+        float w[4 * W];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) acc[i] += __shfl_xor(acc[i], 32);
-    }
-    if (e >= E || lane >= S) return;
-    float* out = a.partial + static_cast<size_t>(at) * 9;
+        for (int i = 0; i < W; ++i) {
+            const float4 x = pt[ne * Q + p][i];
+            w[4 * i] = x.x;
+            w[4 * i + 1] = x.y;
+            w[4 * i + 2] = x.z;
+            w[4 * i + 3] = x.w;
+        }
 #pragma unroll
-    for (int i = 0; i < 9; ++i) out[i] = acc[i];
+        for (int i = 0; i < 3; ++i) acc[i] -= dot3_plain(w[3 * i], d0, w[3 * i + 1], d1, w[3 * i + 2], d2);
+        if constexpr (DAMP) {
+            float c[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) c[i] = w[9 + i * 3] * d0 + w[9 + i * 3 + 1] * d1 + w[9 + i * 3 + 2] * d2;
+            const float gd = w[18] * d0 * d0 + w[21] * d1 * d1 + w[23] * d2 * d2 +
+                             2.f * (w[19] * d0 * d1 + w[20] * d0 * d2 + w[22] * d1 * d2);
+            const float vl = w[24];
+            acc[3] += gd + vl * c[0] * c[0];
+            acc[4] += vl * c[1] * c[0];
+            acc[5] += vl * c[2] * c[0];
+            acc[6] += gd + vl * c[1] * c[1];
+            acc[7] += vl * c[2] * c[1];
+            acc[8] += gd + vl * c[2] * c[2];
+        }
+    }
+    float* out = a.partial + static_cast<size_t>(at) * NP;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) out[i] = QH < Q ? lo[i] + acc[i] : acc[i];
 }
 
 }  // namespace
@@ -1108,10 +1121,13 @@ void OE_FN(launch_batch_fused_tasks_)(const BatchFusedArgs& b, int nblocks, hipS
 #endif
 
 void OE_FN(launch_explicit_elem_)(const ExplicitElemArgs& a, hipStream_t s) {
+    constexpr int S = OE_GATHER_S, Q = OE_GATHER_Q, NE = explicit_elements<S, Q>();
     if (a.fem.E <= 0) return;
-    constexpr int EPB = kExplicitThreads / explicit_lanes<OE_GATHER_Q>();
-    hipLaunchKernelGGL((k_explicit_elem<OE_GATHER_S, OE_GATHER_Q>), dim3((a.fem.E + EPB - 1) / EPB),
-                       dim3(kExplicitThreads), 0, s, a);
+    const dim3 grid((a.fem.E + NE - 1) / NE), block(kExplicitThreads);
+    if (a.damped)
+        hipLaunchKernelGGL((k_explicit_elem<S, Q, true>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((k_explicit_elem<S, Q, false>), grid, block, 0, s, a);
 }
 
 void OE_FN(launch_batch_ju_refresh_)(const BatchRefreshArgs& b, int nblocks, hipStream_t s) {

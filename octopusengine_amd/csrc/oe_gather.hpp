@@ -150,15 +150,17 @@ struct BatchRefreshArgs {
 };
 
 // Element-centric internal forces of the explicit integrator: per element and
-// local node r, the 9 floats (force, then the Hessian block xx xy xz yy yz zz)
-// of node r over the element's Q points at partial[inc_at[e S + r] 9], where
-// inc_at is the owners position of (e, r).
+// local node r, the force of the element's Q points on node r and with damping
+// the Hessian block xx xy xz yy yz zz, at partial[inc_at[e S + r] NP], NP =
+// explicit_partial(damped), where inc_at is the owners position of (e, r).
+constexpr int explicit_partial(bool damped) { return damped ? 9 : 3; }
 struct ExplicitElemArgs {
     PSView ps;
     FemView fem;
     MaterialView mt;
     const int* inc_at;   // E * S
-    float* partial;      // E * S * 9, owners order
+    float* partial;      // E * S * NP, owners order
+    bool damped;
 };
 
 #define OE_GATHER_DECL(S, Q)                                                                                  \

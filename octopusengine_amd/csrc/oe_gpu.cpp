@@ -722,7 +722,7 @@ GPU_FEM_Explicit::GPU_FEM_Explicit(Engine* e, Element el, const HostMesh& mesh, 
     for (size_t j = 0; j < o.own.size(); ++j)
         inc_at[static_cast<size_t>(o.own[j] >> 5) * S + (o.own[j] & 31)] = static_cast<int>(j);
     d_inc_at = DBuf<int>(&eng->pool, inc_at);
-    d_partial = DBuf<float>(&eng->pool, o.own.size() * 9);
+    d_partial = DBuf<float>(&eng->pool, o.own.size() * explicit_partial(_damping != 0.f));
 }
 
 void GPU_FEM_Explicit::step(GPU_ParticleSystem* ps, float dt) {
@@ -738,10 +738,10 @@ void GPU_FEM_Explicit::step(GPU_ParticleSystem* ps, float dt) {
     a.count = n_vertices;
     a.mode = GATHER_EXPLICIT_FORCE;
     if (tile.mode == PASS_TASKS) {
-        ExplicitElemArgs ea{a.ps, a.fem, a.mt, d_inc_at.get(), d_partial.get()};
+        ExplicitElemArgs ea{a.ps, a.fem, a.mt, d_inc_at.get(), d_partial.get(), _damping != 0.f};
         if (!launch_explicit_elem(S, Q, ea, eng->stream)) throw std::invalid_argument("unsupported element");
-        launch_explicit_vertex(a.ps, a.own, d_partial.get(), n_vertices, _damping, nullptr, VertexConstraints{}, dt,
-                               eng->stream);
+        launch_explicit_vertex(a.ps, d_slot_nbo.get(), d_partial.get(), n_vertices, _damping, nullptr,
+                               VertexConstraints{}, dt, eng->stream);
         return;
     }
     if (!launch_gather(S, Q, tile.L, tile.QL, a, eng->stream)) throw std::invalid_argument("unsupported gather tile");
@@ -751,10 +751,9 @@ bool GPU_FEM_Explicit::step_integrate(GPU_ParticleSystem* ps, float dt, const fl
                                       const VertexConstraints& c) {
     if (tile.mode != PASS_TASKS || ps->n != n_vertices) return false;
     const PSView v = ps->get_parameters();
-    ExplicitElemArgs ea{v, fem_view(), mt, d_inc_at.get(), d_partial.get()};
+    ExplicitElemArgs ea{v, fem_view(), mt, d_inc_at.get(), d_partial.get(), _damping != 0.f};
     if (!launch_explicit_elem(S, Q, ea, eng->stream)) throw std::invalid_argument("unsupported element");
-    launch_explicit_vertex(v, OwnersView{d_slot_vid.get(), d_slot_nbo.get(), d_own.get()}, d_partial.get(), n_vertices,
-                           _damping, gravity, c, dt, eng->stream);
+    launch_explicit_vertex(v, d_slot_nbo.get(), d_partial.get(), n_vertices, _damping, gravity, c, dt, eng->stream);
     return true;
 }
 

@@ -308,9 +308,9 @@ struct GPU_FEM_Explicit final : GPU_FEM {
     // The element-centric pass followed by the semi-implicit update and the
     // constraints in its vertex pass; false (nothing launched) in the gather mode.
     bool step_integrate(GPU_ParticleSystem* ps, float dt, const float gravity[3], const VertexConstraints& c);
-    float _damping;
-    // mode PASS_TASKS (the default): element-centric force pass (one element
-    // per 32 lanes, then a per-vertex sum of the element partials);
+    const float _damping;   // sizes d_partial
+    // mode PASS_TASKS (the default): element-centric force pass, then a
+    // per-vertex sum of the element partials;
     // PASS_GATHER: the per-vertex gather with tile L x QL
     GatherTile tile;
     int n_vertices;
@@ -318,7 +318,7 @@ struct GPU_FEM_Explicit final : GPU_FEM {
     DBuf<int2> d_slot_nbo;
     DBuf<int> d_own;
     DBuf<int> d_inc_at;      // E * S: owners position of (element, local node)
-    DBuf<float> d_partial;   // E * S * 9: per (element, local node) force and Hessian block, owners order
+    DBuf<float> d_partial;   // per (element, local node) force, with damping also the Hessian block; owners order
 };
 
 struct GPU_Fix_Constraint final : GPU_Dynamic {

@@ -155,6 +155,11 @@ __device__ __forceinline__ float dot3(float a0, float b0, float a1, float b1, fl
     return fmaf(a0, b0, fmaf(a1, b1, a2 * b2));
 }
 __device__ __forceinline__ float diff2(float a, float b, float c, float d) { return fmaf(a, b, -(c * d)); }
+// The order the compiler gives a plain a0 b0 + a1 b1 + a2 b2.  Hundreds of
+// explicit substeps carry every rounding of the force on, so that pass keeps it.
+__device__ __forceinline__ float dot3_plain(float a0, float b0, float a1, float b1, float a2, float b2) {
+    return fmaf(a2, b2, fmaf(a0, b0, a1 * b1));
+}
 
 // F = Jx * JX_inv (both column-major)
 __device__ __forceinline__ void mat_mul(const float A[9], const float B[9], float C[9]) {
@@ -162,7 +167,7 @@ __device__ __forceinline__ void mat_mul(const float A[9], const float B[9], floa
     for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int r = 0; r < 3; ++r)
-            C[c * 3 + r] = dot3(A[r], B[c * 3], A[3 + r], B[c * 3 + 1], A[6 + r], B[c * 3 + 2]);
+            C[c * 3 + r] = dot3_plain(A[r], B[c * 3], A[3 + r], B[c * 3 + 1], A[6 + r], B[c * 3 + 2]);
 }
 
 // Deformation gradient from nodal displacements u = x - X:
@@ -194,14 +199,16 @@ __device__ __forceinline__ void cofactor(const float F[9], float C[9]) {
 
 // det F = column0 . cof column0.  Elements close to inversion (J < 0.1) get
 // the determinant re-evaluated in double precision.
-__device__ __forceinline__ float det_from_cof(const float F[9], const float C[9]) {
-    float J = dot3(F[0], C[0], F[1], C[1], F[2], C[2]);
+__device__ __forceinline__ float det_fixup(float J, const float F[9]) {
     if (J < 0.1f) {
         const double a0 = F[0], a1 = F[1], a2 = F[2], b0 = F[3], b1 = F[4], b2 = F[5], c0 = F[6], c1 = F[7], c2 = F[8];
         const double d = a0 * (b1 * c2 - b2 * c1) + a1 * (b2 * c0 - b0 * c2) + a2 * (b0 * c1 - b1 * c0);
         J = static_cast<float>(d);
     }
     return J;
+}
+__device__ __forceinline__ float det_from_cof(const float F[9], const float C[9]) {
+    return det_fixup(dot3(F[0], C[0], F[1], C[1], F[2], C[2]), F);
 }
 
 // One (element, quadrature point) contribution (Jx built from displacements) to the force on node r and to
