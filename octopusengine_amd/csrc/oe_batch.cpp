@@ -271,80 +271,157 @@ GatherTimer::~GatherTimer() {
     for (hipEvent_t e : pool) (void)hipEventDestroy(e);
 }
 
-void SideStream::create() {
-    if (stream) return;
-    OE_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    OE_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
-    OE_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
-}
+namespace {
+// One schedule's launches on its stream.
+struct Chain {
+    const Schedule& sch;
+    hipStream_t stream;
+    GatherTimer* timer;
+    BatchVArgs v;
+    BatchGatherArgs g;
+    BatchRefreshArgs r;
+    BatchQ2FusedArgs tk;
+    BatchFusedArgs ft;
 
-SideStream::~SideStream() {
-    if (fork) (void)hipEventDestroy(fork);
-    if (join) (void)hipEventDestroy(join);
-    if (stream) (void)hipStreamDestroy(stream);
-}
+    Chain(const Schedule& s, const DeviceSchedule& dev, const SceneDev* d_scenes, float h, hipStream_t st,
+          GatherTimer* t)
+        : sch(s), stream(st), timer(t), v{d_scenes, dev.vsegs.get(), static_cast<int>(s.vsegs.size()), h, 0},
+          g{d_scenes, dev.segs.get(), 0, 0, 0, h}, r{d_scenes, dev.jsegs.get(), 0, 0, 0},
+          tk{d_scenes, dev.segs.get(), 0, 0, 0, h, s.q2_basis, 0}, ft{d_scenes, dev.segs.get(), 0, 0, 0, h, 0} {}
 
-void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const SceneDev* d_scenes, float dt, int substeps,
-                     hipStream_t stream, GatherTimer* timer, SideStream* side) {
-    if (sch.vsegs.empty()) return;
-    auto is_q2 = [](const Schedule::GLaunch& gl) { return gl.S == 27 && gl.Q == 27; };
-    bool any_q2 = false, any_other = false;
-    for (const Schedule::GLaunch& gl : sch.glaunches) (is_q2(gl) ? any_q2 : any_other) = true;
-    const bool split = side && side->stream && !timer && any_q2 && any_other;
-    const float h = dt / static_cast<float>(substeps);
-    BatchVArgs v{d_scenes, dev.vsegs.get(), static_cast<int>(sch.vsegs.size()), h, 0};
-    BatchGatherArgs g{d_scenes, dev.segs.get(), 0, 0, 0, h};
-    BatchRefreshArgs r{d_scenes, dev.jsegs.get(), 0, 0, 0};
-    BatchQ2FusedArgs tk{d_scenes, dev.segs.get(), 0, 0, 0, h, sch.q2_basis, 0};
-    BatchFusedArgs ft{d_scenes, dev.segs.get(), 0, 0, 0, h, 0};
-    for (int sub = 0; sub < substeps; ++sub) {
-        launch_batch_predict(v, sch.vblocks, stream);
-        for (int it = 0; it < sch.max_iterations; ++it) {
-            g.iteration = r.iteration = tk.iteration = ft.iteration = it;
-            for (const Schedule::JLaunch& jl : sch.jlaunches) {
-                r.seg_first = jl.seg_first;
-                r.seg_count = jl.seg_count;
-                if (!launch_batch_ju_refresh(jl.S, jl.Q, r, jl.nblocks, stream))
-                    throw std::invalid_argument("unsupported element in batch");
-            }
-            if (split) {
-                OE_HIP(hipEventRecord(side->fork, stream));
-                OE_HIP(hipStreamWaitEvent(side->stream, side->fork, 0));
-            }
-            for (const Schedule::GLaunch& gl : sch.glaunches) {
-                const hipStream_t ls = split && is_q2(gl) ? side->stream : stream;
-                g.seg_first = gl.seg_first;
-                g.seg_count = gl.seg_count;
-                if (timer) timer->before(ls, gl.element);
-                if (gl.mode == PASS_TASKS && is_q2(gl)) {
-                    tk.seg_first = gl.seg_first;
-                    tk.seg_count = gl.seg_count;
-                    tk.latency = gl.form == TASKS_LATENCY ? 1 : 0;
-                    if (gl.form == TASKS_THROUGHPUT && q2_pencil(gl.inc))
-                        launch_batch_q2_pencil(tk, gl.nblocks, ls);
-                    else
-                        launch_batch_q2_fused(tk, gl.nblocks, ls);
-                } else if (gl.mode == PASS_TASKS) {
-                    ft.seg_first = gl.seg_first;
-                    ft.seg_count = gl.seg_count;
-                    ft.form = gl.form;
-                    if (!launch_batch_fused_tasks(gl.S, gl.Q, ft, gl.nblocks, ls))
-                        throw std::invalid_argument("unsupported element in batch");
-                } else if (!launch_batch_gather(gl.S, gl.Q, gl.L, gl.QL, gl.mode == PASS_CACHE, g, gl.nblocks, ls)) {
-                    throw std::invalid_argument("unsupported gather tile in batch");
-                }
-                if (timer) timer->after(ls);
-            }
-            if (split) {
-                OE_HIP(hipEventRecord(side->join, side->stream));
-                OE_HIP(hipStreamWaitEvent(stream, side->join, 0));
-            }
-            v.iteration = it;
-            launch_batch_fix_box(v, sch.vblocks, stream);
+    void predict() { launch_batch_predict(v, sch.vblocks, stream); }
+    void velocity() { launch_batch_velocity(v, sch.vblocks, stream); }
+    void refresh(int it) {
+        g.iteration = r.iteration = tk.iteration = ft.iteration = v.iteration = it;
+        for (const Schedule::JLaunch& jl : sch.jlaunches) {
+            r.seg_first = jl.seg_first;
+            r.seg_count = jl.seg_count;
+            if (!launch_batch_ju_refresh(jl.S, jl.Q, r, jl.nblocks, stream))
+                throw std::invalid_argument("unsupported element in batch");
         }
-        launch_batch_velocity(v, sch.vblocks, stream);
+    }
+    void pass(const Schedule::GLaunch& gl) {
+        g.seg_first = tk.seg_first = ft.seg_first = gl.seg_first;
+        g.seg_count = tk.seg_count = ft.seg_count = gl.seg_count;
+        if (timer) timer->before(stream, gl.element);
+        if (gl.mode == PASS_TASKS && gl.element == Hexa27) {
+            tk.latency = gl.form == TASKS_LATENCY ? 1 : 0;
+            if (gl.form == TASKS_THROUGHPUT && q2_pencil(gl.inc))
+                launch_batch_q2_pencil(tk, gl.nblocks, stream);
+            else
+                launch_batch_q2_fused(tk, gl.nblocks, stream);
+        } else if (gl.mode == PASS_TASKS) {
+            ft.form = gl.form;
+            if (!launch_batch_fused_tasks(gl.S, gl.Q, ft, gl.nblocks, stream))
+                throw std::invalid_argument("unsupported element in batch");
+        } else if (!launch_batch_gather(gl.S, gl.Q, gl.L, gl.QL, gl.mode == PASS_CACHE, g, gl.nblocks, stream)) {
+            throw std::invalid_argument("unsupported gather tile in batch");
+        }
+        if (timer) timer->after(stream);
+    }
+    void constraints() { launch_batch_fix_box(v, sch.vblocks, stream); }
+};
+
+// The chains' launches dealt out in turn, so that none waits for the host.
+void run_chains(std::vector<Chain>& chains, int substeps) {
+    int iterations = 0;
+    for (const Chain& c : chains) iterations = std::max(iterations, c.sch.max_iterations);
+    for (int sub = 0; sub < substeps; ++sub) {
+        for (Chain& c : chains) c.predict();
+        for (int it = 0; it < iterations; ++it) {
+            auto runs = [&](const Chain& c) { return it < c.sch.max_iterations; };
+            size_t passes = 0;
+            for (Chain& c : chains)
+                if (runs(c)) {
+                    c.refresh(it);
+                    passes = std::max(passes, c.sch.glaunches.size());
+                }
+            for (size_t i = 0; i < passes; ++i)
+                for (Chain& c : chains)
+                    if (runs(c) && i < c.sch.glaunches.size()) c.pass(c.sch.glaunches[i]);
+            for (Chain& c : chains)
+                if (runs(c)) c.constraints();
+        }
+        for (Chain& c : chains) c.velocity();
     }
 }
+}  // namespace
+
+void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const SceneDev* d_scenes, float dt, int substeps,
+                     hipStream_t stream, GatherTimer* timer) {
+    if (sch.vsegs.empty()) return;
+    std::vector<Chain> chains;
+    chains.emplace_back(sch, dev, d_scenes, dt / static_cast<float>(substeps), stream, timer);
+    run_chains(chains, substeps);
+}
+
+namespace {
+// The scenes of a batch by chain: 27-node hexahedra apart from the other
+// element types, and up to 3 chains of about equal work, the class with more
+// work per chain split first.  A chain's passes wait for one another with the
+// chip partly idle (a pass's last blocks, its launch, blocks that all wait on
+// the same loads); other chains' blocks run there.  Mixed beams of 8-64 x 4-16 x
+// 4-16 cells, 4 / 8 / 16 / 32 / 64 / 128 scenes, ms per 4 substeps: on one stream
+// 21.8 / 23.5 / 26.1 / 34.6 / 53.5 / 87.6; with the Q2 passes on a second stream
+// joined in every iteration 18.2 / 19.4 / 20.9 / 30.2 / 45.9 / 75.1; now 17.0 /
+// 18.1 / 19.2 / 25.0 / 39.4 / 70.9.
+// A fourth chain, on as many hardware queues as the runtime has by default, was
+// slower again (16 scenes 25.2, 32 scenes 31.7, 64 scenes 47.0).
+// A chain keeps at least kChainPoints (incidence, quadrature point) pairs per
+// colour pass (about 15,000 Q2 incidences, or 100,000 P2): below, the passes are
+// launch-bound and more of them only cost the host.
+constexpr int kMaxChains = 1 + Engine::kSideStreams;
+// And no chain may hold over kChainBalance times its share, or the others wait
+// for it at the end of the step.
+constexpr double kChainPoints = 4e5, kChainBalance = 1.15;
+std::vector<std::vector<int>> group_scenes(const std::vector<Scene*>& scenes) {
+    std::vector<int> member[2];   // Hexa27, the others
+    double total[2] = {0.0, 0.0}, pass[2] = {0.0, 0.0};
+    auto work = [&](int i) { return static_cast<double>(scenes[i]->fem->E) * scenes[i]->fem->S * scenes[i]->fem->Q; };
+    for (int i = 0; i < static_cast<int>(scenes.size()); ++i) {
+        const int k = scenes[i]->mesh.element == Hexa27 ? 0 : 1;
+        member[k].push_back(i);
+        total[k] += work(i);
+        pass[k] += work(i) / std::max(1, scenes[i]->vbd_fem->nb_colors());
+    }
+    // member[k] in n groups: largest scene first, each to the group with the least work so far
+    for (std::vector<int>& m : member)
+        std::stable_sort(m.begin(), m.end(), [&](int a, int b) { return work(a) > work(b); });
+    auto dealt = [&](int k, int n) {
+        std::vector<std::vector<int>> g(n);
+        std::vector<double> load(n, 0.0);
+        for (int i : member[k]) {
+            const size_t j = std::min_element(load.begin(), load.end()) - load.begin();
+            g[j].push_back(i);
+            load[j] += work(i);
+        }
+        if (*std::max_element(load.begin(), load.end()) * n > kChainBalance * total[k]) g.clear();
+        return g;
+    };
+    std::vector<std::vector<int>> groups[2];
+    for (int k = 0; k < 2; ++k)
+        if (!member[k].empty()) groups[k] = dealt(k, 1);
+    while (groups[0].size() + groups[1].size() < kMaxChains) {
+        std::vector<std::vector<int>> next;
+        int best = -1;
+        for (int k = 0; k < 2; ++k) {
+            const int n = static_cast<int>(groups[k].size()) + 1;
+            if (n == 1 || pass[k] < kChainPoints * n) continue;
+            if (best >= 0 && total[k] / (n - 1) <= total[best] / groups[best].size()) continue;
+            std::vector<std::vector<int>> g = dealt(k, n);
+            if (g.empty()) continue;
+            next = std::move(g);
+            best = k;
+        }
+        if (best < 0) break;
+        groups[best] = std::move(next);
+    }
+    std::vector<std::vector<int>> out;
+    for (auto& g : groups) out.insert(out.end(), g.begin(), g.end());
+    for (std::vector<int>& g : out) std::sort(g.begin(), g.end());
+    return out;
+}
+}  // namespace
 
 Batch::Batch(Engine* e, std::vector<Scene*> sc) : eng(e), scenes(std::move(sc)), tiles(default_tiles()) {
     if (scenes.empty()) throw std::invalid_argument("empty batch");
@@ -361,13 +438,13 @@ Batch::Batch(Engine* e, std::vector<Scene*> sc) : eng(e), scenes(std::move(sc)),
     flags.reserve(scenes.size());
     for (Scene* s : scenes) flags.emplace_back(&eng->pool, fixed_flags(*s));
     d_scenes.allocate(&eng->pool, scenes.size());
-    side.create();
     rebuild();
     for (Scene* s : scenes) s->batches.push_back(this);
 }
 
 Batch::~Batch() {
     drop_graph();
+    if (fork) (void)hipEventDestroy(fork);
     for (Scene* s : scenes) {
         if (!s) continue;
         auto& v = s->batches;
@@ -391,6 +468,45 @@ void Batch::rebuild() {
     for (size_t i = 0; i < idx.size(); ++i) idx[i] = static_cast<int>(i);
     sched.build(scenes, idx, tiles);
     dsched.upload(eng, sched, eng->stream, true);
+    const std::vector<std::vector<int>> parts = group_scenes(scenes);
+    if (groups.size() != parts.size()) groups = std::vector<Group>(parts.size());
+    for (size_t i = 0; i < parts.size(); ++i) {
+        std::vector<Scene*> sc;
+        for (int k : parts[i]) sc.push_back(scenes[k]);
+        groups[i].sched.build(sc, parts[i], tiles);
+        groups[i].dev.upload(eng, groups[i].sched, eng->stream, true);
+        groups[i].stream = i > 0 ? eng->side_stream(static_cast<int>(i) - 1) : eng->stream;
+        if (i > 0 && !groups[i].join) OE_HIP(hipEventCreateWithFlags(&groups[i].join, hipEventDisableTiming));
+    }
+    if (!fork) OE_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+}
+
+void Batch::launch(float dt, int substeps) {
+    if (streams != 2 || timer.enabled || groups.size() < 2) {
+        launch_schedule(sched, dsched, d_scenes.get(), dt, substeps, eng->stream, timer.enabled ? &timer : nullptr);
+        return;
+    }
+    const float h = dt / static_cast<float>(substeps);
+    std::vector<Chain> chains;
+    OE_HIP(hipEventRecord(fork, eng->stream));
+    for (Group& g : groups) {
+        if (g.join) OE_HIP(hipStreamWaitEvent(g.stream, fork, 0));
+        chains.emplace_back(g.sched, g.dev, d_scenes.get(), h, g.stream, nullptr);
+    }
+    auto join = [&] {
+        for (Group& g : groups)
+            if (g.join) {
+                OE_HIP(hipEventRecord(g.join, g.stream));
+                OE_HIP(hipStreamWaitEvent(eng->stream, g.join, 0));
+            }
+    };
+    try {
+        run_chains(chains, substeps);
+    } catch (...) {
+        join();   // what was launched stays ordered before the engine's later work
+        throw;
+    }
+    join();
 }
 
 void Batch::set_tile(Element e, GatherTile t) {
@@ -420,15 +536,13 @@ void Batch::step(float dt, int substeps) {
     if (broken) throw std::logic_error("a scene of this batch was destroyed");
     if (!(dt > 0.f) || substeps <= 0) throw std::invalid_argument("step needs dt > 0 and substeps > 0");
     if (!use_graph || timer.enabled) {
-        launch_schedule(sched, dsched, d_scenes.get(), dt, substeps, eng->stream, timer.enabled ? &timer : nullptr,
-                        streams == 2 ? &side : nullptr);
+        launch(dt, substeps);
     } else {
         if (!graph_exec || graph_dt != dt || graph_sub != substeps) {
             drop_graph();
             OE_HIP(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
             try {
-                launch_schedule(sched, dsched, d_scenes.get(), dt, substeps, eng->stream, nullptr,
-                                streams == 2 ? &side : nullptr);
+                launch(dt, substeps);
             } catch (...) {
                 hipGraph_t g = nullptr;
                 (void)hipStreamEndCapture(eng->stream, &g);

@@ -99,23 +99,9 @@ struct GatherTimer {
     ~GatherTimer();
 };
 
-// A second stream for the Q2 colour passes of a schedule that also holds other
-// element types: the two chains of colour passes are independent within an
-// iteration, so they run side by side and fill each other's idle issue slots
-// (the Q2 pass is VALU-bound, the P2 pass waits on loads).  The fork and join
-// events order them against the per-iteration passes on the main stream.
-struct SideStream {
-    hipStream_t stream = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
-    void create();
-    ~SideStream();
-};
-
 // Enqueue `substeps` substeps of dt/substeps for every scene of the schedule.
-// With `side` (and no timer) a schedule with Q2 and other element types runs
-// its Q2 colour passes on side->stream.
 void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const SceneDev* d_scenes, float dt, int substeps,
-                     hipStream_t stream, GatherTimer* timer, SideStream* side = nullptr);
+                     hipStream_t stream, GatherTimer* timer);
 
 // The default tile of every element type: a scene's (default_tile) for a
 // server's ticks, and for a batch the same but 28-incidence Q2 pencil blocks.
@@ -130,7 +116,7 @@ struct Batch {
     ~Batch();
     void step(float dt, int substeps);
     void set_graph(bool on);
-    void set_streams(int n);   // 1 or 2 (the Q2 passes on a second stream)
+    void set_streams(int n);   // 1, or 2: the groups side by side
     void set_tile(Element e, GatherTile t);
     void rebuild();
     void scene_destroyed(Scene* s);
@@ -143,9 +129,24 @@ struct Batch {
     Schedule sched;
     DeviceSchedule dsched;
     GatherTimer timer;
-    SideStream side;
 
 private:
+    // Scenes whose steps run on one stream (group 0: the engine's, group i: its
+    // side stream i - 1).  Groups share nothing, so a step forks and joins once.
+    struct Group {
+        Schedule sched;
+        DeviceSchedule dev;
+        hipStream_t stream = nullptr;
+        hipEvent_t join = nullptr;
+        Group() = default;
+        Group(const Group&) = delete;
+        ~Group() {
+            if (join) (void)hipEventDestroy(join);
+        }
+    };
+    std::vector<Group> groups;
+    hipEvent_t fork = nullptr;
+    void launch(float dt, int substeps);
     bool broken = false;   // a scene of the batch was destroyed
     bool use_graph = false;
     int streams = 2;

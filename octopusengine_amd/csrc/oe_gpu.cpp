@@ -31,7 +31,18 @@ Engine::Engine(int dev, size_t budget_bytes) : device(dev) {
     pool.budget = budget_bytes;
 }
 
+hipStream_t Engine::side_stream(int i) {
+    std::lock_guard<std::mutex> lk(side_mu);
+    if (!sides[i]) OE_HIP(hipStreamCreateWithFlags(&sides[i], hipStreamNonBlocking));
+    return sides[i];
+}
+
 Engine::~Engine() {
+    for (hipStream_t s : sides)
+        if (s) {
+            (void)hipStreamSynchronize(s);
+            (void)hipStreamDestroy(s);
+        }
     if (stream) {
         (void)hipStreamSynchronize(stream);
         (void)hipStreamDestroy(stream);

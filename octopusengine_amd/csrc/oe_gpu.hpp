@@ -51,6 +51,13 @@ struct Readback {
 struct Engine {
     int device = 0;
     hipStream_t stream = nullptr;
+    // Further streams for work that forks from `stream` and joins it again (the
+    // groups of a batch), made when first asked for.  All batches of an engine
+    // share them: each would otherwise add its own to the process's few
+    // hardware queues (4 by default), and two streams of one step would land on
+    // the same queue.
+    static constexpr int kSideStreams = 2;
+    hipStream_t side_stream(int i);
     MemoryPool pool;
     bool autotune = false;   // tune the layout of every VBD / explicit scene created
     Readback readback;
@@ -62,6 +69,10 @@ struct Engine {
     ~Engine();
     Engine(const Engine&) = delete;
     Engine& operator=(const Engine&) = delete;
+
+private:
+    std::mutex side_mu;
+    hipStream_t sides[kSideStreams] = {};
 };
 
 struct GPU_ParticleSystem {
