@@ -207,8 +207,9 @@ oe_status oe_batch_set_graph(oe_batch* b, int32_t enable);
  * whole step, and the results are the same.  No counterpart in the reference. */
 oe_status oe_batch_set_streams(oe_batch* b, int32_t n);
 oe_status oe_batch_set_tile(oe_batch* b, int32_t element, int32_t lanes, int32_t qpl, int32_t mode);
-/* Full layout per element type (latency_blocks has no effect: batches run the
- * throughput form); get returns the layout in use. */
+/* Full layout per element type; latency_blocks applies to a colour pass over all
+ * scenes of the type.  A batch starts with the scenes' defaults but longer Q2
+ * blocks where its passes fill the GPU; get returns the layout in use. */
 oe_status oe_batch_set_tile_ex(oe_batch* b, int32_t element, const oe_tile* t);
 oe_status oe_batch_get_tile_ex(oe_batch* b, int32_t element, oe_tile* t);
 /* Autotune every element type of the batch: the candidates are timed on the

@@ -23,11 +23,34 @@ GPU_Box_Limit* find_box(const Scene& s) {
 }
 }  // namespace
 
-std::map<int, GatherTile> default_tiles(bool served) {
+std::map<int, GatherTile> default_tiles() {
     std::map<int, GatherTile> t;
     for (Element e : {Tetra, Hexa, Tetra10, Tetra20, Hexa27}) t[e] = default_tile(e);
-    // a batch's launches hold many blocks: the longer pencil blocks
-    if (!served) t[Hexa27].inc = kQ2PencilIncPerBlock;
+    return t;
+}
+
+// A batch's launches are a server's (default_tile) or much longer, and run
+// beside one another.
+//  * Q2 blocks of 28 incidences from kLongBlocks of them per colour pass on (2 a
+//    SIMD): a block's rounds then overlap other blocks'.  Below, 14 (two rounds
+//    in place of four): 24 beams of 32x8x8 (1,650 blocks of 28) step in 7.7 ms
+//    (8.9 with 28), 32 of them in 9.1 (9.5), 32 mixed beams (2,600) in 14.4 (12.6).
+//  * Q2 passes of fewer than 1024 blocks of 14 take the latency form (a scene and
+//    a server 512): 4 beams of 32x8x8 (546 blocks) step in 3.6 ms (5.3), 6 in 5.4
+//    (5.6), 8 (1,090) in 5.5 either way, 12 in 6.6 (8.0 in the latency form).
+//  * P2 passes of fewer than 256 blocks take the latency or split form (512): 16
+//    beams of 16x4x4 (88 blocks) step in 1.41 ms (1.47 in the throughput form),
+//    64 of them (350) in 1.80 (1.75).
+std::map<int, GatherTile> batch_tiles(const std::vector<Scene*>& scenes) {
+    constexpr double kLongBlocks = 2048;
+    std::map<int, GatherTile> t = default_tiles();
+    double per_pass = 0.0;
+    for (const Scene* s : scenes)
+        if (s->mesh.element == Hexa27)
+            per_pass += 27.0 * s->fem->E / std::max(1, s->vbd_fem->nb_colors());
+    if (per_pass >= kLongBlocks * kQ2PencilIncPerBlock) t[Hexa27].inc = kQ2PencilIncPerBlock;
+    else t[Hexa27].lat_blocks = 1024;
+    t[Tetra10].lat_blocks = 256;
     return t;
 }
 
@@ -113,7 +136,7 @@ void Schedule::clear() {
 }
 
 void Schedule::build(const std::vector<Scene*>& scenes, const std::vector<int>& table_index,
-                     const std::map<int, GatherTile>& tiles, bool want_latency) {
+                     const std::map<int, GatherTile>& tiles, const Schedule* whole) {
     clear();
     int max_colors = 0;
     for (Scene* s : scenes) {
@@ -134,11 +157,14 @@ void Schedule::build(const std::vector<Scene*>& scenes, const std::vector<int>& 
             gl.color = c;
             gl.element = el;
             gl.seg_first = static_cast<int>(segs.size());
-            // Task passes take the latency form when it was asked for, every
-            // scene of the launch has its vertex blocks, and the throughput
-            // form would give fewer than 2 blocks per CU.
+            // Task passes take the latency form when every scene of the launch has
+            // its vertex blocks and the throughput form would give fewer than the
+            // tile's latency_blocks (2 per CU).
             const GatherTile et = tile_of(tiles, el);
-            if (want_latency && et.mode == PASS_TASKS) {
+            if (whole) {
+                for (const GLaunch& w : whole->glaunches)
+                    if (w.color == c && w.element == el) gl.form = w.form;
+            } else if (et.mode == PASS_TASKS) {
                 bool all = true;
                 int64_t through_blocks = 0, incidences = 0;
                 for (Scene* s : scenes) {
@@ -423,7 +449,7 @@ std::vector<std::vector<int>> group_scenes(const std::vector<Scene*>& scenes) {
 }
 }  // namespace
 
-Batch::Batch(Engine* e, std::vector<Scene*> sc) : eng(e), scenes(std::move(sc)), tiles(default_tiles()) {
+Batch::Batch(Engine* e, std::vector<Scene*> sc) : eng(e), scenes(std::move(sc)) {
     if (scenes.empty()) throw std::invalid_argument("empty batch");
     for (size_t i = 0; i < scenes.size(); ++i) {
         Scene* s = scenes[i];
@@ -435,6 +461,7 @@ Batch::Batch(Engine* e, std::vector<Scene*> sc) : eng(e), scenes(std::move(sc)),
         if (s->server) throw std::logic_error("the scene is held by a server");
         check_batchable(*s);
     }
+    tiles = batch_tiles(scenes);
     flags.reserve(scenes.size());
     for (Scene* s : scenes) flags.emplace_back(&eng->pool, fixed_flags(*s));
     d_scenes.allocate(&eng->pool, scenes.size());
@@ -473,7 +500,7 @@ void Batch::rebuild() {
     for (size_t i = 0; i < parts.size(); ++i) {
         std::vector<Scene*> sc;
         for (int k : parts[i]) sc.push_back(scenes[k]);
-        groups[i].sched.build(sc, parts[i], tiles);
+        groups[i].sched.build(sc, parts[i], tiles, &sched);
         groups[i].dev.upload(eng, groups[i].sched, eng->stream, true);
         groups[i].stream = i > 0 ? eng->side_stream(static_cast<int>(i) - 1) : eng->stream;
         if (i > 0 && !groups[i].join) OE_HIP(hipEventCreateWithFlags(&groups[i].join, hipEventDisableTiming));

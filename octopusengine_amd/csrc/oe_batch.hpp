@@ -14,7 +14,8 @@
 //                        fixation + box limit (all vertices, one fused kernel)
 //   velocity update
 // Each scene still sees the reference's order: ascending colours, constraints
-// after every sweep.
+// after every sweep.  A batch deals its scenes into up to three groups, each with
+// this sequence on a stream of its own (group_scenes in oe_batch.cpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -60,11 +61,11 @@ struct Schedule {
     std::map<int, int64_t> vertex_updates_by_element;
 
     void clear();
-    // scenes[i] is placed at SceneDev table index table_index[i]; want_latency
-    // lets task passes too small to fill the GPU (as a server's ticks often
-    // are) take the latency form
+    // scenes[i] is placed at SceneDev table index table_index[i]; task passes
+    // too small to fill the GPU take the latency form, or those of a part of a
+    // schedule the forms of the whole
     void build(const std::vector<Scene*>& scenes, const std::vector<int>& table_index,
-               const std::map<int, GatherTile>& tiles, bool want_latency = false);
+               const std::map<int, GatherTile>& tiles, const Schedule* whole = nullptr);
 };
 
 // Device copies of a schedule's tables (grown on demand, reused across uploads).
@@ -103,9 +104,10 @@ struct GatherTimer {
 void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const SceneDev* d_scenes, float dt, int substeps,
                      hipStream_t stream, GatherTimer* timer);
 
-// The default tile of every element type: a scene's (default_tile) for a
-// server's ticks, and for a batch the same but 28-incidence Q2 pencil blocks.
-std::map<int, GatherTile> default_tiles(bool served = false);
+// The tile of every element type: a scene's (default_tile), which a server's
+// ticks start with, and what a batch of these scenes starts with.
+std::map<int, GatherTile> default_tiles();
+std::map<int, GatherTile> batch_tiles(const std::vector<Scene*>& scenes);
 
 // A batch registers itself with its scenes (Scene::batches).  A scene may be
 // in several batches but appear once per batch, and a scene held by a server

@@ -27,10 +27,11 @@ constexpr int kQ2FusedMaxSlots = 64;
 // blocks of 7 tasks at a time, in up to 5 rounds; chosen by a tile of 14, 21,
 // 28 or 35 incidences per block.  Other tile sizes (up to 32) take the 27-lane
 // throughput form.
-//  * 28 (4 rounds): batches, whose launches hold enough blocks to cover the
+//  * 28 (4 rounds): batches whose launches hold enough blocks to cover the
 //    longer blocks (256-scene step 47.2 ms; 51.4 ms with the 27-lane form).
-//  * 14 (2 rounds): single scenes and the server, whose launches are short of
-//    blocks (served p99 6.6 ms; 7.8 ms at 28 and 7.0 ms with the 27-lane form).
+//  * 14 (2 rounds): single scenes, smaller batches (batch_tiles) and the server,
+//    whose launches are short of blocks (served p99 6.6 ms; 7.8 ms at 28 and
+//    7.0 ms with the 27-lane form).
 // A scene whose vertices have more incident elements than the tile's blocks
 // hold takes the next size up (q2_pencil_fit): the kernel runs blocks of any
 // of these sizes, so scenes of one launch may differ.

@@ -5,7 +5,7 @@
 
 namespace oe {
 
-Server::Server(Engine* eng, int max_batch, int nstreams) : eng_(eng), max_batch_(max_batch), tiles_(default_tiles(true)) {
+Server::Server(Engine* eng, int max_batch, int nstreams) : eng_(eng), max_batch_(max_batch), tiles_(default_tiles()) {
     if (max_batch < 1 || nstreams < 1 || nstreams > 8) throw std::invalid_argument("max_batch >= 1, 1 <= streams <= 8");
     slots_.resize(nstreams);
     for (StreamSlot& s : slots_) {
@@ -235,7 +235,7 @@ bool Server::try_launch(std::unique_lock<std::mutex>& lk, int si) {
     launching_++;   // holds add_scene() off the table until the tick is in flight
     lk.unlock();
     // plan + launch outside the lock so that submit() is never blocked by it
-    slot.sched.build(sc, idx, tiles_, true);
+    slot.sched.build(sc, idx, tiles_);
     slot.dev.upload(eng_, slot.sched, slot.stream, false);
     launch_schedule(slot.sched, slot.dev, table, dt, sub, slot.stream, nullptr);
     OE_HIP(hipEventRecord(slot.done, slot.stream));

@@ -39,3 +39,27 @@ def test_groups_give_the_same_steps(engine, name):
     for s in sets:
         for x in s:
             x.close()
+
+
+@pytest.mark.parametrize("el,cells,n", [(oe.HEXA27, (8, 2, 2), 1), (oe.HEXA27, (16, 4, 4), 33),
+                                        (oe.HEXA27, (16, 4, 4), 60), (oe.TETRA10, (8, 2, 2), 1),
+                                        (oe.TETRA10, (16, 4, 4), 12), (oe.TETRA10, (16, 4, 4), 40)])
+def test_small_batches(engine, el, cells, n):
+    """Batches on both sides of the lines between the forms of their passes
+    against the throughput form: the same terms in another order, two ulps of a
+    coordinate below 1 m after a step; and the same steps on one stream."""
+    out = []
+    for lat, streams in ((None, 2), (None, 1), (0, 2)):
+        s = [oe.make_scene(engine, el, cells) for _ in range(n)]
+        b = oe.Batch(engine, s)
+        b.set_streams(streams)
+        if lat is not None:
+            t = b.get_tile_ex(el)
+            b.set_tile_ex(el, t["lanes"], t["qpl"], oe.PASS_TASKS, t["inc_per_block"], lat)
+        b.step(0.005, 1)
+        out.append(np.stack([x.positions().astype(np.float64) for x in s]))
+        b.close()
+        for x in s:
+            x.close()
+    assert np.array_equal(out[0], out[1])
+    assert np.abs(out[0] - out[2]).max() <= 1.2e-7
