@@ -26,7 +26,7 @@ CXX = shutil.which("g++") or "g++"
 COMMON = ["-O3", "-std=c++17", "-fPIC"]
 # Packed FP32 instructions are disabled for all device code.
 HIP_FLAGS = COMMON + [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-                      "-fno-gpu-rdc"]
+                      "-fno-gpu-rdc", "-mllvm", "-amdgpu-kernarg-preload-count=4"]
 # Host-only geometry / graph code: no FMA contraction, so float expressions are
 # rounded term by term.
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off"]

@@ -480,9 +480,10 @@ __device__ __forceinline__ void point_block(const PSView& ps, const FemView& f, 
 }
 
 template <int S, int Q>
-__global__ __launch_bounds__(kFusedThreads) void k_point_tasks(FusedTaskArgs a) {
+__global__ __launch_bounds__(kFusedThreads) void k_point_tasks(const int4* blocks, int first, int count,
+                                                               FusedTaskArgs a) {
     __shared__ PointLDS<S, Q> sh;
-    const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
+    const int4 blk = gload(blocks, first + xcd_block(blockIdx.x, count));
     point_block<S, Q>(a.ps, a.fem, a.own, a.mt, a.y, a.damping, a.dt, blk, sh);
 }
 
@@ -767,10 +768,11 @@ __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, 
 }
 
 template <int S, int Q, bool LAT>
-__global__ __launch_bounds__(kFusedThreads) void k_fused_tasks(FusedTaskArgs a, ShapeArg<S> g) {
+__global__ __launch_bounds__(kFusedThreads) void k_fused_tasks(const int4* blocks, int first, int count,
+                                                               FusedTaskArgs a, ShapeArg<S> g) {
     __shared__ float part[LAT ? kFusedIncPerBlockLat : kFusedIncPerBlock][9];
     __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, LAT>()];
-    const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
+    const int4 blk = gload(blocks, first + xcd_block(blockIdx.x, count));
     fused_block<S, Q, LAT>(a.ps, a.fem, a.own, a.mt, g, a.y, a.damping, a.dt, blk, part,
                               dn_lds[threadIdx.x >> 6]);
 }
@@ -1090,15 +1092,18 @@ void OE_FN(launch_fused_tasks_)(const FusedTaskArgs& a, hipStream_t s) {
     if (a.count <= 0) return;
 #if OE_GATHER_S == 10
     if (a.form == TASKS_THROUGHPUT) {
-        hipLaunchKernelGGL((k_fused_tasks<S, Q, false>), dim3(a.count), dim3(kFusedThreads), 0, s, a, shape_arg());
+        hipLaunchKernelGGL((k_fused_tasks<S, Q, false>), dim3(a.count), dim3(kFusedThreads), 0, s, a.blocks,
+                           a.first_block, a.count, a, shape_arg());
         return;
     }
     if (a.form == TASKS_LATENCY) {
-        hipLaunchKernelGGL((k_fused_tasks<S, Q, true>), dim3(a.count), dim3(kFusedThreads), 0, s, a, shape_arg());
+        hipLaunchKernelGGL((k_fused_tasks<S, Q, true>), dim3(a.count), dim3(kFusedThreads), 0, s, a.blocks,
+                           a.first_block, a.count, a, shape_arg());
         return;
     }
 #endif
-    hipLaunchKernelGGL((k_point_tasks<S, Q>), dim3(a.count), dim3(kFusedThreads), 0, s, a);
+    hipLaunchKernelGGL((k_point_tasks<S, Q>), dim3(a.count), dim3(kFusedThreads), 0, s, a.blocks, a.first_block, a.count,
+                       a);
 }
 
 void OE_FN(launch_batch_fused_tasks_)(const BatchFusedArgs& b, int nblocks, hipStream_t s) {

@@ -675,6 +675,11 @@ GPU_PBD_FEM::GPU_PBD_FEM(Engine* e, Element el, const HostMesh& mesh, float youn
         d_p1_nodes = DBuf<int4>(&eng->pool, nodes);
         d_p1_rec = DBuf<float4>(&eng->pool, rec);
         d_color_begin = DBuf<int>(&eng->pool, std::vector<int>(sched.color_begin.begin(), sched.color_begin.end()));
+    } else if (version == Quadrature || version == OptiShared) {
+        std::vector<int> topo(static_cast<size_t>(E) * S);
+        for (int i = 0; i < E; ++i)
+            std::copy_n(&mesh.topo[static_cast<size_t>(sched.eids[i]) * S], S, &topo[static_cast<size_t>(i) * S]);
+        d_topo = DBuf<int>(&eng->pool, topo);
     }
 }
 
@@ -709,6 +714,7 @@ void GPU_PBD_FEM::step(GPU_ParticleSystem* ps, float dt) {
     a.eids = d_eids.get();
     a.p1_nodes = d_p1_nodes.get();
     a.p1_rec = d_p1_rec.get();
+    a.topo = d_topo.get();
     a.dt = dt;
     for (int c = 0; c < colors.nb_color; ++c) {
         a.first = sched.color_begin[c];

@@ -307,6 +307,7 @@ struct GPU_PBD_FEM final : GPU_FEM {
     DBuf<int> d_eids;
     // linear tetrahedra: the elements' node ids and records in schedule order
     // (a colour's elements consecutive), and the colours' first elements
+    DBuf<int> d_topo;   // the V2 form's node ids, S per element in the order of d_eids
     DBuf<int4> d_p1_nodes;
     DBuf<float4> d_p1_rec;   // 3 per element: JX_inv (9), V
     DBuf<int> d_color_begin;

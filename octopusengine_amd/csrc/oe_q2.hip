@@ -348,8 +348,9 @@ __device__ __forceinline__ void q2_block(const PSView& ps, const FemView& fem, c
 }
 
 template <bool LAT>
-__global__ __launch_bounds__(kQ2FusedThreads, LAT ? 1 : 6) void k_q2_fused(Q2FusedArgs a) {
-    const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
+__global__ __launch_bounds__(kQ2FusedThreads, LAT ? 1 : 6) void k_q2_fused(const int4* blocks, int first, int count,
+                                                                          Q2FusedArgs a) {
+    const int4 blk = gload(blocks, first + xcd_block(blockIdx.x, count));
     q2_block<LAT>(a.ps, a.fem, a.own, a.mt, a.basis, a.y, a.damping, a.dt, blk);
 }
 
@@ -381,9 +382,11 @@ __global__ __launch_bounds__(kQ2FusedThreads, LAT ? 1 : 6) void k_batch_q2_fused
 void launch_q2_fused(const Q2FusedArgs& a, hipStream_t s) {
     if (a.count <= 0) return;
     if (a.latency)
-        hipLaunchKernelGGL(k_q2_fused<true>, dim3(a.count), dim3(kQ2FusedThreads), 0, s, a);
+        hipLaunchKernelGGL(k_q2_fused<true>, dim3(a.count), dim3(kQ2FusedThreads), 0, s, a.blocks, a.first_block,
+                           a.count, a);
     else
-        hipLaunchKernelGGL(k_q2_fused<false>, dim3(a.count), dim3(kQ2FusedThreads), 0, s, a);
+        hipLaunchKernelGGL(k_q2_fused<false>, dim3(a.count), dim3(kQ2FusedThreads), 0, s, a.blocks, a.first_block,
+                           a.count, a);
 }
 
 void launch_batch_q2_fused(const BatchQ2FusedArgs& b, int nblocks, hipStream_t s) {

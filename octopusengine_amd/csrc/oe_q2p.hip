@@ -285,8 +285,8 @@ __device__ __forceinline__ void pencil_block(const PSView& ps, const FemView& fe
     if (lane < blk.y) solve_slot_at(ps, slot_vid, slot_nbo, y, damping, dt, part, blk.z);
 }
 
-__global__ __launch_bounds__(64) void k_q2_pencil(Q2FusedArgs a) {
-    const int4 blk = gload(a.blocks, a.first_block + xcd_block(blockIdx.x, gridDim.x));
+__global__ __launch_bounds__(64) void k_q2_pencil(const int4* blocks, int first, int count, Q2FusedArgs a) {
+    const int4 blk = gload(blocks, first + xcd_block(blockIdx.x, count));
     pencil_block(a.ps, a.fem, a.own, a.mt, a.basis, a.y, a.damping, a.dt, blk);
 }
 
@@ -308,7 +308,8 @@ __global__ __launch_bounds__(64) void k_batch_q2_pencil(BatchQ2FusedArgs b) {
 }  // namespace
 
 void launch_q2_pencil(const Q2FusedArgs& a, hipStream_t s) {
-    if (a.count > 0) hipLaunchKernelGGL(k_q2_pencil, dim3(a.count), dim3(64), 0, s, a);
+    if (a.count > 0)
+        hipLaunchKernelGGL(k_q2_pencil, dim3(a.count), dim3(64), 0, s, a.blocks, a.first_block, a.count, a);
 }
 
 void launch_batch_q2_pencil(const BatchQ2FusedArgs& b, int nblocks, hipStream_t s) {

@@ -187,11 +187,11 @@ __device__ __forceinline__ void p1_project(const MaterialView& mt, float dt, con
 // the chain nodes -> positions -> ~450 instructions; reading the nodes again
 // for the second constraint, after an element id and an index load, it took
 // 5.9 us per colour.
-__global__ __launch_bounds__(64) void k_xpbd_p1(XpbdArgs a) {
+__global__ __launch_bounds__(64) void k_xpbd_p1(const int4* nodes, int first, int count, XpbdArgs a) {
     const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= a.count) return;
-    const size_t i = static_cast<size_t>(a.first) + t;
-    const int4 n4 = gload(a.p1_nodes, i);
+    if (t >= count) return;
+    const size_t i = static_cast<size_t>(first) + t;
+    const int4 n4 = gload(nodes, i);
     const float4 r0 = gload(a.p1_rec, 3 * i), r1 = gload(a.p1_rec, 3 * i + 1), r2 = gload(a.p1_rec, 3 * i + 2);
     const int n[4] = {n4.x, n4.y, n4.z, n4.w};
     float4 u[4];
@@ -350,12 +350,14 @@ struct V2Plan {
     float dp[KP][3];     // their dN at point q
     int qn[QN];          // the points of the lane's part
     float dn[QN][3];     // dN of node k there
-    __device__ __forceinline__ void init(const float* dN, int lane) {
+    __device__ __forceinline__ void place(int lane) {
         const int sp = lane % WP, sn = lane % WN;
         point = sp < Q;
         node = sn < S;
         q = point ? sp : Q - 1;
         k = node ? sn : S - 1;
+    }
+    __device__ __forceinline__ void init(const float* dN, int lane) {
 #pragma unroll
         for (int j = 0; j < KP; ++j) {
             const int n = lane / WP * KP + j;
@@ -451,24 +453,29 @@ __device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, con
 // colour), 20-node tetrahedra 10.16 -> 7.45 ms (424 per colour), against
 // 256-thread blocks with workgroup barriers, rolled sums and 4-byte LDS reads.
 template <int S, int Q, bool NARROW>
-__global__ __launch_bounds__(64) void k_xpbd_v2(XpbdArgs a) {
+__global__ __launch_bounds__(64) void k_xpbd_v2(const int* topo, int first, int count, XpbdArgs a) {
     using P_ = V2Plan<S, Q, NARROW>;
     constexpr int EPB = 64 / P_::LPE;
     __shared__ float4 sx[EPB][S];
     __shared__ float4 sP[EPB][Q * 3];
     const int le = threadIdx.x / P_::LPE, lane = threadIdx.x % P_::LPE;
     const int ei = blockIdx.x * EPB + le;
-    const bool valid = ei < a.count;
+    const bool valid = ei < count;
     // a group past the colour's end works on its last element and stores nothing
-    const int eid = gload(a.eids, a.first + (valid ? ei : a.count - 1));
+    const int at = first + (valid ? ei : count - 1);
     P_ pl;
-    pl.init(a.fem.dN, lane);
-    const int vid = gload(a.fem.topo, static_cast<size_t>(eid) * S + pl.k);
+    pl.place(lane);
+    const int vid = gload(topo, static_cast<size_t>(at) * S + pl.k);
+    const int eid = gload(a.eids, at);
+    __builtin_amdgcn_sched_barrier(0);
+    float4 u = gload(static_cast<const float4*>(a.ps.p), vid);
+    const float w = gload(a.ps.w, vid);
     float JXi[9], V;
     load_element_record(a.fem, eid, pl.q, JXi, V);
-    float4 u = gload(static_cast<const float4*>(a.ps.p), vid);
+    __builtin_amdgcn_sched_barrier(0);
+    pl.init(a.fem.dN, lane);
     const float keep = u.w;
-    u.w = gload(a.ps.w, vid);
+    u.w = w;
     if (lane < S) sx[le][lane] = u;
     wave_lds_sync();
     v2_project(a.mt, a.dt, pl, JXi, V, sx[le], sP[le]);
@@ -487,7 +494,8 @@ void launch_v0(const XpbdArgs& a, hipStream_t s) {
 template <int S, int Q, bool NARROW = false>
 void launch_v2(const XpbdArgs& a, hipStream_t s) {
     constexpr int EPB = 64 / V2Plan<S, Q, NARROW>::LPE;
-    hipLaunchKernelGGL((k_xpbd_v2<S, Q, NARROW>), dim3((a.count + EPB - 1) / EPB), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_xpbd_v2<S, Q, NARROW>), dim3((a.count + EPB - 1) / EPB), dim3(64), 0, s, a.topo, a.first,
+                       a.count, a);
 }
 
 }  // namespace
@@ -500,7 +508,7 @@ bool launch_xpbd(int S, int Q, bool v0_form, const XpbdArgs& a, hipStream_t s) {
     if (a.count <= 0) return true;
     if (v0_form) {
         if (S == 4 && Q == 1) {
-            hipLaunchKernelGGL(k_xpbd_p1, dim3((a.count + 63) / 64), dim3(64), 0, s, a);
+            hipLaunchKernelGGL(k_xpbd_p1, dim3((a.count + 63) / 64), dim3(64), 0, s, a.p1_nodes, a.first, a.count, a);
             return true;
         }
         if (S == 8 && Q == 8) { launch_v0<8, 8>(a, s); return true; }

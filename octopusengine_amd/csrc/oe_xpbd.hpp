@@ -24,6 +24,7 @@ struct XpbdArgs {
     // elements in the order of eids
     const int4* p1_nodes;
     const float4* p1_rec;
+    const int* topo;   // the V2 form's node ids, S per element in the order of eids
 };
 
 // A whole run of substeps of a small linear-tetrahedron scene in one launch of
