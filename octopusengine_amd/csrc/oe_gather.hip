@@ -331,6 +331,7 @@ struct PointLDS {
     // node values per group; the odd row stride spreads the groups over the banks
     float4 xs[LQ > 1 ? G : 1][LQ > 1 ? (S | 1) : 1];
     float part[kFusedIncPerBlock][9];
+    int2 range[kFusedMaxSlots];         // per slot: first partial, partials
     float dn[LQ > 1 ? Q * S * 3 : 1];   // (k Q + q) 3 + c: neighbouring lanes read neighbouring words
 };
 
@@ -472,11 +473,14 @@ __device__ __forceinline__ void point_block(const PSView& ps, const FemView& f, 
             for (int i = 0; i < 9; ++i) sh.part[base + g][i] = acc.v[i];
         }
     }
-    __syncthreads();
     if (t0 < n_slots) {
         slot_state_settle(st);
-        if (st.free != 0) solve_slot_from_lds(ps, st, sh.part, first_own, damping, dt);
+        sh.range[t0] = make_int2(st.first_inc - first_own, st.n_inc);
     }
+    __syncthreads();
+    sum_slots<kFusedThreads>(sh.part, sh.range, n_slots);
+    __syncthreads();
+    if (t0 < n_slots && st.free != 0) solve_slot_from_sum(ps, st, sh.part[st.first_inc - first_own], damping, dt);
 }
 
 template <int S, int Q>

@@ -315,20 +315,56 @@ __device__ __forceinline__ void vbd_local_solve(const Acc9& a, const dvec3& p, c
     }
 }
 
-// Sum of a slot's partials (part[j], j = its owners index - first_own, in
-// the owners order) and the local solve; writes the new position.
-__device__ __forceinline__ void solve_slot_from_lds(const PSView& ps, const SlotState& st, const float (*part)[9],
-                                                    int first_own, float damping, float dt) {
-    Acc9 acc;
-    acc_zero(acc);
-    for (int j = st.first_inc - first_own, e = j + st.n_inc; j < e; ++j) {
+// The sums of a block's slots, in place: slot s's partials part[range[s].x ..
+// range[s].x + range[s].y), in order, into its first row.  A thread takes one of
+// the nine values of one slot; one thread adding all nine of its slot, an
+// incidence after the other, was the longest stage of a pass (2 of 3.9 us in a
+// block of linear tetrahedra, whose vertices have some 24 incidences).  A
+// substep of the 64x16x16 beam P1 268 -> 211 us, Q1 628 -> 582, of the 16x4x4
+// quadratic one 573 -> 522, of the 32x8x8 Q2 one 1257 -> 1220.
+template <int THREADS>
+__device__ __forceinline__ void sum_slots(float (*part)[9], const int2* range, int n_slots) {
+    constexpr int N = 8;   // reads in flight
+    for (int t = threadIdx.x; t < 9 * n_slots; t += THREADS) {
+        const int s = t / 9, i = t - 9 * s;
+        const int2 r = range[s];
+        float sum = 0.f;
+        for (int j = 0; j < r.y; j += N) {
+            float x[N];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) acc.v[i] += part[j][i];
+            for (int k = 0; k < N; ++k) x[k] = part[r.x + min(j + k, r.y - 1)][i];
+#pragma unroll
+            for (int k = 0; k < N; ++k) sum += j + k < r.y ? x[k] : 0.f;
+        }
+        part[r.x][i] = sum;
     }
+}
+
+// The local solve of a slot whose partials are summed (sum); writes the new position.
+__device__ __forceinline__ void solve_slot_from_sum(const PSView& ps, const SlotState& st, const float (&sum)[9],
+                                                    float damping, float dt) {
+    Acc9 acc;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) acc.v[i] = sum[i];
     double dx[3];
     const dvec3 p = dunpack(st.p, ps.lo_unit);
     vbd_local_solve(acc, p, dunpack(st.last_p, ps.lo_unit), dunpack(st.y, ps.lo_unit), st.m, damping, dt, dx);
     gstore(ps.p, st.vid, dpack(dvec3{p.x + dx[0], p.y + dx[1], p.z + dx[2]}, ps.lo_inv));
+}
+
+// The same with one thread adding the slot's partials.  The P2 latency form keeps
+// it: its launches fill the chip, and two barriers and four waves' worth of sums
+// cost it more than the chain (64x16x16: 1.04 against 1.00 ms a substep).
+__device__ __forceinline__ void solve_slot_from_lds(const PSView& ps, const SlotState& st, const float (*part)[9],
+                                                    int first_own, float damping, float dt) {
+    float sum[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) sum[i] = 0.f;
+    for (int j = st.first_inc - first_own, e = j + st.n_inc; j < e; ++j) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) sum[i] += part[j][i];
+    }
+    solve_slot_from_sum(ps, st, sum, damping, dt);
 }
 
 // Phase 2 of the fused task kernels for one slot: add the slot's partials

@@ -324,6 +324,7 @@ __device__ __forceinline__ void q2_block(const PSView& ps, const FemView& fem, c
     __shared__ float part[LAT ? kQ2FusedIncPerBlockLat : kQ2FusedIncPerBlock][9];
     const int half = threadIdx.x >> 5;
     if constexpr (LAT) {
+        __shared__ int2 range[kQ2FusedMaxSlots];
         // the slot state rides along the element chain (a thread past the
         // block's slots loads the last one and does not use it; every vertex
         // block has a slot)
@@ -333,11 +334,14 @@ __device__ __forceinline__ void q2_block(const PSView& ps, const FemView& fem, c
         const LanePlan P = lane_plan(basis);
         q2_task_run(ps, fem, mt, P, own.own, blk.z, blk.w, half, sh[half], part,
                     [&] { slot_state_level1(own, ts, st); }, [&] { slot_state_level2(ps, y, st); });
-        __syncthreads();
         if (t < blk.y) {
             slot_state_settle(st);
-            if (st.free != 0) solve_slot_from_lds(ps, st, part, blk.z, damping, dt);
+            range[t] = make_int2(st.first_inc - blk.z, st.n_inc);
         }
+        __syncthreads();
+        sum_slots<kQ2FusedThreads>(part, range, blk.y);
+        __syncthreads();
+        if (t < blk.y && st.free != 0) solve_slot_from_sum(ps, st, part[st.first_inc - blk.z], damping, dt);
     } else {
         const int wave_first = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) & ~63);
         const LanePlan P = lane_plan(basis);
