@@ -655,7 +655,7 @@ def main():
                    "vertices": bat["vertices"], "vertex_updates_per_step": bat["vertex_updates_per_step"],
                    "gather_launches_per_step": bat["gather_launches_per_step"],
                    "batch_streams": args.batch_streams,
-                   "launch": "eager (value; with 2 batch streams the Q2 colour passes run beside the P2 ones); "
+                   "launch": "eager (value; with 2 batch streams groups of scenes run side by side); "
                              "roofline from a second run of as many steps with HIP events around every colour-pass "
                              "launch, all on one stream, for the kernel with the largest share of a step "
                              "(every colour-pass kernel in roofline_by_kernel)"},

@@ -115,10 +115,9 @@ oe_status oe_scene_set_graph(oe_scene* s, int32_t enable);
  * tasks - one per incidence of the colour, sum-factorised gradients for
  * 27-node hexahedra - then vertex solves).  Mode 1 is a VBD option.  On an
  * explicit scene mode 2 (the default) selects the element-centric force pass
- * (one element per 32 lanes, then a per-vertex sum of the element partials)
- * and mode 0 the per-vertex gather with this tile.  No counterpart in the reference,
- * whose kernels fix the thread layout per version
- * (src/GPU/VBD/GPU_VBD_FEM.cu:712-756). */
+ * (then a per-vertex sum of the element partials) and mode 0 the per-vertex
+ * gather with this tile.  No counterpart in the reference, whose kernels fix the
+ * thread layout per version (src/GPU/VBD/GPU_VBD_FEM.cu:712-756). */
 oe_status oe_scene_set_tile(oe_scene* s, int32_t lanes, int32_t qpl, int32_t mode);
 oe_status oe_scene_get_tile(oe_scene* s, int32_t* lanes, int32_t* qpl, int32_t* mode);
 /* The full colour-pass layout: the gather knobs above plus, for element

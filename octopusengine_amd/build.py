@@ -24,7 +24,8 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 CXX = shutil.which("g++") or "g++"
 
 COMMON = ["-O3", "-std=c++17", "-fPIC"]
-# Packed FP32 instructions are disabled for all device code.
+# Packed FP32 instructions are disabled for all device code.  A kernel's leading
+# scalar arguments (4 dwords) are preloaded into scalar registers.
 HIP_FLAGS = COMMON + [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                       "-fno-gpu-rdc", "-mllvm", "-amdgpu-kernarg-preload-count=4"]
 # Host-only geometry / graph code: no FMA contraction, so float expressions are

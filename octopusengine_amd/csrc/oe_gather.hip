@@ -317,7 +317,8 @@ __global__ __launch_bounds__(256) void k_batch_ju_refresh(BatchRefreshArgs b) {
 // ceil(incidences Q / L) work items per lane in turn, each loading and unpacking
 // all S nodes; here a lane loads S / LQ nodes, passes them to its group through
 // LDS, and runs one point.  Against the gather (the former default): a frame of
-// 4 steps of the 64x16x16 beam Q1 4.35 -> 2.72 ms, P1 1.24 -> 1.18 ms; 16 P3
+// 4 steps of the 64x16x16 beam Q1 4.35 -> 2.72 ms, P1 1.24 -> 1.18 ms (2.53 and
+// 0.94 with the slots' sums spread over the block, sum_slots); 16 P3
 // beams of 32x8x8 in a batch 22.6 -> 8.2 ms a step.  Against a thread per
 // incidence: a step of the quadratic 16x4x4 beam 721 -> 627 us.
 // A block takes a vertex block's incidences kFusedThreads / LQ at a time (more

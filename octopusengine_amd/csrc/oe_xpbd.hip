@@ -186,7 +186,7 @@ __device__ __forceinline__ void p1_project(const MaterialView& mt, float dt, con
 // read once and written once for its two constraints.  Bound by the launch and
 // the chain nodes -> positions -> ~450 instructions; reading the nodes again
 // for the second constraint, after an element id and an index load, it took
-// 5.9 us per colour.
+// 5.9 us per colour; with the first arguments preloaded 3.2 us.
 __global__ __launch_bounds__(64) void k_xpbd_p1(const int4* nodes, int first, int count, XpbdArgs a) {
     const int t = blockIdx.x * 64 + threadIdx.x;
     if (t >= count) return;
@@ -449,9 +449,13 @@ __device__ __forceinline__ void v2_project(const MaterialView& mt, float dt, con
 // never span waves, so no workgroup barrier is needed and the blocks spread
 // over the chip).  Bound by one wave's chain: launch 1.6 us, three dependent
 // loads, then about 950 instructions (27 nodes).  A frame of 50 substeps of the
-// 32 x 8 x 8 beams: 27-node hexahedra 4.84 -> 3.05 ms (227 elements per
-// colour), 20-node tetrahedra 10.16 -> 7.45 ms (424 per colour), against
+// 32 x 8 x 8 beams: 27-node hexahedra 4.84 -> 2.76 ms (227 elements per
+// colour), 20-node tetrahedra 10.16 -> 7.25 ms (424 per colour), against
 // 256-thread blocks with workgroup barriers, rolled sums and 4-byte LDS reads.
+// The arguments the chain starts with come first and are preloaded into scalar
+// registers; the node ids lie in colour order, so they do not wait for the
+// element id, and the positions are issued before the dN table (P2 64x16x16,
+// 3,300 elements per colour: 161 -> 147 us a substep).
 template <int S, int Q, bool NARROW>
 __global__ __launch_bounds__(64) void k_xpbd_v2(const int* topo, int first, int count, XpbdArgs a) {
     using P_ = V2Plan<S, Q, NARROW>;
