@@ -309,6 +309,10 @@ void build_vertex_blocks(const OwnersCSR& o, int max_inc, int max_slots, std::ve
         };
         for (int s = o.color_begin[c]; s < o.color_begin[c + 1]; ++s) {
             const int nb = o.slot_nb[s];
+            if (nb == 0) {   // no partials to add and no row for their sum
+                flush();
+                continue;
+            }
             if (nb > max_inc)
                 throw std::invalid_argument("a vertex has " + std::to_string(nb) + " incident elements, more than the " +
                                             std::to_string(max_inc) + " of a fused task block");

@@ -147,7 +147,10 @@ OwnersCSR build_owners(const HostMesh& m, const Coloration& col, bool by_valence
 // total, 4 ints per block {first slot, slot count, first owners index,
 // incidence count}, colour-major; color_begin[c] = first block of colour c.
 // Throws std::invalid_argument when one vertex alone has more than max_inc
-// incidences.
+// incidences.  A vertex that no element uses is in no block, so a block has no
+// more slots than incidences: with no energy its local problem is solved by the
+// inertia target, where the predictor put it, and what a constraint made of it
+// a new solve and the constraint would only make again.
 void build_vertex_blocks(const OwnersCSR& o, int max_inc, int max_slots, std::vector<int32_t>& blocks,
                          std::vector<int32_t>& color_begin);
 
