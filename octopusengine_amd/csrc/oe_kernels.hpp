@@ -118,11 +118,14 @@ __device__ __forceinline__ float lanes_sum(float x) {
 }
 // Sum over the lanes that are a multiple of W apart inside aligned groups of
 // L lanes (4 <= W <= L): rotations inside a row, then across rows and halves.
+// Each step adds two values that both partners hold, the half row first, so
+// every lane ends with the same bits; with the quarter first, neighbouring
+// parts would add their four values in two orders.
 template <int W, int L>
 __device__ __forceinline__ float parts_sum(float x) {
     static_assert(W >= 4 && W <= L && L <= 64 && (W == L || L >= 16), "parts of 4 lanes and more, whole rows");
-    if constexpr (W <= 4 && L >= 16) x = dpp_add<0x124>(x);   // row_ror:4
     if constexpr (W <= 8 && L >= 16) x = dpp_add<0x128>(x);   // row_ror:8
+    if constexpr (W <= 4 && L >= 16) x = dpp_add<0x124>(x);   // row_ror:4
     if constexpr (W <= 16 && L >= 32) x = row_pair_add(x);
     if constexpr (W <= 32 && L >= 64) x = half_pair_add(x);
     return x;
