@@ -227,13 +227,15 @@ __device__ __forceinline__ void block_lds_sync() {
 // A run of substeps of a small linear-tetrahedron scene in one workgroup.  A
 // colour of such a scene is a wave or a few of work (59 elements on the
 // 16x4x4 beam), and a substep has ~28 of them: as launches the frame is the
-// launches.  Here the positions stay in LDS (xyz and the inverse mass, its
-// sign set on masked vertices), a colour boundary is a workgroup barrier, and
-// the next colour's element is loaded while the current one computes.  One
-// compute unit does all the work, so the form is for scenes whose positions fit
-// LDS (kXpbdResidentVertices), where a colour is at most ~6 waves.  The
-// arithmetic is that of k_xpbd_p1 and the vertex passes, in their order.
+// launches.  Here the positions stay in LDS (xyz and the inverse mass, its sign
+// bit set on masked vertices: the zero of an infinite mass has one too), a colour
+// boundary is a workgroup barrier, and the next colour's element is loaded while
+// the current one computes.  One compute unit does all the work, so the form is
+// for scenes whose positions fit LDS (kXpbdResidentVertices), where a colour is
+// at most ~6 waves.  The arithmetic is that of k_xpbd_p1 and the vertex passes, in
+// their order.
 constexpr int kXpbdResidentThreads = 512;
+__device__ __forceinline__ bool unmasked(float w) { return __float_as_int(w) >= 0; }
 __global__ __launch_bounds__(kXpbdResidentThreads) void k_xpbd_p1_resident(XpbdResidentArgs a) {
     constexpr int T = kXpbdResidentThreads;
     __shared__ float4 pos[kXpbdResidentVertices];
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(kXpbdResidentThreads) void k_xpbd_p1_resident(XpbdR
                     x[k][2] = u.z;
                     ws[k] = u.w;
                     w[k] = fabsf(u.w);
-                    free[k] = u.w > 0.f;
+                    free[k] = unmasked(u.w);
                 }
                 p1_project(a.mt, a.dt, el, w, free, x);
 #pragma unroll
@@ -306,7 +308,7 @@ __global__ __launch_bounds__(kXpbdResidentThreads) void k_xpbd_p1_resident(XpbdR
             if (a.c.fixed || a.c.has_box) {
                 const bool is_fixed = a.c.fixed && gload(a.c.fixed, i) != 0;
                 const float4 X = gload(static_cast<const float4*>(a.ps.init_p), i);
-                constrain(a.ps, i, p, is_fixed, q.w > 0.f ? 1 : 0, X, a.c.t.com, a.c.t.offset, a.c.t.R, a.c.has_box,
+                constrain(a.ps, i, p, is_fixed, unmasked(q.w) ? 1 : 0, X, a.c.t.com, a.c.t.offset, a.c.t.R, a.c.has_box,
                           a.c.lo, a.c.hi);
                 if (is_fixed) ws = -w;
             }
