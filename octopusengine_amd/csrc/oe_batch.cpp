@@ -29,6 +29,10 @@ std::map<int, GatherTile> default_tiles() {
     return t;
 }
 
+bool needs_gather(const Scene& s) {
+    return s.mesh.element != Tetra10 && s.mesh.element != Hexa27 && !s.vbd_fem->fits_tasks();
+}
+
 // A batch's launches are a server's (default_tile) or much longer, and run
 // beside one another.
 //  * Q2 blocks of 28 incidences from kLongBlocks of them per colour pass on (2 a
@@ -45,9 +49,11 @@ std::map<int, GatherTile> batch_tiles(const std::vector<Scene*>& scenes) {
     constexpr double kLongBlocks = 2048;
     std::map<int, GatherTile> t = default_tiles();
     double per_pass = 0.0;
-    for (const Scene* s : scenes)
+    for (const Scene* s : scenes) {
+        if (needs_gather(*s)) t[s->mesh.element].mode = PASS_GATHER;
         if (s->mesh.element == Hexa27)
             per_pass += 27.0 * s->fem->E / std::max(1, s->vbd_fem->nb_colors());
+    }
     if (per_pass >= kLongBlocks * kQ2PencilIncPerBlock) t[Hexa27].inc = kQ2PencilIncPerBlock;
     else t[Hexa27].lat_blocks = 1024;
     t[Tetra10].lat_blocks = 256;

@@ -108,6 +108,11 @@ void launch_schedule(const Schedule& sch, const DeviceSchedule& dev, const Scene
 // ticks start with, and what a batch of these scenes starts with.
 std::map<int, GatherTile> default_tiles();
 std::map<int, GatherTile> batch_tiles(const std::vector<Scene*>& scenes);
+// Whether default layouts that are to hold s take its element type to the
+// gather: a vertex of more elements than a task block holds, of the types that
+// fall back (linear tetrahedra, 8-node hexahedra, 20-node tetrahedra) as the
+// scene by itself does.  The other two are refused with such a vertex.
+bool needs_gather(const Scene& s);
 
 // A batch registers itself with its scenes (Scene::batches).  A scene may be
 // in several batches but appear once per batch, and a scene held by a server

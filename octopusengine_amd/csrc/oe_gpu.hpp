@@ -268,6 +268,8 @@ struct GPU_VBD_FEM final : GPU_FEM {
     // time for the types that have no other form; 0 = the kernel's maximum)
     int fit_inc(int inc) const;
     int max_incidences = 0;   // most incident elements of one vertex
+    // every vertex fits a task block of the kernel's maximum
+    bool fits_tasks() const { return max_incidences <= max_task_inc(element); }
     // The tables already built for `inc` (std::logic_error if not): for
     // step(), which may run under HIP graph capture and must not allocate.
     const TaskTables& built_tables(int inc) const;

@@ -51,7 +51,11 @@ int Server::add_scene(Scene* s) {
     idle_cv_.wait(lk, [&] { return (inflight_.empty() && launching_ == 0) || !error_.empty(); });
     if (!error_.empty()) throw std::runtime_error(error_);
     flags_.emplace_back(&eng_->pool, fixed_flags(*s));
-    host_table_.push_back(make_scene_dev(*s, flags_.back().get(), tiles_));
+    std::map<int, GatherTile> tiles = tiles_;
+    // the scenes already held can run the gather too: their entries hold what it reads
+    if (!told_.count(s->mesh.element) && needs_gather(*s)) tiles[s->mesh.element].mode = PASS_GATHER;
+    host_table_.push_back(make_scene_dev(*s, flags_.back().get(), tiles));
+    tiles_ = std::move(tiles);
     scenes_.push_back(s);
     scene_busy_.push_back(0);
     slot_open_.push_back(0);
@@ -106,6 +110,7 @@ void Server::set_tile(Element e, GatherTile t) {
         if (scenes_[i] && scenes_[i]->mesh.element == e)
             changed.emplace_back(i, make_scene_dev(*scenes_[i], flags_[i].get(), tiles));
     tiles_ = std::move(tiles);
+    told_.insert(e);
     for (const auto& c : changed) host_table_[c.first] = c.second;
     table_uploaded_ = 0;
     grow_table();

@@ -30,6 +30,7 @@
 #include <condition_variable>
 #include <deque>
 #include <mutex>
+#include <set>
 #include <thread>
 #include <unordered_set>
 #include <vector>
@@ -99,6 +100,7 @@ private:
     DBuf<SceneDev> table_;
     size_t table_uploaded_ = 0;
     std::map<int, GatherTile> tiles_;
+    std::set<int> told_;   // element types whose layout set_tile chose
     std::vector<StreamSlot> slots_;
     std::vector<char> scene_busy_;
     std::vector<int64_t> slot_open_;           // submitted and not yet completed, per slot
