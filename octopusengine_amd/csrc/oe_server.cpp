@@ -50,17 +50,31 @@ int Server::add_scene(Scene* s) {
     // the device table is reallocated only while nothing is in flight
     idle_cv_.wait(lk, [&] { return (inflight_.empty() && launching_ == 0) || !error_.empty(); });
     if (!error_.empty()) throw std::runtime_error(error_);
-    flags_.emplace_back(&eng_->pool, fixed_flags(*s));
+    DBuf<unsigned char> flags(&eng_->pool, fixed_flags(*s));
     std::map<int, GatherTile> tiles = tiles_;
     // the scenes already held can run the gather too: their entries hold what it reads
     if (!told_.count(s->mesh.element) && needs_gather(*s)) tiles[s->mesh.element].mode = PASS_GATHER;
-    host_table_.push_back(make_scene_dev(*s, flags_.back().get(), tiles));
+    const SceneDev dev = make_scene_dev(*s, flags.get(), tiles);
+    // a refused scene, or one the table has no memory for, leaves every list as it was
+    const size_t n = scenes_.size();
+    try {
+        flags_.push_back(std::move(flags));
+        host_table_.push_back(dev);
+        scenes_.push_back(s);
+        scene_busy_.push_back(0);
+        slot_open_.push_back(0);
+        grow_table();
+    } catch (...) {
+        flags_.resize(n);
+        host_table_.resize(n);
+        scenes_.resize(n);
+        scene_busy_.resize(n);
+        slot_open_.resize(n);
+        table_uploaded_ = std::min(table_uploaded_, n);
+        throw;
+    }
     tiles_ = std::move(tiles);
-    scenes_.push_back(s);
-    scene_busy_.push_back(0);
-    slot_open_.push_back(0);
-    grow_table();
-    const int slot = static_cast<int>(scenes_.size()) - 1;
+    const int slot = static_cast<int>(n);
     s->server = this;
     s->server_slot = slot;
     return slot;

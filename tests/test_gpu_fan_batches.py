@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import octopusengine_amd as oe
-from meshes import hex_book, tet_fan
+from meshes import hex_book, p1_to_p2, tet_fan
 from scenes import max_err
 
 pytestmark = pytest.mark.gpu
@@ -84,3 +84,38 @@ def test_server_keeps_a_layout_it_was_told(engine):
     s.step(0.005, 1)   # still its own
     srv.close()
     s.close()
+
+
+def test_a_refused_scene_leaves_the_server_as_it_was(engine):
+    """A quadratic fan is refused; scenes added after it keep their own fixed
+    vertices when the layout is set anew."""
+    cells = (6, 2, 2)
+    fixings = [((1e-6, 0.0, 0.0), (-1.0, 0.0, 0.0)), ((1.0 - 1e-6, 0.0, 0.0), (1.0, 0.0, 0.0))]
+
+    def beam(fix):
+        s = oe.make_scene(engine, oe.TETRA10, cells, young=1e5, poisson=0.45, fix_x0=False)
+        s.fix_plane(*fix)
+        return s
+    held, alone = ([beam(f) for f in fixings] for _ in range(2))
+    refused = oe.Scene(engine, oe.TETRA10, *p1_to_p2(*tet_fan(300)), iterations=2)
+    srv = oe.Server(engine, max_batch=4, streams=1)
+    slots = [srv.add_scene(held[0])]
+    with pytest.raises(oe.OEError):
+        srv.add_scene(refused)
+    slots.append(srv.add_scene(held[1]))
+    assert slots == [0, 1]
+    t = srv.get_tile_ex(oe.TETRA10)
+    srv.set_tile_ex(oe.TETRA10, t["lanes"], t["qpl"], t["mode"], t["inc_per_block"], t["latency_blocks"])
+    for _ in range(2):
+        for k in slots:
+            srv.submit(k, 0.005, 1)
+        srv.drain()
+        for s in alone:
+            s.step(0.005, 1)
+    for x, y in zip(held, alone):
+        assert np.array_equal(x.masks(), y.masks())
+        assert max_err(x.positions(), y.positions()) <= 1e-6
+    refused.step(0.005, 1)
+    srv.close()
+    for s in held + alone + [refused]:
+        s.close()
