@@ -120,6 +120,16 @@ std::vector<bool> latency_pattern(GPU_VBD_FEM& f, const GatherTile& t) {
     return pat;
 }
 
+// the same colour passes of an element type in a batch
+bool same_passes(Element el, const GatherTile& a, const GatherTile& b) {
+    if (a.mode != b.mode) return false;
+    if (a.mode != PASS_TASKS) return a.L == b.L && a.QL == b.QL;
+    auto inc = [&](const GatherTile& t) {
+        return t.inc > 0 ? t.inc : el == Hexa27 ? kQ2FusedIncPerBlock : max_task_inc(el);
+    };
+    return inc(a) == inc(b) && a.lat_blocks == b.lat_blocks;
+}
+
 void release_unused(GPU_VBD_FEM& f) {
     if (!f.cached()) f.ju.reset();
     const int keep = f.tasks() ? f.fit_inc(f.tile.inc) : -1;
@@ -326,9 +336,14 @@ std::vector<TuneRecord> autotune_batch(Batch& b, bool force) {
     try {
         for (int el : to_time) {
             std::vector<GatherTile> cands;
-            // batches run the throughput form only: one threshold per block size
+            // one threshold per block size, and the layout that the batch started with, whose
+            // threshold may be another: tuning picks nothing that it timed slower than that
             for (const GatherTile& t : tile_candidates(static_cast<Element>(el), true, tasks_ok[el]))
                 if (t.mode != PASS_TASKS || t.lat_blocks == kLatencyBlocks) cands.push_back(t);
+            const GatherTile start = batch_tiles(b.scenes).at(el);
+            if (std::none_of(cands.begin(), cands.end(),
+                             [&](const GatherTile& t) { return same_passes(static_cast<Element>(el), t, start); }))
+                cands.push_back(start);
             auto run = [&](const GatherTile& t, int reps) -> double {
                 try {
                     b.set_tile(static_cast<Element>(el), t);
