@@ -524,10 +524,11 @@ bool launch_xpbd(int S, int Q, bool v0_form, const XpbdArgs& a, hipStream_t s) {
         return false;
     }
     if (S == 8 && Q == 8) {
-        // 32 lanes per element up to two waves per SIMD (4,096 elements), 8 past
-        // that: a substep of the 64x16x16 beam (2,048 elements per colour) takes
-        // 51.9 us with 32 lanes and 62 with 8, of 128x32x32 (16,384) 118 and 78
-        if (a.count <= 1024) launch_v2<8, 8>(a, s);
+        // 32 lanes per element up to one wave per SIMD (2,048 elements), 8 past
+        // that.  A substep (the ten colours and the vertex pass) with 32 and with
+        // 8 lanes: largest colour 2,047 elements (64x16x16 beam) 45.2 and 45.7 us,
+        // 2,303 (72x16x16) 49.3 and 46.7, 4,095 51.9 and 47.7, 8,191 68.4 and 52.2
+        if (a.count <= 2048) launch_v2<8, 8>(a, s);
         else launch_v2<8, 8, true>(a, s);
         return true;
     }
