@@ -27,7 +27,6 @@
 // on the command line) so that the template instances build in parallel.
 #include <cmath>
 #include <stdexcept>
-#include <type_traits>
 
 #include "oe_gather.hpp"
 #include "oe_host.hpp"
@@ -511,28 +510,6 @@ __global__ __launch_bounds__(kFusedThreads) void k_batch_point_tasks(BatchFusedA
 }
 
 #if OE_GATHER_S == 10   // one thread per incidence: quadratic tetrahedra in larger launches
-// The Jx contraction reads the shape-derivative table from device memory, except
-// for quadratic tetrahedra, whose gradients follow from two scalars (P2Factors).
-template <int S, class Grad>
-__device__ __forceinline__ void jx_from_grad(const float (&xs)[S][3], const Grad& grad, int base, float Jx[9]) {
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Jx[i] = 0.f;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-        const float d0 = grad.at(base + 3 * k), d1 = grad.at(base + 3 * k + 1), d2 = grad.at(base + 3 * k + 2);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            Jx[0 + c] = fmaf(xs[k][c], d0, Jx[0 + c]);
-            Jx[3 + c] = fmaf(xs[k][c], d1, Jx[3 + c]);
-            Jx[6 + c] = fmaf(xs[k][c], d2, Jx[6 + c]);
-        }
-    }
-}
-struct GradInMemory {
-    const float* dN;
-    __device__ __forceinline__ float at(int i) const { return gload(dN, i); }
-};
-
 // Quadratic tetrahedra.  With M_ii the corner and M_ij the edge values, u =
 // sum_i l_i (2 l_i - 1) M_ii + 4 sum_{i<j} l_i l_j M_ij in the barycentric
 // coordinates l, so the derivative along xi_c (l_c against l_0) is
@@ -572,41 +549,20 @@ struct P2Gradients {
             for (int k = 0; k < 3; ++k) Jx[3 * c + k] = fmaf(f.k4, E[c][corner][k], base[3 * c + k]);
     }
 };
-// what a fused kernel takes besides its arguments: the P2 factors, or nothing
-struct NoFactors {};
-template <int S>
-using ShapeArg = std::conditional_t<S == 10, P2Factors, NoFactors>;
-
-// In the throughput form of the fused blocks, shape-derivative tables of at
-// most kDnLdsFloats floats (P1, P2, Q1) are copied to LDS, one copy per wave,
-// at the start of a block: a lane's dN_r at each point is then an LDS read,
-// not a device-memory load that the point loop waits on (P2 batch: 84.9
-// against 89.1 us per colour pass).  The latency form keeps the loads: it
-// issues the vertex state's loads first, and vector-memory loads complete in
-// order, so the copy's LDS write would wait for them (single P2 scene: 1.22
-// against 1.19 ms per step).
-constexpr int kDnLdsFloats = 256;
-template <int S, int Q, bool LAT>
-constexpr bool dn_in_lds() { return !LAT && S * Q * 3 <= kDnLdsFloats; }
-template <int S, int Q, bool LAT>
-constexpr int dn_lds_size() { return dn_in_lds<S, Q, LAT>() ? S * Q * 3 : 1; }
-
+// In the throughput form the shape-derivative table is copied to LDS, one copy
+// per wave, at the start of a block: a lane's dN_r at each point is then an LDS
+// read, not a device-memory load that the point loop waits on (batch: 84.9
+// against 89.1 us per colour pass).  The latency form keeps the loads: it issues
+// the vertex state's loads first, and vector-memory loads complete in order, so
+// the copy's LDS write would wait for them (single scene: 1.22 against 1.19 ms
+// per step).
 template <int S, int Q, bool DNL>
-__device__ __forceinline__ void dnr_at(const FemView& f, const float* dnw, int q, int r, float dnr[3]) {
-    if constexpr (DNL) {
-        const float* d = dnw + (q * S + r) * 3;
-        dnr[0] = d[0];
-        dnr[1] = d[1];
-        dnr[2] = d[2];
-    } else {
-        load_dnr(f.dN, (q * S + r) * 3, dnr);
-    }
-}
+constexpr int dn_lds_size() { return DNL ? S * Q * 3 : 1; }
 
 // Partial (force, Hessian) of local node r of element eid over its Q points.
 // dnw: the wave's LDS copy of the shape-derivative table (DNL only).
 template <int S, int Q, bool DNL>
-__device__ __forceinline__ void elem_partial(const FemView& f, const MaterialView& mt, const ShapeArg<S>& shape,
+__device__ __forceinline__ void elem_partial(const FemView& f, const MaterialView& mt, const P2Factors& shape,
                                              int eid, int r, const float (&xs)[S][3], const float* dnw, Acc9& acc) {
     acc_zero(acc);
     // affine: one record per element, JX_inv and |det B|, V_q = |det B| w_q
@@ -616,43 +572,33 @@ __device__ __forceinline__ void elem_partial(const FemView& f, const MaterialVie
         for (int i = 0; i < 9; ++i) JXi[i] = gload(f.jxv, static_cast<size_t>(eid) * 10 + i);
         detB = gload(f.jxv, static_cast<size_t>(eid) * 10 + 9);
     }
-    float Ju[9], V = 0.f;
-    if constexpr (S == 10) {
-        // dN_r at the four points: issued here with the record's loads when it
-        // comes from memory (in the point loop each would be waited for)
-        float dnr[Q][3];
-        if constexpr (!DNL) {
+    // dN_r at the four points: issued here with the record's loads when it
+    // comes from memory (in the point loop each would be waited for)
+    float dnr[Q][3];
+    if constexpr (!DNL) {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) load_dnr(f.dN, (q * S + r) * 3, dnr[q]);
-        }
-        V = detB * gload(f.wq, 0);   // the rule's four weights are equal (shape_arg)
-        P2Gradients g;
-        g.init(xs, shape);
+        for (int q = 0; q < Q; ++q) load_dnr(f.dN, (q * S + r) * 3, dnr[q]);
+    }
+    float Ju[9], V = detB * gload(f.wq, 0);   // the rule's four weights are equal (shape_arg)
+    P2Gradients g;
+    g.init(xs, shape);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            g.at(kP2Corner[q], shape, Ju);
-            if constexpr (DNL) dnr_at<S, Q, DNL>(f, dnw, q, r, dnr[q]);
-            if (!f.affine) load_element_record(f, eid, q, JXi, V);
-            nh_contrib(Ju, JXi, V, dnr[q], mt, acc);
-            acc_settle(acc);   // or the four points' sums are formed together at the end (138 VGPRs, 3 waves)
+    for (int q = 0; q < Q; ++q) {
+        g.at(kP2Corner[q], shape, Ju);
+        if constexpr (DNL) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) dnr[q][c] = dnw[(q * S + r) * 3 + c];
         }
-    } else {
-#pragma unroll 1
-        for (int q = 0; q < Q; ++q) {
-            float dnr[3];
-            jx_from_grad<S>(xs, GradInMemory{f.dN}, q * S * 3, Ju);
-            dnr_at<S, Q, DNL>(f, dnw, q, r, dnr);
-            if (f.affine) V = detB * gload(f.wq, q);
-            else load_element_record(f, eid, q, JXi, V);
-            nh_contrib(Ju, JXi, V, dnr, mt, acc);
-        }
+        if (!f.affine) load_element_record(f, eid, q, JXi, V);
+        nh_contrib(Ju, JXi, V, dnr[q], mt, acc);
+        acc_settle(acc);   // or the four points' sums are formed together at the end (138 VGPRs, 3 waves)
     }
 }
 
 // Phase 1 of a fused block: the partials of the block's incidences into LDS.
 template <int S, int Q, bool DNL>
 __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f, const OwnersView& own,
-                                             const MaterialView& mt, const ShapeArg<S>& grad, const int4 blk,
+                                             const MaterialView& mt, const P2Factors& shape, const int4 blk,
                                              float (*part)[9], float* dnw) {
     const int first_own = blk.z, n_inc = blk.w;
     const int t0 = threadIdx.x;
@@ -691,7 +637,7 @@ __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f,
         for (int k = 0; k < S; ++k) rel_node(h[k], h[0], ps.lo_unit, xs[k]);
         const int eid = pk >> 5, r = pk & 31;
         Acc9 acc;
-        elem_partial<S, Q, DNL>(f, mt, grad, eid, r, xs, dnw, acc);
+        elem_partial<S, Q, DNL>(f, mt, shape, eid, r, xs, dnw, acc);
 #pragma unroll
         for (int i = 0; i < 9; ++i) part[t][i] = acc.v[i];
     }
@@ -709,7 +655,7 @@ __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f,
 // batch pass on one GPU.)
 template <int S, int Q, class AfterOwner, class AfterTopo>
 __device__ __forceinline__ void fused_phase1_lat(const PSView& ps, const FemView& f, const OwnersView& own,
-                                                 const MaterialView& mt, const ShapeArg<S>& grad, const int4 blk,
+                                                 const MaterialView& mt, const P2Factors& shape, const int4 blk,
                                                  float (*part)[9], AfterOwner&& after_owner, AfterTopo&& after_topo) {
     static_assert(kFusedRuns == 1, "one incidence per thread");
     const int first_own = blk.z, n_inc = blk.w;
@@ -731,7 +677,7 @@ __device__ __forceinline__ void fused_phase1_lat(const PSView& ps, const FemView
     for (int k = 0; k < S; ++k) rel_node(h[k], h[0], ps.lo_unit, xs[k]);
     const int eid = pk >> 5, r = pk & 31;
     Acc9 acc;
-    elem_partial<S, Q, false>(f, mt, grad, eid, r, xs, nullptr, acc);
+    elem_partial<S, Q, false>(f, mt, shape, eid, r, xs, nullptr, acc);
     if (has) {
 #pragma unroll
         for (int i = 0; i < 9; ++i) part[t0][i] = acc.v[i];
@@ -740,7 +686,7 @@ __device__ __forceinline__ void fused_phase1_lat(const PSView& ps, const FemView
 
 template <int S, int Q, bool LAT>
 __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, const OwnersView& own,
-                                            const MaterialView& mt, const ShapeArg<S>& grad, const float4* y,
+                                            const MaterialView& mt, const P2Factors& shape, const float4* y,
                                             float damping, float dt, const int4 blk, float (*part)[9], float* dnw) {
     const int first_slot = blk.x, n_slots = blk.y, first_own = blk.z;
     const int t0 = threadIdx.x;
@@ -750,7 +696,7 @@ __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, 
         // block has a slot)
         SlotState st{};
         const int ts = first_slot + min(t0, n_slots - 1);
-        fused_phase1_lat<S, Q>(ps, f, own, mt, grad, blk, part, [&] { slot_state_level1(own, ts, st); },
+        fused_phase1_lat<S, Q>(ps, f, own, mt, shape, blk, part, [&] { slot_state_level1(own, ts, st); },
                                [&] { slot_state_level2(ps, y, st); });
         __syncthreads();
         if (t0 < n_slots) {
@@ -764,7 +710,7 @@ __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, 
         const int ts = first_slot + min(t0, n_slots - 1);
         const int slot_vid = gload(own.slot_vid, ts);
         const int2 slot_nbo = gload(own.slot_nbo, ts);
-        fused_phase1<S, Q, dn_in_lds<S, Q, LAT>()>(ps, f, own, mt, grad, blk, part, dnw);
+        fused_phase1<S, Q, !LAT>(ps, f, own, mt, shape, blk, part, dnw);
         __syncthreads();
         // phase 2: one thread per slot, partials in the owners order, local solve
         if (t0 >= n_slots) return;
@@ -774,18 +720,18 @@ __device__ __forceinline__ void fused_block(const PSView& ps, const FemView& f, 
 
 template <int S, int Q, bool LAT>
 __global__ __launch_bounds__(kFusedThreads) void k_fused_tasks(const int4* blocks, int first, int count,
-                                                               FusedTaskArgs a, ShapeArg<S> g) {
+                                                               FusedTaskArgs a, P2Factors g) {
     __shared__ float part[LAT ? kFusedIncPerBlockLat : kFusedIncPerBlock][9];
-    __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, LAT>()];
+    __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, !LAT>()];
     const int4 blk = gload(blocks, first + xcd_block(blockIdx.x, count));
     fused_block<S, Q, LAT>(a.ps, a.fem, a.own, a.mt, g, a.y, a.damping, a.dt, blk, part,
                               dn_lds[threadIdx.x >> 6]);
 }
 
 template <int S, int Q, bool LAT>
-__global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedArgs b, ShapeArg<S> g) {
+__global__ __launch_bounds__(kFusedThreads) void k_batch_fused_tasks(BatchFusedArgs b, P2Factors g) {
     __shared__ float part[LAT ? kFusedIncPerBlockLat : kFusedIncPerBlock][9];
-    __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, LAT>()];
+    __shared__ float dn_lds[kFusedThreads / 64][dn_lds_size<S, Q, !LAT>()];
     const int bid = xcd_block(blockIdx.x, gridDim.x);
     const BatchSeg seg = find_seg(b.segs, b.seg_first, b.seg_count, bid);
     const SceneDev& sd = b.scenes[seg.scene];
@@ -1061,10 +1007,10 @@ int OE_FN(refresh_elements_per_block_)() { return refresh_epb<OE_GATHER_Q>(); }
 namespace {
 // The P2 factors from the element's quadrature points, checked against its
 // shape-derivative table (to float rounding: the reference's points are floats
-// whose coordinates add to 1 within an ulp).  Nothing for the other types.
-const ShapeArg<OE_GATHER_S>& shape_arg() {
-    static const ShapeArg<OE_GATHER_S> g = [] {
-        ShapeArg<OE_GATHER_S> t{};
+// whose coordinates add to 1 within an ulp).
+const P2Factors& shape_arg() {
+    static const P2Factors g = [] {
+        P2Factors t{};
         const ShapeTable& st = shape_table(Tetra10);
         const double b = st.qpoints[0], a = (1.0 - b) / 3.0;
         for (int q = 0; q < 4; ++q)
