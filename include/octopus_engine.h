@@ -207,8 +207,10 @@ oe_status oe_batch_set_graph(oe_batch* b, int32_t enable);
 oe_status oe_batch_set_streams(oe_batch* b, int32_t n);
 oe_status oe_batch_set_tile(oe_batch* b, int32_t element, int32_t lanes, int32_t qpl, int32_t mode);
 /* Full layout per element type; latency_blocks applies to a colour pass over all
- * scenes of the type.  A batch starts with the scenes' defaults but longer Q2
- * blocks where its passes fill the GPU; get returns the layout in use. */
+ * scenes of the type.  A batch starts with the scenes' defaults (the gather for
+ * linear tetrahedra, 8-node hexahedra and 20-node tetrahedra when a vertex of one
+ * of their scenes has more elements than a task block holds) but longer Q2 blocks
+ * where its passes fill the GPU; get returns the layout in use. */
 oe_status oe_batch_set_tile_ex(oe_batch* b, int32_t element, const oe_tile* t);
 oe_status oe_batch_get_tile_ex(oe_batch* b, int32_t element, oe_tile* t);
 /* Autotune every element type of the batch: the candidates are timed on the
@@ -251,7 +253,9 @@ oe_status oe_server_destroy(oe_server* sv);
  * oe_scene_destroy waits for them and releases the slot. */
 oe_status oe_server_add_scene(oe_server* sv, oe_scene* s, int32_t* slot);
 /* Layout of one element type's colour passes in every tick (default: the
- * scene defaults, with 14 incidences per block for 27-node hexahedra).
+ * scene defaults, with 14 incidences per block for 27-node hexahedra; until a
+ * layout is set, a scene with a vertex of more elements than a task block holds
+ * takes its type to the gather, as in a batch).
  * Refused (OE_ERR_STATE) while requests are pending or in flight; get returns
  * the layout in use.  No counterpart in the reference. */
 oe_status oe_server_set_tile_ex(oe_server* sv, int32_t element, const oe_tile* t);

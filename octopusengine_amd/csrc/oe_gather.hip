@@ -304,9 +304,8 @@ __global__ __launch_bounds__(256) void k_batch_ju_refresh(BatchRefreshArgs b) {
 }
 
 #if OE_GATHER_S != 27   // 27-node hexahedra have their own task kernels
-// Fused element tasks (see FusedTaskArgs).  Phase 1: thread t of the block
-// takes the incidences t, t + kFusedThreads, ... of the vertex block.  Fixed
-// vertices are not skipped there: phase 2 skips them.
+// Element tasks (see FusedTaskArgs).  Fixed vertices' incidences are not skipped:
+// their solves are.
 //
 // Point tasks: the task form with an incidence's points spread over LQ lanes
 // (LQ PPL >= Q), for linear tetrahedra (1 lane), 8-node hexahedra (8), 20-node
@@ -596,6 +595,7 @@ __device__ __forceinline__ void elem_partial(const FemView& f, const MaterialVie
 }
 
 // Phase 1 of a fused block: the partials of the block's incidences into LDS.
+// Thread t takes the incidences t, t + kFusedThreads, ... of the vertex block.
 template <int S, int Q, bool DNL>
 __device__ __forceinline__ void fused_phase1(const PSView& ps, const FemView& f, const OwnersView& own,
                                              const MaterialView& mt, const P2Factors& shape, const int4 blk,

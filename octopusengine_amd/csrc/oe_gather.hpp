@@ -88,13 +88,14 @@ struct BatchGatherArgs {
 // count, first owners index, incidence count}) whose incidences fit
 // kFusedIncPerBlock.  Its threads first take the incidences (element e, local
 // node r) and put the force / Hessian partial of node r over the points of e in
-// LDS; then one thread per slot adds its vertex's partials in the owners order
-// and runs the local solve.  Quadratic tetrahedra have three forms, each with
+// LDS; then a slot's partials are added in the owners order and one thread per
+// slot runs the local solve.  Quadratic tetrahedra have three forms, each with
 // vertex blocks of its own:
-//   throughput  one thread per incidence;
+//   throughput  one thread per incidence, and one adds a slot's partials;
 //   latency     the same, the vertex state loaded along the element chain, for
 //               launches too small to fill the GPU;
-//   split       point tasks, a lane per point, for launches smaller still.
+//   split       point tasks, a lane per point, the sums spread over the block
+//               (sum_slots), for launches smaller still.
 // The other types have point tasks only (oe_gather.hip, k_point_tasks).
 enum TaskForm : int { TASKS_THROUGHPUT = 0, TASKS_LATENCY = 1, TASKS_SPLIT = 2 };
 constexpr int kFusedThreads = 256;

@@ -254,8 +254,9 @@ struct GPU_VBD_FEM final : GPU_FEM {
     // (incidences per block), built on first use and kept while the scene
     // lives: batches and servers hold pointers into them.
     std::map<int, TaskTables> thr_tables;
-    // Vertex blocks of the kernels' latency form (one task per thread or
-    // half-wave); empty when a vertex has more incidences than one holds.
+    // Quadratic elements: vertex blocks of the kernels' latency form (one task
+    // per thread or half-wave); empty when a vertex has more incidences than one
+    // holds.
     TaskTables lat_tables;
     bool lat_built = false;
     TaskTables split_tables;   // quadratic tetrahedra: vertex blocks of the point-task form
@@ -273,7 +274,7 @@ struct GPU_VBD_FEM final : GPU_FEM {
     // The tables already built for `inc` (std::logic_error if not): for
     // step(), which may run under HIP graph capture and must not allocate.
     const TaskTables& built_tables(int inc) const;
-    const TaskTables* latency_tables();   // null when absent
+    const TaskTables* latency_tables();   // null when absent, as for the linear types and 20-node tetrahedra
     const TaskTables* split_form();       // null for other types than quadratic tetrahedra
     void prepare_tasks();                 // the tables of the current tile
     bool tasks() const {
@@ -307,9 +308,9 @@ struct GPU_PBD_FEM final : GPU_FEM {
     ElementSchedule sched;
     XPBD_FEM_VERSION version;
     DBuf<int> d_eids;
+    DBuf<int> d_topo;   // the V2 form's node ids, S per element in the order of d_eids
     // linear tetrahedra: the elements' node ids and records in schedule order
     // (a colour's elements consecutive), and the colours' first elements
-    DBuf<int> d_topo;   // the V2 form's node ids, S per element in the order of d_eids
     DBuf<int4> d_p1_nodes;
     DBuf<float4> d_p1_rec;   // 3 per element: JX_inv (9), V
     DBuf<int> d_color_begin;

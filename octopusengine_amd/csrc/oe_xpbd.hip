@@ -125,13 +125,6 @@ __global__ __launch_bounds__(256) void k_xpbd_v0(XpbdArgs a) {
     }
 }
 
-// Lanes of one element in the V2 projection.  The point stage gives a
-// quadrature point WP lanes' worth of room, PP times over: part p sums its KP
-// nodes of every point's Jx.  The node stage gives the nodes WN lanes, PN
-// times over: part p sums its QN points of every node's gradient.  A colour
-// holds a few hundred elements, far too few to fill the chip, so a pass lasts
-// as long as one wave's chain of instructions: the sums are split over as many
-// lanes as an element can use, and LDS is read 16 bytes at a time.
 // One linear tetrahedron, both constraints: x the nodes' values, w their
 // inverse masses, free whether a node may move.  dN is (-1,-1,-1) and the unit
 // vectors, so Jx holds edge differences and the gradient of node k > 0 is
@@ -330,6 +323,13 @@ __global__ __launch_bounds__(kXpbdResidentThreads) void k_xpbd_p1_resident(XpbdR
     }
 }
 
+// Lanes of one element in the V2 projection.  The point stage gives a
+// quadrature point WP lanes' worth of room, PP times over: part p sums its KP
+// nodes of every point's Jx.  The node stage gives the nodes WN lanes, PN
+// times over: part p sums its QN points of every node's gradient.  A colour
+// holds a few hundred elements, far too few to fill the chip, so a pass lasts
+// as long as one wave's chain of instructions: the sums are split over as many
+// lanes as an element can use, and LDS is read 16 bytes at a time.
 // NARROW (8-node hexahedra, 8 lanes): colours that fill the chip by themselves.
 template <int S, int Q, bool NARROW = false>
 struct V2Lanes;
